@@ -895,6 +895,183 @@ __global__ void __launch_bounds__(64)
     lcnt[L.cnt_off + (int64_t)(L.src_end - L.src_begin) * L.cap + i] = ne > L.maxnb ? 1 : 0;
 }
 
+// OR over the quad of lanes (all four active).
+__device__ __forceinline__ unsigned quad_or(unsigned v) {
+  v |= (unsigned)__builtin_amdgcn_update_dpp((int)v, (int)v, 0xB1, 0xF, 0xF, false);
+  v |= (unsigned)__builtin_amdgcn_update_dpp((int)v, (int)v, 0x4E, 0xF, 0xF, false);
+  return v;
+}
+
+// The search with S lanes per target (64 / S targets per wavefront, S
+// wavefronts per entry of the block table): lane s of a target tests its
+// candidates j with j mod S = s, and the masks are the OR of the S lanes', so
+// the lists are k_nlist's.  For launches of few targets, which latency bounds
+// (nlist_split_blocks): S times the wavefronts, each with 1/S of the tests and
+// about half the candidates to stage; a launch that fills the chip pays S
+// times k_nlist's work per strip instead (3D dam break of 1.4M: 441 us against
+// 309).
+template <int D, typename R, int WIN, int S_>
+__global__ void __launch_bounds__(64)
+    k_nlist_split(Pool<R> P, const SysDesc *__restrict__ sd, const int *__restrict__ n_dev,
+                  const LTask *__restrict__ lt, const SrcDesc *__restrict__ srcs,
+                  const Grid *__restrict__ grids, const CellArr *__restrict__ carr,
+                  const int *__restrict__ cells, const Blk *__restrict__ blk, int nblk, int *lcnt,
+                  int *lidx, const long long *__restrict__ bbmin,
+                  const long long *__restrict__ bbmax, int span) {
+  static_assert(S_ == 4, "quad_or joins four lanes");
+  __shared__ double sx[D][WIN];
+  const int lb = xcd_block(nblk * S_);
+  const Blk b = blk[lb / S_];
+  const LTask L = lt[b.item];
+  const int lane = threadIdx.x, sl = lane % S_;
+  const int i = b.first + (lb % S_) * (64 / S_) + lane / S_;
+  const SysDesc S = sd[L.sys];
+  const bool live = i < n_dev[L.sys];
+  if (__builtin_amdgcn_ballot_w64(live) == 0ull) return;
+  const int64_t gi = S.off + (live ? i : 0);
+  double xi[D];
+#pragma unroll
+  for (int d = 0; d < D; ++d) xi[d] = P.x[d][gi];
+  int2 *emask = reinterpret_cast<int2 *>(lidx + L.list_off) + i;
+  int *ebase = lidx + L.list_off + 2 * (int64_t)L.maxnb * L.cap + i;
+  int ne = 0;  // entries of this target
+  int cq = 0;  // entries of the current source
+  for (int q = L.src_begin; q < L.src_end; ++q) {
+    const SrcDesc Q = srcs[q];
+    const Grid G = grids[Q.grid];
+    cq = 0;
+    if (G.ncells > 0) {
+      const int *cs = cells + carr[Q.carr].off;
+      const int self_j = Q.pk == PK_SELF ? i : -1;
+      const double c2 = Q.cutoff2;
+      const int64_t poff = sd[Q.partner].off;
+      bool act = live;  // as in k_nlist
+      if (Q.pk == PK_DYNAMIC && bbmin) {
+#pragma unroll
+        for (int d = 0; d < D; ++d) {
+          const double mn = double_of(bbmin[Q.partner * 3 + d]);
+          const double mx = double_of(bbmax[Q.partner * 3 + d]);
+          const double gap = mn - xi[d] > xi[d] - mx ? mn - xi[d] : xi[d] - mx;
+          act = act && !(gap > Q.cell * (1.0 + 1e-9));
+        }
+      }
+      int c[D];
+      target_cell<D>(xi, G, Q.cell, c);
+      constexpr int NST = (D == 3) ? 9 : 3;
+      if (__builtin_amdgcn_ballot_w64(act) != 0ull) {
+        // every strip's range up front: one latency instead of one a strip
+        int n0[NST], n1[NST];
+#pragma unroll
+        for (int st = 0; st < NST; ++st) {
+          n0[st] = n1[st] = 1;
+          if (act) {
+            const int sb = strip_base<D>(c, G, st);
+            n0[st] = cs[sb];
+            n1[st] = cs[sb + 3];
+          }
+        }
+#pragma unroll
+        for (int st = 0; st < NST; ++st) {
+          const int j0 = n0[st] - 1, j1 = n1[st] - 1;
+          bool pend = j0 < j1;
+          if (__builtin_amdgcn_ballot_w64(pend) == 0ull) continue;
+          int base = j0;
+          unsigned lo = 0u, hi = 0u;
+          auto flush = [&]() {
+            lo = quad_or(lo);
+            hi = quad_or(hi);
+            const unsigned sdl = (unsigned)(self_j - base);
+            const unsigned sbit = 1u << (sdl & 31u);
+            lo &= sdl < 32u ? ~sbit : ~0u;
+            hi &= sdl - 32u < 32u ? ~sbit : ~0u;
+            if (live && (lo | hi) != 0u) {
+              if (ne < L.maxnb && sl == 0) {
+                emask[(int64_t)ne * L.cap] = make_int2((int)lo, (int)hi);
+                ebase[(int64_t)ne * L.cap] = base;
+              }
+              ++ne;
+              ++cq;
+            }
+            lo = hi = 0u;
+          };
+          const int wmax = wave_red_dpp<true>(j1 - j0);
+          while (true) {
+            const int glo = wave_red_dpp<false>(pend ? j0 : INT_MAX);
+            if (glo == INT_MAX) break;
+            const bool mem = pend && j0 - glo <= span * wmax;
+            const int ghi = wave_red_dpp<true>(mem ? j1 : INT_MIN);
+            for (int w0 = glo; w0 < ghi; w0 += WIN) {
+              const int w1 = ghi - w0 < WIN ? ghi : w0 + WIN;
+              __syncthreads();  // the previous window has been read
+              for (int t = lane; t < w1 - w0; t += 64) {
+#pragma unroll
+                for (int k = 0; k < D; ++k) sx[k][t] = P.x[k][poff + w0 + t];
+              }
+              __syncthreads();
+              // the target's candidates in the window, [js, je): the same for
+              // its S lanes, so they store a full mask together
+              const int js = j0 > w0 ? j0 : w0;
+              const int je = mem ? (j1 < w1 ? j1 : w1) : 0;
+              if (js < je) {
+                if (js >= base + 64) {
+                  flush();
+                  base += 64;
+                }
+                while (true) {
+                  const int ce = je < base + 64 ? je : base + 64;
+                  const int jb = js > base ? js : base;
+                  int d = jb - base + ((sl - jb) & (S_ - 1));
+                  const int t0 = base - w0, de = ce - base;
+                  unsigned long long cur = 0ull;
+                  for (; d + 3 * S_ < de; d += 4 * S_) {
+                    double r[4];
+#pragma unroll
+                    for (int u = 0; u < 4; ++u) {
+                      const double a0 = xi[0] - sx[0][t0 + d + u * S_];
+                      r[u] = a0 * a0;
+                    }
+#pragma unroll
+                    for (int k = 1; k < D; ++k)
+#pragma unroll
+                      for (int u = 0; u < 4; ++u) {
+                        const double ak = xi[k] - sx[k][t0 + d + u * S_];
+                        r[u] = r[u] + ak * ak;
+                      }
+                    const unsigned m4 = (unsigned)(r[0] < c2) | ((unsigned)(r[1] < c2) << S_) |
+                                        ((unsigned)(r[2] < c2) << (2 * S_)) |
+                                        ((unsigned)(r[3] < c2) << (3 * S_));
+                    cur |= (unsigned long long)m4 << d;
+                  }
+                  for (; d < de; d += S_) {
+                    const double a0 = xi[0] - sx[0][t0 + d];
+                    double r2 = a0 * a0;
+#pragma unroll
+                    for (int k = 1; k < D; ++k) {
+                      const double ak = xi[k] - sx[k][t0 + d];
+                      r2 = r2 + ak * ak;
+                    }
+                    cur |= (unsigned long long)(unsigned)(r2 < c2) << d;
+                  }
+                  lo |= (unsigned)cur;
+                  hi |= (unsigned)(cur >> 32);
+                  if (base + 64 >= je) break;
+                  flush();
+                  base += 64;
+                }
+              }
+            }
+            if (mem) pend = false;
+          }
+          flush();
+        }
+      }
+    }
+    if (live && sl == 0) lcnt[L.cnt_off + (int64_t)(q - L.src_begin) * L.cap + i] = cq;
+  }
+  if (live && sl == 0)
+    lcnt[L.cnt_off + (int64_t)(L.src_end - L.src_begin) * L.cap + i] = ne > L.maxnb ? 1 : 0;
+}
+
 // Functors over the accepted partners of each target (one stage).
 template <int D, typename R, int FAM, bool CNT>
 __global__ void __launch_bounds__(GR_BLOCK)
@@ -1103,8 +1280,25 @@ template void launch_sweep<float>(hipStream_t, const Pool<float> &, const SweepA
 template void launch_sweep<double>(hipStream_t, const Pool<double> &, const SweepArgs &, int, int,
                                    bool);
 
+// Up to this many blocks of 64 targets the search takes four lanes per target:
+// with one, such a launch has at most about two wavefronts per SIMD, and a
+// wavefront's own chain of loads and tests is the launch's time.  Measured, us
+// with one / four lanes: 3D dam breaks of 422 blocks 92 / 52, 1000 88 / 56,
+// 1954 101 / 89, 3375 121 / 122, 5593 163 / 181; 2D of 313 blocks 20 / 16,
+// 1250 19.7 / 18.8, 2552 24 / 28 (EP columns of 1600 blocks 21 / 24).
+template <int D>
+constexpr int nlist_split_blocks() {
+  return D == 3 ? 2400 : 1200;
+}
+
 template <int D, typename R, int WIN>
 static void nlist_one(hipStream_t s, const Pool<R> &P, const NlistArgs &a) {
+  if (a.nblk <= nlist_split_blocks<D>()) {
+    k_nlist_split<D, R, WIN, 4><<<a.nblk * 4, 64, 0, s>>>(P, a.sd, a.n, a.lt, a.srcs, a.grids,
+                                                          a.carr, a.cells, a.blk, a.nblk, a.lcnt,
+                                                          a.lidx, a.bbmin, a.bbmax, a.span);
+    return;
+  }
   k_nlist<D, R, WIN><<<a.nblk, 64, 0, s>>>(P, a.sd, a.n, a.lt, a.srcs, a.grids, a.carr, a.cells,
                                            a.blk, a.nblk, a.lcnt, a.lidx, a.bbmin, a.bbmax,
                                            a.span);
