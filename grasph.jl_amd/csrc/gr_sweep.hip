@@ -45,6 +45,15 @@ struct Acc<double> {
   __device__ inline double get() const { return s; }
 };
 
+// One pair's term instead of a sum (k_sweep_split adds the terms of several
+// lanes in order).
+template <typename R>
+struct Term {
+  R t = 0;
+  __device__ inline void add(R v) { t = v; }
+  __device__ inline R get() const { return t; }
+};
+
 // Julia's ^(Float64, Integer) for the LJ powers in FP64; plain products in FP32.
 __device__ inline double pow_i(double x, int n) {
   double y = 1.0, xnlo = 0.0, ynlo = 0.0;
@@ -168,8 +177,8 @@ constexpr int FAM_FORCE_FLUID = NFAM + 1;
 // particle, with the same FP32 operations, so the sums are unchanged.
 constexpr int FAM_FORCE_FLUID_INV = NFAM + 2;
 
-// Target particle: its state and its sums.
-template <int D, typename R, int FAM>
+// Target particle: its state and its sums (A: Acc, or Term for one pair's).
+template <int D, typename R, int FAM, typename A = Acc<R>>
 struct Gather {
   static constexpr bool FORCE =
       FAM == FAM_FORCE || FAM == FAM_FORCE_FLUID || FAM == FAM_FORCE_FLUID_INV;
@@ -182,8 +191,8 @@ struct Gather {
   R vi[D], ri, pi, iri;
   R si[GR_MAXNS];
   int NS;
-  Acc<R> adv[D], adr;
-  Acc<R> asr[GR_MAXNS], avo[3];
+  A adv[D], adr;
+  A asr[GR_MAXNS], avo[3];
 
   __device__ inline void load(const Pool<R> P, const SysDesc &S, const Task &T, int64_t gi) {
 #pragma unroll
@@ -1227,11 +1236,291 @@ __global__ void __launch_bounds__(GR_BLOCK)
 }
 
 // ---------------------------------------------------------------------------
+// Functors with four lanes per target
+// ---------------------------------------------------------------------------
+
+// DPP move within quads of lanes: CTRL a quad_perm.
+template <int CTRL>
+__device__ __forceinline__ int quad_mov(int v) {
+  return __builtin_amdgcn_update_dpp(v, v, CTRL, 0xF, 0xF, false);
+}
+template <int CTRL>
+__device__ __forceinline__ float quad_mov(float v) {
+  return __int_as_float(quad_mov<CTRL>(__float_as_int(v)));
+}
+template <int CTRL>
+__device__ __forceinline__ double quad_mov(double v) {
+  return __hiloint2double(quad_mov<CTRL>(__double2hiint(v)), quad_mov<CTRL>(__double2loint(v)));
+}
+// Transpose in the quad: lane s gets the four lanes' x[s], in lane order.
+template <typename R>
+__device__ __forceinline__ void quad_transpose(R *x, int s) {
+  const bool b0 = s & 1, b1 = s & 2;
+  // z[r] = x[s ^ r], to be read by lane s ^ r
+  const R u0 = b0 ? x[1] : x[0], u1 = b0 ? x[0] : x[1];
+  const R u2 = b0 ? x[3] : x[2], u3 = b0 ? x[2] : x[3];
+  const R z0 = b1 ? u2 : u0, z1 = b1 ? u3 : u1, z2 = b1 ? u0 : u2, z3 = b1 ? u1 : u3;
+  const R y1 = quad_mov<0xB1>(z1), y2 = quad_mov<0x4E>(z2), y3 = quad_mov<0x1B>(z3);
+  // the value from lane k is y[k ^ s]
+  const R v0 = b0 ? y1 : z0, v1 = b0 ? z0 : y1, v2 = b0 ? y3 : y2, v3 = b0 ? y2 : y3;
+  x[0] = b1 ? v2 : v0;
+  x[1] = b1 ? v3 : v1;
+  x[2] = b1 ? v0 : v2;
+  x[3] = b1 ? v1 : v3;
+}
+
+// The terms of one pair as a list, and a target's sums from one.
+template <int D, typename R, int FAM>
+struct Terms {
+  static constexpr bool STRAIN = FAM == FAM_STRAIN;
+  static constexpr int N = STRAIN ? (D == 2 ? 4 : 9) : D + 1;
+  static constexpr int NG = (N + 3) / 4;  // groups of four
+  template <typename G>
+  __device__ static inline void get(const G &g, R *t) {
+    if constexpr (!STRAIN) {
+#pragma unroll
+      for (int d = 0; d < D; ++d) t[d] = g.adv[d].t;
+      t[D] = g.adr.t;
+    } else if constexpr (D == 2) {
+      t[0] = g.asr[0].t;
+      t[1] = g.asr[1].t;
+      t[2] = g.NS == 4 ? g.asr[3].t : g.asr[2].t;
+      t[3] = g.avo[0].t;
+    } else {
+#pragma unroll
+      for (int k = 0; k < 6; ++k) t[k] = g.asr[k].t;
+#pragma unroll
+      for (int k = 0; k < 3; ++k) t[6 + k] = g.avo[k].t;
+    }
+  }
+  template <typename G>
+  __device__ static inline void set(G &g, const double *t) {
+    if constexpr (!STRAIN) {
+#pragma unroll
+      for (int d = 0; d < D; ++d) g.adv[d].s = t[d];
+      g.adr.s = t[D];
+    } else if constexpr (D == 2) {
+      g.asr[0].s = t[0];
+      g.asr[1].s = t[1];
+      if (g.NS == 4)
+        g.asr[3].s = t[2];
+      else
+        g.asr[2].s = t[2];
+      g.avo[0].s = t[3];
+    } else {
+#pragma unroll
+      for (int k = 0; k < 6; ++k) g.asr[k].s = t[k];
+#pragma unroll
+      for (int k = 0; k < 3; ++k) g.avo[k].s = t[6 + k];
+    }
+  }
+};
+
+// k_sweep_list with the four lanes of a quad per target (16 targets per
+// wavefront, four times the wavefronts): lane s evaluates the partners of rank
+// 4r + s of each list entry, then lane c adds component c of the four lanes'
+// terms in their order.  Every sum is the one k_sweep_list makes, addition by
+// addition, so the results are the same bits.  For launches of few targets
+// (sweep_split_targets): there a lane's chain of loads bounds the launch, 0.7
+// to 1.1 us a partner, and this one walks a quarter of it.  Rounds end with
+// their list entry and the terms are exchanged (19 moves a round), so a launch
+// that fills the chip is slower with it (3D dam break of 1.4M: 456 us against
+// 349).
+template <int D, typename R, int FAM, bool CNT>
+__global__ void __launch_bounds__(64)
+    k_sweep_split(Pool<R> P, const SysDesc *__restrict__ sd, const int *__restrict__ n_dev,
+                  const Task *__restrict__ tasks, const SrcDesc *__restrict__ srcs,
+                  const Grid *__restrict__ grids, const CellArr *__restrict__ carr,
+                  const int *__restrict__ cells, const Blk *__restrict__ blk, int nblk,
+                  unsigned long long *pair_count, const LTask *__restrict__ lt,
+                  const int *__restrict__ lcnt, const int *__restrict__ lidx, int nsub) {
+  // nsub workgroups of 16 targets take one entry of the block table
+  const int lb = xcd_block(nblk * nsub);
+  const Blk b = blk[lb / nsub];
+  const Task T = tasks[b.item];
+  const LTask L = lt[T.ltask >= 0 ? T.ltask : 0];
+  const int sl = threadIdx.x & 3;
+  const int i = b.first + (lb % nsub) * 16 + (threadIdx.x >> 2);
+  const SysDesc S = sd[T.sys];
+  const bool live = i < n_dev[T.sys];
+  const int64_t gi = S.off + (live ? i : 0);
+  Gather<D, R, FAM> Gt;
+  Gt.load(P, S, T, gi);
+  unsigned long long ns = 0, no = 0;
+  const int nls = L.src_end - L.src_begin;
+  const bool overflow =
+      live && (T.ltask < 0 || lcnt[L.cnt_off + (int64_t)nls * L.cap + i] != 0);
+  using TT = Terms<D, R, FAM>;
+  double sum[TT::NG] = {};
+  if (live && !overflow) {
+    Gather<D, R, FAM, Term<R>> Gp;
+    Gp.load(P, S, T, gi);
+    constexpr bool CMP = Gather<D, R, FAM>::COMPACT;
+    const int2 *emask = reinterpret_cast<const int2 *>(lidx + L.list_off) + i;
+    const int *ebase = lidx + L.list_off + 2 * (int64_t)L.maxnb * L.cap + i;
+    // -1 for each of the lanes before this one in the quad, as the addend
+    // that drops a mask's lowest bit
+    const unsigned c1 = sl > 0 ? ~0u : 0u, c2 = sl > 1 ? ~0u : 0u, c3 = sl > 2 ? ~0u : 0u;
+    auto wide = [](unsigned c) { return ((unsigned long long)c << 32) | c; };
+    for (int q = T.src_begin; q < T.src_end; ++q) {
+      const SrcDesc Q = srcs[q];
+      int e = 0;
+      for (int l = 0; l < Q.lsrc; ++l) e += lcnt[L.cnt_off + (int64_t)l * L.cap + i];
+      const int eend = e + lcnt[L.cnt_off + (int64_t)Q.lsrc * L.cap + i];
+      if (e >= eend) continue;
+      const int64_t poff = sd[Q.partner].off;
+      SrcK<R> K;
+      K.load(Q);
+      const double da = (Q.pk == PK_DYNAMIC) ? Gp.da_of(Q) : 0.0;
+      const bool nb = needs_b<FAM>(Q);
+      const bool ns_a = CMP && needs_s<FAM>(Q), ns_b = ns_a && Gp.NS > 4;
+      unsigned long long m = 0ull;
+      int base = 0, jn = 0;
+      bool vn = false;
+      int2 mpre = emask[(int64_t)e * L.cap];
+      int bpre = ebase[(int64_t)e * L.cap];
+      // the quad's next (up to four) partners: whether there are any, and
+      // this lane's (jn, vn)
+      auto next = [&]() -> bool {
+        if (m == 0ull) {
+          if (e >= eend) return false;
+          base = bpre;
+          m = ((unsigned long long)(unsigned)mpre.y << 32) | (unsigned)mpre.x;
+          ++e;
+          if (e < eend) {
+            mpre = emask[(int64_t)e * L.cap];
+            bpre = ebase[(int64_t)e * L.cap];
+          }
+        }
+        unsigned long long w = m;
+        w &= w + wide(c1);
+        w &= w + wide(c2);
+        w &= w + wide(c3);
+        vn = w != 0ull;
+        if (vn) jn = base + __builtin_ctzll(w);
+        w &= w - 1ull;
+        if (!vn) w = 0ull;
+        // the mask after the quad's last lane
+        m = ((unsigned long long)(unsigned)quad_mov<0xFF>((int)(w >> 32)) << 32) |
+            (unsigned)quad_mov<0xFF>((int)w);
+        return true;
+      };
+      RecA<R> An{};
+      RecB<R> Bn{};
+      RecC Cn{};
+      RecS Sn{};
+      auto fetch = [&]() {
+        if constexpr (CMP) {
+          Cn = P.rc[poff + jn];
+          if (ns_a) Sn.a = P.rs[poff + jn].a;
+          if (ns_b) Sn.b = P.rs[poff + jn].b;
+        } else {
+          An = P.ra[poff + jn];
+          if (nb) Bn = P.rb[poff + jn];
+        }
+      };
+      auto run = [&](auto dk) {
+        jn = bpre;  // a lane without a partner in the first round reads this one
+        bool have = next();
+        fetch();
+        while (have) {
+          const int64_t gj = poff + jn;
+          const bool v = vn;
+          const RecA<R> Aj = An;
+          const RecB<R> Bj = Bn;
+          const RecC Cj = Cn;
+          const RecS Sj = Sn;
+          have = next();
+          fetch();
+          R t[TT::NG * 4] = {};
+          {
+            double dx[D] = {};
+            double r2 = 0.0;
+            if constexpr (!CMP) {
+#pragma unroll
+              for (int d = 0; d < D; ++d) dx[d] = Gp.xi[d] - Aj.x[d];
+              r2 = dx[0] * dx[0];
+#pragma unroll
+              for (int d = 1; d < D; ++d) r2 = r2 + dx[d] * dx[d];
+            }
+            if (CNT && v) {
+              if (Q.pk == PK_SELF)
+                ++ns;
+              else
+                ++no;
+            }
+            Gp.adr.t = (R)0;  // a static boundary pair adds no density term
+            Gp.template pair<decltype(dk)::value>(P, Q, K, gj, Aj, Bj, Cj, Sj, dx, r2, da);
+            TT::get(Gp, t);
+          }
+#pragma unroll
+          for (int g = 0; g < TT::NG; ++g) {
+            if (D == 3 && TT::STRAIN && g == 2 && !T.write_vor) continue;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) t[4 * g + k] = v ? t[4 * g + k] : (R)0;
+            quad_transpose(t + 4 * g, sl);
+            // adding the zero of a lane without a partner changes nothing: no
+            // sum is -0 (they start at +0)
+#pragma unroll
+            for (int k = 0; k < 4; ++k) sum[g] += (double)t[4 * g + k];
+          }
+        }
+      };
+      if (Q.pk == PK_DYNAMIC)
+        run(std::integral_constant<int, 1>{});
+      else
+        run(std::integral_constant<int, 0>{});
+    }
+  }
+  // every lane of the quad takes all its components
+  double tot[TT::NG * 4];
+#pragma unroll
+  for (int g = 0; g < TT::NG; ++g) {
+    tot[4 * g] = quad_mov<0x00>(sum[g]);
+    tot[4 * g + 1] = quad_mov<0x55>(sum[g]);
+    tot[4 * g + 2] = quad_mov<0xAA>(sum[g]);
+    tot[4 * g + 3] = quad_mov<0xFF>(sum[g]);
+  }
+  TT::set(Gt, tot);
+  if (overflow && sl == 0)
+    gather_direct<D, R, FAM>(Gt, P, sd, T, srcs, grids, carr, cells, i, ns, no);
+  count_pairs<CNT>(pair_count, ns, no);
+  if (live && sl == 0) Gt.store(P, S, T, gi);
+}
+
+// ---------------------------------------------------------------------------
 // Launchers
 // ---------------------------------------------------------------------------
 
+// Up to this many targets a launch of force or strain-rate sweeps takes four
+// lanes per target (k_sweep_split).  Measured, us with one / four lanes (FP32):
+// 3D dam breaks of 27k targets 89 / 39, 64k 79 / 47, 125k 95 / 74, 216k
+// 107 / 114; visco-plastic columns (both stages) 32k 137 / 74, 144k 176 / 163,
+// 256k 216 / 245; 2D dam breaks 20k 21 / 13, 80k 21 / 17, 163k 26 / 29; EP
+// columns 26k 79 / 53, 102k 90 / 75, 205k 109 / 108; FP64 alike (3D 27k
+// 130 / 68, 125k 167 / 158, 216k 238 / 242).
+template <int D>
+constexpr int64_t sweep_split_targets() {
+  return D == 3 ? 150000 : 115000;
+}
+
 template <int D, typename R, int FAM>
 static void launch_one(hipStream_t s, const Pool<R> &P, const SweepArgs &a, bool cnt) {
+  if constexpr (FAM == FAM_FORCE || FAM == FAM_FORCE_FLUID || FAM == FAM_FORCE_FLUID_INV ||
+                FAM == FAM_STRAIN) {
+    if (a.lt && (int64_t)a.nblk * a.block <= sweep_split_targets<D>()) {
+      const int nsub = a.block / 16;
+      if (cnt)
+        k_sweep_split<D, R, FAM, true><<<a.nblk * nsub, 64, 0, s>>>(
+            P, a.sd, a.n, a.tasks, a.srcs, a.grids, a.carr, a.cells, a.blk, a.nblk, a.pair_count,
+            a.lt, a.lcnt, a.lidx, nsub);
+      else
+        k_sweep_split<D, R, FAM, false><<<a.nblk * nsub, 64, 0, s>>>(
+            P, a.sd, a.n, a.tasks, a.srcs, a.grids, a.carr, a.cells, a.blk, a.nblk, a.pair_count,
+            a.lt, a.lcnt, a.lidx, nsub);
+      return;
+    }
+  }
   if (a.lt) {
     // the block table steps by a.block targets (64, 128 or 256)
     if (cnt)
