@@ -317,12 +317,16 @@ struct Plan {
   std::vector<int> real_list;
   DBuf d_real_list, d_bbase_real, blk_real;
   int nblk_real = 0, n_real = 0;
+  // tiles of the counting sort's table for the real and the ghost systems (0:
+  // more keys than a table is kept for, the step sorts by radix)
+  int tiles_real = 0, tiles_ghost = 0;
   // ghosts
   std::vector<int> ghost_list;
   // ghost generation: blocks of source particles per ghost system, and the
   // first (boundary, source block) count slot of each ghost system
   DBuf d_ghost_list, d_bbase_ghost, d_gslot, blk_ghost, blk_gsrc;
   int nblk_ghost = 0, nblk_gsrc = 0, n_ghost = 0, n_gslot = 0;
+  bool gslot_scan = false;  // a ghost system has too many slots to add up per workgroup
   // grids
   std::vector<int> inters;
   std::vector<std::pair<int, bool>> carr_state;  // (cell array, built by this plan)
@@ -397,14 +401,16 @@ struct gr_ctx {
   // tables
   DBuf d_sd, d_n, d_st, d_bnd, d_kmin, d_kmax, d_bbmin, d_bbmax, d_kbase, d_krange, d_flags;
   DBuf d_sysfault;  // per system: GR_FAULT_* bits raised by the step's kernels
-  int bb_rs = 0;  // entries per replica of d_bbmin / d_bbmax (GR_BB_REP replicas)
+  int bb_rs = 0;  // entries per replica of d_bbmin / d_bbmax (GR_BB_REP + 1 replicas)
   bool bb_valid = false;  // d_bbmin / d_bbmax hold the bounds of a step's key pass
   DBuf d_grids, d_carr, d_cellsz, d_inter_sys, d_inter_carr, cells;
   std::vector<CellArr> carr;
   int64_t cells_cap = 0;
   std::vector<StepSys> stepsys;
   // sort / scan scratch
-  DBuf keys, vals, keys2, vals2, hist, cand, cand_scan, scan_bsum, bagg;
+  DBuf keys, vals, keys2, vals2, krank, hist, cand, cand_scan, scan_bsum, bagg;
+  DBuf ktable;          // the counting sort's table (key_table_bytes)
+  int ktable_tiles = 0;
   int64_t sort_cap = 0, cand_cap = 0, cellblk_cap = 0;
   DBuf d_pairs;
   DBuf lidx, lcnt;
@@ -667,7 +673,7 @@ void commit(gr_ctx *c) {
   if (bnds.empty()) bnds.resize(1);
   c->d_bnd.upload(bnds, c->stream);
   std::vector<int> z(ns * 3, 0);
-  std::vector<long long> zl((size_t)ns * 3 * GR_BB_REP, 0);
+  std::vector<long long> zl((size_t)ns * 3 * (GR_BB_REP + 1), 0);
   c->d_kmin.upload(z, c->stream);
   c->d_kmax.upload(z, c->stream);
   c->d_bbmin.upload(zl, c->stream);
@@ -703,6 +709,7 @@ void commit(gr_ctx *c) {
     c->vals.alloc(sc * 4);
     c->keys2.alloc(sc * 4);
     c->vals2.alloc(sc * 4);
+    c->krank.alloc(sc * 4);
     // the radix sort's tile counts start at zero (each sort leaves them so)
     c->hist.alloc(radix_scratch_bytes((int)sc));
     HIPCHK(hipMemsetAsync(c->hist.p, 0, c->hist.bytes, c->stream));
@@ -1015,9 +1022,31 @@ int64_t cell_capacity(gr_ctx *c, const InterH &in, const double *mn, const doubl
   return std::min<int64_t>(cells + 1, (int64_t)1 << 30);
 }
 
-// Bounding boxes of the given real systems (device reduction, host readback).
-void host_bbox(gr_ctx *c, const std::vector<int> &systems, std::vector<double> &mn,
-               std::vector<double> &mx) {
+// Position bounds per system and dimension on the host.
+struct HostBounds {
+  std::vector<long long> mn, mx;  // ordered integers
+  static double dbl(long long i) {  // ordered int64 -> double (ord_of's inverse)
+    const long long b = i < 0 ? (i ^ 0x7FFFFFFFFFFFFFFFLL) : i;
+    double d;
+    memcpy(&d, &b, 8);
+    return d;
+  }
+  double lo(int s, int d) const { return dbl(mn[(size_t)s * 3 + d]); }
+  double hi(int s, int d) const { return dbl(mx[(size_t)s * 3 + d]); }
+};
+
+// Read back the folded bounds (replica 0 of d_bbmin / d_bbmax).
+void read_bounds(gr_ctx *c, HostBounds &h) {
+  const size_t n = c->sys.size() * 3;
+  h.mn.resize(n);
+  h.mx.resize(n);
+  HIPCHK(hipMemcpyAsync(h.mn.data(), c->d_bbmin.p, n * 8, hipMemcpyDeviceToHost, c->stream));
+  HIPCHK(hipMemcpyAsync(h.mx.data(), c->d_bbmax.p, n * 8, hipMemcpyDeviceToHost, c->stream));
+  HIPCHK(hipStreamSynchronize(c->stream));
+}
+
+// Bounds of the given real systems (device reduction, host readback).
+void host_bounds(gr_ctx *c, const std::vector<int> &systems, HostBounds &h) {
   commit(c);
   std::vector<int> list;
   std::vector<Blk> blk;
@@ -1033,25 +1062,61 @@ void host_bbox(gr_ctx *c, const std::vector<int> &systems, std::vector<double> &
   launch_key_minmax(c->stream, xp_pool(c, c->cur), c->d_sd.as<SysDesc>(), c->d_n.as<int>(),
                     db.as<Blk>(), (int)blk.size(), c->D, c->d_bbmin.as<long long>(),
                     c->d_bbmax.as<long long>(), c->bb_rs, dl.as<int>(), (int)list.size(), true);
-  const int ns = (int)c->sys.size();
-  std::vector<long long> bmn(ns * 3), bmx(ns * 3);
-  HIPCHK(hipMemcpyAsync(bmn.data(), c->d_bbmin.p, ns * 3 * 8, hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(hipMemcpyAsync(bmx.data(), c->d_bbmax.p, ns * 3 * 8, hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(hipStreamSynchronize(c->stream));
-  auto dof = [](long long i) {
-    long long u = i < 0 ? (i ^ 0x7FFFFFFFFFFFFFFFLL) : i;
-    double d;
-    memcpy(&d, &u, 8);
-    return d;
-  };
+  read_bounds(c, h);
+}
+
+// Union bounding box of the given real systems.
+void host_bbox(gr_ctx *c, const std::vector<int> &systems, std::vector<double> &mn,
+               std::vector<double> &mx) {
+  HostBounds h;
+  host_bounds(c, systems, h);
   mn.assign(3, INFINITY);
   mx.assign(3, -INFINITY);
   for (int s : systems)
     for (int d = 0; d < c->D; ++d) {
       if (c->sys[s].n == 0) continue;
-      mn[d] = std::min(mn[d], dof(bmn[s * 3 + d]));
-      mx[d] = std::max(mx[d], dof(bmx[s * 3 + d]));
+      mn[d] = std::min(mn[d], h.lo(s, d));
+      mx[d] = std::max(mx[d], h.hi(s, d));
     }
+}
+
+// Steps between two checks of the cell arrays' capacity, and the cells kept
+// free on every side of the systems' current extent.  With dt = CFL·h/c a
+// particle at speed v moves CFL·(v/c)·h per step: a chunk moves a subsonic
+// particle (v < c, CFL <= 1) at most 16 h = 8 cells.
+constexpr int kGrowChunk = 16;
+constexpr int kGrowMargin = 8;
+
+// Tiles of a counting table for the listed systems' cell keys, `margin` cells
+// wider than their bounds on every side; 0 beyond kMaxKeyTiles (8M keys, 68 MB
+// of table, whose scan would cost as much as the radix passes).  A ghost
+// system's bounds are its source's, widened by twice its cutoff (a mirror
+// moves a particle by at most that).  Also 0 where a system's cells hold more
+// than kKeyCellMean particles on average: the rank within the cell grows with
+// them (sort of 200k particles in motion, 3D: table 49 us at 32 a cell, 68 at
+// 128, 83 at 256, 105 at 512, radix kernels 74 to 87; 20k in 2D: 31, 35, 39,
+// 49 against 49 to 58).
+constexpr int kMaxKeyTiles = 8192;
+constexpr double kKeyCellMean = 256.0;
+int key_tiles(gr_ctx *c, const std::vector<int> &systems, const HostBounds &h, int margin) {
+  double keys = 1.0;
+  for (int s : systems) {
+    const SysH &S = c->sys[s];
+    const bool ghost = S.kind == GR_SYS_GHOST;
+    const double cut = c->stepsys[s].sort_cutoff, pad = ghost ? 4.0 * S.gcut : 0.0;
+    double r = 1.0, cells = 1.0;
+    for (int d = 0; d < c->D; ++d) {
+      const double ext = h.hi(ghost ? S.src : s, d) - h.lo(ghost ? S.src : s, d);
+      if (!(std::isfinite(ext) && ext >= 0.0)) continue;  // faulted: one key
+      r *= std::floor((ext + pad) / cut) + 2.0 + 2.0 * margin;
+      cells *= std::floor(ext / cut) + 1.0;
+    }
+    keys += r;
+    if (!(keys < 1e12)) return 0;
+    if (!ghost && (double)S.n > kKeyCellMean * cells) return 0;
+  }
+  const double t = std::floor(keys / key_table_tile()) + 1.0;
+  return t <= kMaxKeyTiles ? (int)t : 0;
 }
 
 // Destroy every captured step graph (device tables or pools they point to
@@ -1221,6 +1286,9 @@ void plan_ghosts(gr_ctx *c, Plan &P, const std::vector<int> &ghosts) {
   P.blk_gsrc.upload(sblk, c->stream);
   P.nblk_ghost = (int)blk.size();
   P.nblk_gsrc = (int)sblk.size();
+  // up to 8192 slots a system, every workgroup that holds ghosts adds up the
+  // slots before its own (32 loads a thread) instead of three scan kernels
+  for (int g : ghosts) P.gslot_scan = P.gslot_scan || ghost_slots(c, c->sys[g]) > 8192;
 }
 
 // Stage plans of a batch of integrators: updater tables (with the fused EOS
@@ -1648,6 +1716,19 @@ Plan &get_plan(gr_ctx *c, const std::vector<int> &integs) {
   }
   c->carr_used = nullptr;
   plan_grids(c, *P, inters, &used);
+  if (!reals.empty()) {  // key tables with room for a few chunks of steps
+    HostBounds hb;
+    host_bounds(c, reals, hb);
+    P->tiles_real = key_tiles(c, reals, hb, kGrowMargin + 4);
+    P->tiles_ghost = ghosts.empty() ? 0 : key_tiles(c, ghosts, hb, kGrowMargin + 4);
+    const int t = std::max(P->tiles_real, P->tiles_ghost);
+    if (t > c->ktable_tiles) {
+      c->ktable.alloc(key_table_bytes(t));
+      HIPCHK(hipMemsetAsync(c->ktable.p, 0, c->ktable.bytes, c->stream));
+      c->ktable_tiles = t;
+      drop_graphs(c);
+    }
+  }
   HIPCHK(hipStreamSynchronize(c->stream));
   Plan &ref = *P;
   c->plans[integs] = std::move(P);
@@ -1676,6 +1757,19 @@ void all_real(gr_ctx *c, const Blk *&blk, int &nblk) {
 // Step phases
 // ---------------------------------------------------------------------------
 
+// The counting sort of a step's real or ghost systems (after their bounds).
+void key_sort(gr_ctx *c, const XP &xs, const DBuf &blk, int nblk, const DBuf &bbase,
+              const DBuf &list, int nlist, int n, int tiles) {
+  launch_key_sort(c->stream, xs, c->d_sd.as<SysDesc>(), c->d_n.as<int>(), c->d_st.as<StepSys>(),
+                  blk.as<Blk>(), nblk, bbase.as<int>(), c->D, list.as<int>(), nlist, n,
+                  c->d_bbmin.as<long long>(), c->d_bbmax.as<long long>(), c->bb_rs,
+                  c->d_kmin.as<int>(), c->d_kmax.as<int>(), c->d_krange.as<unsigned>(),
+                  c->d_kbase.as<unsigned>(), c->keys.as<unsigned>(), c->vals.as<int>(),
+                  c->keys2.as<unsigned>(), c->vals2.as<int>(), c->krank.as<unsigned>(),
+                  c->d_flags.as<int>(), c->d_sysfault.as<int>(), c->ktable.as<unsigned>(),
+                  c->ktable_tiles, tiles);
+}
+
 // half: also take the leapfrog half step of the plan's integrated systems
 // in the permutation (run_step, when it follows the sort directly in data).
 template <typename R>
@@ -1683,6 +1777,28 @@ void phase_sort_real(gr_ctx *c, Plan &P, bool half = false, int pack = 0) {
   if (P.real_list.empty()) return;
   hipStream_t s = c->stream;
   const XP xs = xp_pool(c, c->cur);
+  const Blk *arb;
+  int arn;
+  if (P.tiles_real > 0) {  // a step: counting sort (the bounds' replicas are reset already)
+    launch_key_minmax(s, xs, c->d_sd.as<SysDesc>(), c->d_n.as<int>(), P.blk_real.as<Blk>(),
+                      P.nblk_real, c->D, c->d_bbmin.as<long long>(), c->d_bbmax.as<long long>(),
+                      c->bb_rs, P.d_real_list.as<int>(), (int)P.real_list.size(), false,
+                      c->d_flags.as<int>());
+    key_sort(c, xs, P.blk_real, P.nblk_real, P.d_bbase_real, P.d_real_list,
+             (int)P.real_list.size(), P.n_real, P.tiles_real);
+    all_real(c, arb, arn);
+    const KeyTable kt =
+        key_table_view(c->ktable.as<unsigned>(), c->ktable_tiles, P.tiles_real, c->keys2.as<unsigned>(),
+                       c->d_krange.as<unsigned>(), c->d_kbase.as<unsigned>(),
+                       P.d_real_list.as<int>(), (int)P.real_list.size());
+    Pool<R> A = pool_view<R>(c, c->cur), B = pool_view<R>(c, 1 - c->cur);
+    launch_permute_real<R>(s, A, B, c->d_sd.as<SysDesc>(), arb, arn, P.d_bbase_real.as<int>(),
+                           c->vals.as<int>(), c->vals2.as<int>(), c->d_flags.as<int>(),
+                           c->vadj_any ? 1 : 0, c->D, c->d_st.as<StepSys>(),
+                           half ? P.d_halfsys.as<int>() : nullptr, pack, &kt);
+    c->cur = 1 - c->cur;
+    return;
+  }
   launch_minmax_reset(s, P.d_real_list.as<int>(), (int)P.real_list.size(),
                       c->d_bbmin.as<long long>(), c->d_bbmax.as<long long>(), c->bb_rs);
   launch_key_minmax(s, xs, c->d_sd.as<SysDesc>(), c->d_n.as<int>(), P.blk_real.as<Blk>(),
@@ -1699,8 +1815,6 @@ void phase_sort_real(gr_ctx *c, Plan &P, bool half = false, int pack = 0) {
                    c->hist.as<unsigned>());
   launch_radix_sort(s, c->keys.as<unsigned>(), c->vals.as<int>(), c->keys2.as<unsigned>(),
                     c->vals2.as<int>(), c->hist.as<unsigned>(), P.n_real, c->d_flags.as<int>());
-  const Blk *arb;
-  int arn;
   all_real(c, arb, arn);
   Pool<R> A = pool_view<R>(c, c->cur), B = pool_view<R>(c, 1 - c->cur);
   launch_permute_real<R>(s, A, B, c->d_sd.as<SysDesc>(), arb, arn,
@@ -1710,21 +1824,40 @@ void phase_sort_real(gr_ctx *c, Plan &P, bool half = false, int pack = 0) {
   c->cur = 1 - c->cur;
 }
 
-// Generation (flags, scan, scatter to scratch) + sort (scratch → pool).
+// Generation (counts, scatter to scratch) + sort (scratch → pool).
 template <typename R>
 void phase_ghosts(gr_ctx *c, Plan &P, bool generate, bool sort) {
   if (P.ghost_list.empty()) return;
   hipStream_t s = c->stream;
   const XP x = xp_pool(c, c->cur);
   Pool<R> A = pool_view<R>(c, c->cur);
+  const bool table = generate && sort && P.tiles_ghost > 0;
   if (generate) {
     launch_ghost_count(s, x, c->d_sd.as<SysDesc>(), c->d_bnd.as<Bnd>(), P.blk_gsrc.as<Blk>(),
-                       P.nblk_gsrc, P.d_gslot.as<int>(), c->D, c->cand.as<int>());
-    launch_scan(s, c->cand.as<int>(), c->cand_scan.as<int>(), c->scan_bsum.as<int>(), P.n_gslot);
+                       P.nblk_gsrc, P.d_gslot.as<int>(), c->D, c->cand.as<int>(),
+                       table ? c->d_flags.as<int>() : nullptr);
+    if (P.gslot_scan)
+      launch_scan(s, c->cand.as<int>(), c->cand_scan.as<int>(), c->scan_bsum.as<int>(), P.n_gslot);
     launch_ghost_scatter(s, x, xpw_gxs(c), c->gidx_s.as<int>(), c->gbnd_s.as<int>(),
                          c->gnrm.as<int>(), c->d_sd.as<SysDesc>(), c->d_bnd.as<Bnd>(),
                          P.blk_gsrc.as<Blk>(), P.nblk_gsrc, P.d_gslot.as<int>(),
-                         c->cand_scan.as<int>(), c->D, c->d_n.as<int>());
+                         c->cand.as<int>(), P.gslot_scan ? c->cand_scan.as<int>() : nullptr, c->D,
+                         c->d_n.as<int>(), table ? c->d_bbmin.as<long long>() : nullptr,
+                         c->d_bbmax.as<long long>(), c->bb_rs);
+  }
+  if (table) {  // a step: counting sort (the bounds' replicas are reset already)
+    const XP gx = xp_gxs(c);
+    key_sort(c, gx, P.blk_ghost, P.nblk_ghost, P.d_bbase_ghost, P.d_ghost_list,
+             (int)P.ghost_list.size(), P.n_ghost, P.tiles_ghost);
+    const KeyTable kt =
+        key_table_view(c->ktable.as<unsigned>(), c->ktable_tiles, P.tiles_ghost, c->keys2.as<unsigned>(),
+                       c->d_krange.as<unsigned>(), c->d_kbase.as<unsigned>(),
+                       P.d_ghost_list.as<int>(), (int)P.ghost_list.size());
+    launch_permute_ghost(s, gx, c->gidx_s.as<int>(), c->gbnd_s.as<int>(), xpw_pool(c, c->cur),
+                         A.gidx, A.gbnd, c->d_sd.as<SysDesc>(), c->d_n.as<int>(),
+                         P.blk_ghost.as<Blk>(), P.nblk_ghost, P.d_bbase_ghost.as<int>(),
+                         c->vals.as<int>(), c->vals2.as<int>(), c->d_flags.as<int>(), c->D, &kt);
+    return;
   }
   const XP gx = xp_gxs(c);
   launch_minmax_reset(s, P.d_ghost_list.as<int>(), (int)P.ghost_list.size(),
@@ -1897,13 +2030,6 @@ void phase_xsph(gr_ctx *c, Plan &P) {
   launch_xsph<R>(s, A, sd, st, c->d_n.as<int>(), P.blk_int.as<Blk>(), P.nblk_int, c->D, 2);
 }
 
-// Steps between two checks of the cell arrays' capacity, and the cells kept
-// free on every side of the systems' current extent.  With dt = CFL·h/c a
-// particle at speed v moves CFL·(v/c)·h per step: a chunk moves a subsonic
-// particle (v < c, CFL <= 1) at most 16 h = 8 cells.
-constexpr int kGrowChunk = 16;
-constexpr int kGrowMargin = 8;
-
 // The bounds of the last key pass (replica 0 of d_bbmin / d_bbmax, exact
 // doubles) against each interaction's cell arrays: an interaction whose grid,
 // kGrowMargin cells wider on every side, would not fit gets new arrays sized
@@ -1913,18 +2039,16 @@ constexpr int kGrowMargin = 8;
 bool grow_cells(gr_ctx *c, const Plan &P) {
   if (P.inters.empty()) return false;
   const int ns = (int)c->sys.size();
-  std::vector<long long> bmn((size_t)ns * 3), bmx((size_t)ns * 3);
-  HIPCHK(hipMemcpyAsync(bmn.data(), c->d_bbmin.p, bmn.size() * 8, hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(hipMemcpyAsync(bmx.data(), c->d_bbmax.p, bmx.size() * 8, hipMemcpyDeviceToHost, c->stream));
   std::vector<int> nn(ns);
   HIPCHK(hipMemcpyAsync(nn.data(), c->d_n.p, ns * sizeof(int), hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(hipStreamSynchronize(c->stream));
-  auto dbl = [](long long i) {  // ordered int64 -> double (ord_of's inverse)
-    const long long b = i < 0 ? (i ^ 0x7FFFFFFFFFFFFFFFLL) : i;
-    double d;
-    memcpy(&d, &b, 8);
-    return d;
+  HostBounds hb;
+  read_bounds(c, hb);
+  auto outgrown = [&](const std::vector<int> &list, int tiles) {
+    if (list.empty() || tiles == 0) return false;
+    const int t = key_tiles(c, list, hb, kGrowMargin);
+    return t == 0 || t > tiles;
   };
+  const bool tables = outgrown(P.real_list, P.tiles_real) || outgrown(P.ghost_list, P.tiles_ghost);
   bool grew = false;
   for (int it : P.inters) {
     InterH &in = c->inter[it];
@@ -1934,7 +2058,7 @@ bool grow_cells(gr_ctx *c, const Plan &P) {
     for (int sid : {in.a, in.b}) {
       if (sid < 0 || nn[sid] <= 0) continue;
       for (int d = 0; d < c->D; ++d) {
-        const double lo = dbl(bmn[sid * 3 + d]), hi = dbl(bmx[sid * 3 + d]);
+        const double lo = hb.lo(sid, d), hi = hb.hi(sid, d);
         finite = finite && std::isfinite(lo) && std::isfinite(hi);
         mn[d] = any ? std::min(mn[d], lo) : lo;
         mx[d] = any ? std::max(mx[d], hi) : hi;
@@ -1971,9 +2095,10 @@ bool grow_cells(gr_ctx *c, const Plan &P) {
     }
     grew = true;
   }
-  if (!grew) return false;
+  if (!grew && !tables) return false;
   drop_graphs(c);
   c->plans.clear();
+  if (!grew) return true;  // the next plan takes larger key tables
   if ((size_t)std::max<int64_t>(c->cells_cap, 1) * 4 > c->cells.bytes)
     c->cells.alloc(std::max<int64_t>(c->cells_cap, 1) * 4);
   c->d_carr.upload(c->carr, c->stream);
@@ -2146,10 +2271,20 @@ void do_steps(gr_ctx *c, const std::vector<int> &integs, int nsteps) {
   // chunks of at most kGrowChunk steps; between chunks the cell arrays
   // follow the systems' spread (grow_cells), so a flow that runs out over
   // thousands of steps never outgrows its grids
+  // the step's bounds passes find their replicas reset (each step's sort leaves
+  // them so; other users of the bounds do not)
+  auto reset_bounds = [&]() {
+    launch_minmax_reset(c->stream, P->d_real_list.as<int>(), (int)P->real_list.size(),
+                        c->d_bbmin.as<long long>(), c->d_bbmax.as<long long>(), c->bb_rs);
+    launch_minmax_reset(c->stream, P->d_ghost_list.as<int>(), (int)P->ghost_list.size(),
+                        c->d_bbmin.as<long long>(), c->d_bbmax.as<long long>(), c->bb_rs);
+  };
+  if (nsteps > 0) reset_bounds();
   for (int k0 = 0; k0 < nsteps; k0 += kGrowChunk) {
     if ((k0 > 0 || c->bb_valid) && grow_cells(c, *P)) {
       P = &get_plan(c, integs);
       mark_grids(c, *P);
+      reset_bounds();
     }
     const int k1 = std::min(nsteps, k0 + kGrowChunk);
     for (int k = k0; k < k1; ++k) {

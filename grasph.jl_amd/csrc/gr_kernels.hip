@@ -147,13 +147,15 @@ __device__ inline void radix_add_runs(unsigned bin, bool valid, unsigned *cnt) {
 //
 // The workgroups of a launch run concurrently, so they all see the initial
 // bounds and most of them take their atomics; those atomics are spread over
-// GR_BB_REP replicas of the bounds (stride `rs`), one for the workgroups of
-// each XCD, and folded into replica 0 afterwards (k_key_base, k_bb_fold).
+// replicas 1 .. GR_BB_REP of the bounds (stride `rs`), one for the workgroups
+// of each XCD, and folded into replica 0 afterwards (key_space, k_bb_fold).
+// `flags`: also clear the sort's inversion flag for the key pass that follows.
 template <int D, int PER>
 __global__ void k_key_minmax(XP xs, const SysDesc *sd, const int *n_dev, const Blk *blk, int nblk,
-                             long long *bbmin, long long *bbmax, int rs) {
-  bbmin += (blockIdx.x % GR_BB_REP) * rs;
-  bbmax += (blockIdx.x % GR_BB_REP) * rs;
+                             long long *bbmin, long long *bbmax, int rs, int *flags) {
+  if (flags && blockIdx.x == 0 && threadIdx.x == 0) flags[0] = 0;
+  bbmin += (1 + blockIdx.x % GR_BB_REP) * rs;
+  bbmax += (1 + blockIdx.x % GR_BB_REP) * rs;
   __shared__ long long red[2][GR_BLOCK / 64][3];
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int b0 = blockIdx.x * PER;
@@ -234,29 +236,39 @@ __global__ void k_minmax_reset(const int *list, int nlist, long long *bbmin, lon
   const int r = t / (nlist * 3);
   t -= r * nlist * 3;
   int s = list[t / 3], d = t % 3;
-  bbmin[r * rs + s * 3 + d] = LLONG_MAX;
-  bbmax[r * rs + s * 3 + d] = LLONG_MIN;
+  bbmin[(r + 1) * rs + s * 3 + d] = LLONG_MAX;
+  bbmax[(r + 1) * rs + s * 3 + d] = LLONG_MIN;
 }
 
-// Fold the replicas of the listed systems' bounds into replica 0.
-__device__ __forceinline__ void bb_fold(long long *bbmin, long long *bbmax, int rs, int e) {
-  long long a = bbmin[e], b = bbmax[e];
+// The bounds of entry e over the replicas.
+__device__ __forceinline__ void bb_fold(const long long *bbmin, const long long *bbmax, int rs,
+                                        int e, long long &mn, long long &mx) {
+  long long a = LLONG_MAX, b = LLONG_MIN;
 #pragma unroll
-  for (int r = 1; r < GR_BB_REP; ++r) {
+  for (int r = 1; r <= GR_BB_REP; ++r) {
     const long long u = bbmin[r * rs + e], v = bbmax[r * rs + e];
     a = u < a ? u : a;
     b = v > b ? v : b;
   }
-  bbmin[e] = a;
-  bbmax[e] = b;
+  mn = a;
+  mx = b;
 }
 __global__ void k_bb_fold(const int *list, int nlist, long long *bbmin, long long *bbmax, int rs) {
   const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t < nlist * 3) bb_fold(bbmin, bbmax, rs, list[t / 3] * 3 + t % 3);
+  if (t < nlist * 3) {
+    const int e = list[t / 3] * 3 + t % 3;
+    bb_fold(bbmin, bbmax, rs, e, bbmin[e], bbmax[e]);
+  }
 }
 
 // Threads of k_key_base: one per listed system in each round.
 #define KB_THREADS 1024
+// Up to this many systems (a lane each) and workgroups, every workgroup of the
+// counting sort's key pass finds the key bases itself, which saves a launch
+// (2D dam break of 23k particles: sort 33 -> 30 us); with more workgroups the
+// repeated work costs more (5700 workgroups: 145 us against 131).
+#define KC_SYSTEMS 64
+#define KC_BLOCKS 512
 
 // Key space of each listed system: lexicographic linearisation of
 // (k1 - kmin1, ..., kD - kminD), bases prefix-summed in list order.  Ghost
@@ -268,10 +280,83 @@ __global__ void k_bb_fold(const int *list, int nlist, long long *bbmin, long lon
 __device__ inline double unord_d(long long o) {
   return __longlong_as_double(o < 0 ? (o ^ 0x7FFFFFFFFFFFFFFFLL) : o);
 }
+struct KeySpace {
+  int kmin[3], kmax[3];
+  unsigned kr[3];        // cells per dimension; kr[0] == 0 marks a faulted system
+  long long mn[3], mx[3];  // position bounds (ordered integers)
+  int fault;             // GR_FAULT_*
+};
+// The key space of system s (n > 0 particles); returns its number of keys.
+__device__ inline unsigned long long key_space(int D, double cutoff, const long long *bbmin,
+                                               const long long *bbmax, int rs, int s,
+                                               KeySpace &K) {
+  unsigned long long range = 1;
+  bool nonfinite = false;
+  for (int d = 0; d < 3; ++d) {
+    bb_fold(bbmin, bbmax, rs, s * 3 + d, K.mn[d], K.mx[d]);
+    K.kmin[d] = K.kmax[d] = 0;
+    K.kr[d] = 1u;
+    if (d >= D) continue;
+    const double lo = unord_d(K.mn[d]), hi = unord_d(K.mx[d]);
+    const int ka = key_comp(lo, cutoff), kb = key_comp(hi, cutoff);
+    K.kmin[d] = ka < kb ? ka : kb;
+    K.kmax[d] = ka < kb ? kb : ka;
+    long long r = (long long)K.kmax[d] - (long long)K.kmin[d] + 1;
+    if (!(lo <= hi)) r = 1LL << 32;  // NaN
+    K.kr[d] = (unsigned)r;
+    // any product of 2^32 or more overflows the 32-bit keys: saturate there so
+    // that neither this product nor the prefix sum wraps
+    range = (range > 0xFFFFFFFFull || r > 0xFFFFFFFFLL) ? (1ull << 32)
+                                                         : range * (unsigned long long)r;
+    nonfinite = nonfinite || !(lo <= hi) || !isfinite(lo) || !isfinite(hi);
+  }
+  if (range > (1ull << 32)) range = 1ull << 32;
+  // a system whose bounds are not finite, or whose own keys need 32 bits or
+  // more, is faulted: all its keys become its base (the sort keeps its
+  // order), so the systems after it keep their keys and the step goes on for
+  // them
+  K.fault = 0;
+  if (nonfinite || range >= 0xFFFFFFFFull) {
+    K.fault = nonfinite ? GR_FAULT_NONFINITE : GR_FAULT_DOMAIN;
+    for (int d = 0; d < D; ++d) {
+      K.kmin[d] = K.kmax[d] = 0;
+      K.kr[d] = d == 0 ? 0u : 1u;
+    }
+    range = 1;
+  }
+  return range;
+}
+// Store what the later kernels read of a system's key space.
+__device__ inline void key_space_store(const KeySpace &K, int s, bool live, long long *bbmin,
+                                       long long *bbmax, int *kmin, int *kmax, unsigned *krange,
+                                       int *flags, int *sysfault) {
+  for (int d = 0; d < 3; ++d) {
+    bbmin[s * 3 + d] = K.mn[d];
+    bbmax[s * 3 + d] = K.mx[d];
+    krange[s * 3 + d] = live ? K.kr[d] : 1u;
+    if (live) {
+      kmin[s * 3 + d] = K.kmin[d];
+      kmax[s * 3 + d] = K.kmax[d];
+    }
+  }
+  if (live && K.fault) {
+    atomicOr(&sysfault[s], K.fault);
+    atomicOr(&flags[1], 8);
+  }
+}
+// Flags of the whole key range: overflow, the bound of the keys and the radix
+// passes below it.  The running base only grows, so overflowing at some system
+// means the total overflows.
+__device__ inline void key_flags(unsigned long long total, int *flags) {
+  if (total >= 0xFFFFFFFFull) atomicOr(&flags[1], 1);
+  flags[2] = (int)(unsigned)(total < 0xFFFFFFFFull ? total : 0xFFFFFFFFull);
+  flags[3] = radix_passes((unsigned)flags[2]);
+}
+
 __global__ void __launch_bounds__(KB_THREADS)
     k_key_base(const int *list, int nlist, int D, int pad, const int *n_dev, const StepSys *st,
                long long *bbmin, long long *bbmax, int rs, int *kmin, int *kmax,
-               unsigned *kbase, unsigned *krange, int *flags, int *sysfault) {
+               unsigned *kbase, unsigned *krange, int *flags, int *sysfault, int keep) {
   // one workgroup: the systems' key ranges in parallel, KB_THREADS at a time,
   // and their exclusive prefix sum (each system's keys start after the ranges
   // of the systems listed before it, plus one padding key each when `pad`)
@@ -284,46 +369,11 @@ __global__ void __launch_bounds__(KB_THREADS)
     int s = -1;
     if (q < nlist) {
       s = list[q];
-      for (int d = 0; d < 3; ++d) bb_fold(bbmin, bbmax, rs, s * 3 + d);
-      if (n_dev[s] > 0) {
-        range = 1;
-        const double cutoff = st[s].sort_cutoff;
-        for (int d = 0; d < D; ++d) {
-          const int ka = key_comp(unord_d(bbmin[s * 3 + d]), cutoff);
-          const int kb = key_comp(unord_d(bbmax[s * 3 + d]), cutoff);
-          const int lo = ka < kb ? ka : kb, hi = ka < kb ? kb : ka;
-          kmin[s * 3 + d] = lo;
-          kmax[s * 3 + d] = hi;
-          long long r = (long long)hi - (long long)lo + 1;
-          if (!(unord_d(bbmin[s * 3 + d]) <= unord_d(bbmax[s * 3 + d]))) r = 1LL << 32;  // NaN
-          krange[s * 3 + d] = (unsigned)r;
-          // any product of 2^32 or more overflows the 32-bit keys: saturate
-          // there so that neither this product nor the prefix sum wraps
-          range = (range > 0xFFFFFFFFull || r > 0xFFFFFFFFLL) ? (1ull << 32)
-                                                               : range * (unsigned long long)r;
-        }
-        if (range > (1ull << 32)) range = 1ull << 32;
-        // a system whose bounds are not finite, or whose own keys need 32
-        // bits or more, is faulted: all its keys become its base (the
-        // stable sort keeps its order), so the systems after it keep
-        // their keys and the step goes on for them
-        bool nonfinite = false;
-        for (int d = 0; d < D; ++d)
-          nonfinite = nonfinite || !(unord_d(bbmin[s * 3 + d]) <= unord_d(bbmax[s * 3 + d])) ||
-                      !isfinite(unord_d(bbmin[s * 3 + d])) || !isfinite(unord_d(bbmax[s * 3 + d]));
-        if (nonfinite || range >= 0xFFFFFFFFull) {
-          atomicOr(&sysfault[s], nonfinite ? GR_FAULT_NONFINITE : GR_FAULT_DOMAIN);
-          atomicOr(&flags[1], 8);
-          for (int d = 0; d < D; ++d) {
-            kmin[s * 3 + d] = 0;
-            kmax[s * 3 + d] = 0;
-            krange[s * 3 + d] = d == 0 ? 0u : 1u;  // krange[0] == 0 marks it
-          }
-          range = 1;
-        }
-      } else {
-        for (int d = 0; d < D; ++d) krange[s * 3 + d] = 1;
-      }
+      KeySpace K;
+      const bool live = n_dev[s] > 0;
+      range = key_space(D, st[s].sort_cutoff, bbmin, bbmax, rs, s, K);
+      if (!live) range = 0;
+      key_space_store(K, s, live, bbmin, bbmax, kmin, kmax, krange, flags, sysfault);
       range += pad ? 1 : 0;
     }
     unsigned long long inc = range;
@@ -343,13 +393,8 @@ __global__ void __launch_bounds__(KB_THREADS)
     __syncthreads();  // wsum is written again for the next systems
   }
   if (t == 0) {
-    flags[0] = 0;
-    // the running base only grows, so overflowing at some system means the
-    // total overflows
-    if (carry >= 0xFFFFFFFFull) flags[1] |= 1;
-    // every key is below this bound: radix passes above its top bit are identities
-    flags[2] = (int)(unsigned)(carry < 0xFFFFFFFFull ? carry : 0xFFFFFFFFull);
-    flags[3] = radix_passes((unsigned)flags[2]);
+    if (!keep) flags[0] = 0;
+    key_flags(carry, flags);
   }
 }
 
@@ -571,6 +616,313 @@ __device__ __forceinline__ const int *radix_sorted_vals(const int *vals, const i
 }
 
 // ---------------------------------------------------------------------------
+// Counting sort of the step: one table entry per key
+//
+// The keys of a step are cells, a few per 100 particles, so they are sorted by
+// counting: k_key_count writes the keys and takes each particle a place in its
+// cell (one atomic per run of equal keys along a wavefront), k_key_scan turns
+// the counts into the cells' starts, k_key_place puts every particle into its
+// cell, and the permutations order each cell by the particles' former places
+// (the sort is stable): a particle's rank is the number of smaller former
+// places in its cell, which holds a handful.  Against the radix sort's scan
+// and scatter kernel per 8-bit digit (each 3 to 16 us, four of each launched
+// whatever the key range) it takes two kernels.  Sort phase, radix before:
+// 3D dam break of 1.4M particles 158 -> 140 us, 2D dam break of 23k 50 -> 30,
+// 2D column of 12.8k 40 -> 28 (its ghosts, generated and sorted, 56 -> 28).
+// Bound by the launches below 100k particles; at 1.4M by the atomics
+// (k_key_count 33 us of the 140, the scan and the placement 9) and the moved
+// bytes of the permutation (53 us).
+//
+// Table (key_table_bytes): counts, starts, tile sums, laid out for the tiles it
+// was allocated with.  Every count and sum a sort raises is zero again when it
+// has ended.  `cap`, a multiple of KT_TILE less one, bounds the keys of the
+// step's sort; with more keys than that (a system that has run out since the
+// plan was made), one wavefront of k_key_place sorts the step's keys by radix.
+// ---------------------------------------------------------------------------
+
+#define KT_TILE 1024  // keys per workgroup of the scan
+#define KT_RANKS 8    // former places compared at a time in the rank within a cell
+// Copies of each tile's sum: k_key_count's atomics are spread over them (a tile
+// takes one from each of some 100 wavefronts; with one copy the kernel took
+// 154 us instead of 40 in the 3D dam break of 1.4M particles).
+#define KT_REP 16
+
+// Lane's place among the valid lanes' run of equal `k` (valid lanes come
+// first): lane of the run's head, and its length at the head.
+__device__ inline int run_head(unsigned k, bool valid, int &len) {
+  const int lane = threadIdx.x & 63;
+  const unsigned prev = __shfl_up(k, 1, 64);
+  const unsigned long long V = __ballot(valid);
+  const unsigned long long H = __ballot(valid && (lane == 0 || prev != k));
+  const unsigned long long le = lane == 63 ? ~0ull : ((2ull << lane) - 1ull);
+  const unsigned long long ends = (H | ~V) & ~le;
+  const int next = ends ? __ffsll((long long)ends) - 1 : 64;
+  const int head = (H & le) ? 63 - __clzll((long long)(H & le)) : lane;
+  len = next - lane;
+  return head;
+}
+
+template <int D>
+__global__ void __launch_bounds__(GR_BLOCK)
+    k_key_count(XP xs, const SysDesc *sd, const int *n_dev, const StepSys *st, const Blk *blk,
+                const int *bbase, const int *list, int nlist, long long *bbmin, long long *bbmax,
+                int rs, int *kmin, int *kmax, unsigned *krange, unsigned *kbase, unsigned *keys,
+                int *vals, unsigned *rank, int *flags, int *sysfault, unsigned *count,
+                unsigned *tsum, unsigned cap, int inl) {
+  __shared__ int s_kmin[3];
+  __shared__ unsigned s_kr[3], s_base, s_total;
+  __shared__ unsigned kw[GR_BLOCK / 64];
+  const Blk b = blk[blockIdx.x];
+  const int s = b.item;
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int i = b.first + threadIdx.x;
+  const int n = n_dev[s];
+  const int64_t gi = sd[s].off + i;
+  if (b.first >= n && blockIdx.x != 0) {  // beyond the live ghosts
+    if (i < sd[s].cap) {
+      keys[bbase[s] + i] = 0xFFFFFFFFu;
+      vals[bbase[s] + i] = (int)gi;
+    }
+    return;
+  }
+  const double cutoff = st[s].sort_cutoff;
+  double x[D];
+#pragma unroll
+  for (int d = 0; d < D; ++d) x[d] = i < n ? xs[d][gi] : 0.0;
+  if (inl) {
+    // the key bases, found by every workgroup for itself (the first stores them)
+    if (w == 0) {
+      unsigned long long range = 0;
+      int q = -1;
+      KeySpace K;
+      if (lane < nlist) {
+        q = list[lane];
+        const bool live = n_dev[q] > 0;
+        range = key_space(D, st[q].sort_cutoff, bbmin, bbmax, rs, q, K);
+        if (!live) range = 0;
+        if (blockIdx.x == 0)
+          key_space_store(K, q, live, bbmin, bbmax, kmin, kmax, krange, flags, sysfault);
+      }
+      unsigned long long inc = range;
+      for (int o = 1; o < 64; o <<= 1) {
+        const unsigned long long u = __shfl_up(inc, o, 64);
+        if (lane >= o) inc += u;
+      }
+      if (q >= 0 && blockIdx.x == 0) kbase[q] = (unsigned)(inc - range);
+      if (q == s) {
+        for (int d = 0; d < 3; ++d) {
+          s_kmin[d] = K.kmin[d];
+          s_kr[d] = K.kr[d];
+        }
+        s_base = (unsigned)(inc - range);
+      }
+      if (lane == 63) {
+        s_total = (unsigned)(inc < 0xFFFFFFFFull ? inc : 0xFFFFFFFFull);
+        if (blockIdx.x == 0) key_flags(inc, flags);
+      }
+    }
+  } else if (threadIdx.x == 0) {
+    for (int d = 0; d < 3; ++d) {
+      s_kmin[d] = kmin[s * 3 + d];
+      s_kr[d] = krange[s * 3 + d];
+    }
+    s_base = kbase[s];
+    s_total = (unsigned)flags[2];
+  }
+  __syncthreads();
+  const bool faulted = s_kr[0] == 0u;
+  auto key_of = [&](const double *p) {
+    unsigned k = 0;
+#pragma unroll
+    for (int d = 0; d < D; ++d)
+      k = k * s_kr[d] + (unsigned)(key_comp(p[d], cutoff) - s_kmin[d]);
+    return s_base + (faulted ? 0u : k);
+  };
+  unsigned key = 0xFFFFFFFFu, kn = 0u;
+  if (i < n) {
+    key = key_of(x);
+    // the key after the workgroup's last particle, the only neighbour key
+    // that no thread of this workgroup computes for itself
+    if (threadIdx.x == GR_BLOCK - 1 && i + 1 < n) {
+      double xn[D];
+#pragma unroll
+      for (int d = 0; d < D; ++d) xn[d] = xs[d][gi + 1];
+      kn = key_of(xn);
+    }
+  }
+  if (lane == 0) kw[w] = key;
+  __syncthreads();
+  unsigned k2 = __shfl_down(key, 1, 64);
+  if (lane == 63) k2 = w + 1 < GR_BLOCK / 64 ? kw[w + 1] : kn;
+  const bool inv = i + 1 < n && k2 < key;
+  if (__syncthreads_or(inv) && threadIdx.x == 0 && ld_dev(&flags[0]) == 0) atomicOr(&flags[0], 1);
+  if (i >= sd[s].cap) key = 0xFFFFFFFFu;
+  const bool valid = i < n;
+  const int p = bbase[s] + i;
+  if (i < sd[s].cap) {
+    keys[p] = key;
+    vals[p] = (int)gi;
+  }
+  if (s_total > cap) return;  // sorted by k_key_place's workgroup
+  int len;
+  int head = run_head(key, valid, len);
+  unsigned r0 = 0;
+  if (valid && head == lane) r0 = atomicAdd(&count[key], (unsigned)len);
+  r0 = __shfl(r0, head, 64);
+  if (valid) rank[p] = faulted ? (unsigned)i : r0 + (unsigned)(lane - head);
+  head = run_head(key / KT_TILE, valid, len);
+  if (valid && head == lane)
+    atomicAdd(&tsum[key / KT_TILE * KT_REP + blockIdx.x % KT_REP], (unsigned)len);
+}
+
+// Starts of KT_TILE keys: the sums of the tiles before them, then a scan.
+__global__ void __launch_bounds__(GR_BLOCK)
+    k_key_scan(unsigned *count, const unsigned *tsum, unsigned *start, const int *flags,
+               unsigned cap) {
+  const unsigned total = (unsigned)flags[2];
+  const unsigned tile = blockIdx.x;
+  if (total > cap || tile * KT_TILE > total) return;
+  __shared__ unsigned wsum[GR_BLOCK / 64], psum[GR_BLOCK / 64];
+  const int t = threadIdx.x, lane = t & 63, w = t >> 6;
+  uint4 *c4 = reinterpret_cast<uint4 *>(count + (size_t)tile * KT_TILE) + t;
+  const uint4 c = *c4;
+  *c4 = make_uint4(0u, 0u, 0u, 0u);
+  if (flags[0] == 0) return;  // already in order: nothing reads the starts
+  unsigned before = 0;
+  for (unsigned k = t; k < tile * KT_REP; k += GR_BLOCK) before += tsum[k];
+  const unsigned sum = c.x + c.y + c.z + c.w;
+  unsigned inc = sum;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const unsigned u = __shfl_up(inc, o, 64);
+    if (lane >= o) inc += u;
+    before += __shfl_xor(before, o, 64);
+  }
+  if (lane == 63) {
+    wsum[w] = inc;
+    psum[w] = before;
+  }
+  __syncthreads();
+  unsigned run = inc - sum;
+  for (int q = 0; q < GR_BLOCK / 64; ++q) run += psum[q] + (q < w ? wsum[q] : 0u);
+  reinterpret_cast<uint4 *>(start + (size_t)tile * KT_TILE)[t] =
+      make_uint4(run, run + c.x, run + c.x + c.y, run + c.x + c.y + c.z);
+}
+
+// Stable radix sort of N pairs by one wavefront, in place with (k1, v1) as the
+// other buffer: four 8-bit passes.
+__device__ void radix_one_wave(unsigned *k0, int *v0, unsigned *k1, int *v1, int N,
+                               unsigned *base) {
+  const int lane = threadIdx.x & 63;
+  const unsigned long long lt = lane == 0 ? 0ull : (~0ull >> (64 - lane));
+  for (int pass = 0; pass < 4; ++pass) {
+    const int shift = 8 * pass;
+    unsigned *ki = pass & 1 ? k1 : k0, *ko = pass & 1 ? k0 : k1;
+    int *vi = pass & 1 ? v1 : v0, *vo = pass & 1 ? v0 : v1;
+    for (int d = lane; d < 256; d += 64) base[d] = 0u;
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+    for (int e = lane; e < N; e += 64) atomicAdd(&base[(ki[e] >> shift) & 255u], 1u);
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+    unsigned carry = 0;
+    for (int d0 = 0; d0 < 256; d0 += 64) {
+      const unsigned c = base[d0 + lane];
+      unsigned inc = c;
+      for (int o = 1; o < 64; o <<= 1) {
+        const unsigned u = __shfl_up(inc, o, 64);
+        if (lane >= o) inc += u;
+      }
+      base[d0 + lane] = carry + inc - c;
+      carry += __shfl(inc, 63, 64);
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+    for (int e0 = 0; e0 < N; e0 += 64) {
+      const int e = e0 + lane;
+      const bool valid = e < N;
+      const unsigned k = valid ? ki[e] : 0u;
+      const int v = valid ? vi[e] : 0;
+      const unsigned d = (k >> shift) & 255u;
+      unsigned long long m = __ballot(valid);
+      for (int q = 0; q < 8; ++q) {
+        const unsigned long long bal = __ballot((d >> q) & 1u);
+        m &= ((d >> q) & 1u) ? bal : ~bal;
+      }
+      const unsigned at = base[d];
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+      if (valid) {
+        const unsigned r = (unsigned)__popcll(m & lt);
+        ko[at + r] = k;
+        vo[at + r] = v;
+        if (r == 0) base[d] = at + (unsigned)__popcll(m);
+      }
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+    }
+    // the next pass reads what this one wrote to memory
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "agent");
+  }
+}
+
+// Every particle to its cell's slots (former place and key); also the tile
+// sums and the listed systems' bounds back to their initial values.
+__global__ void __launch_bounds__(GR_BLOCK)
+    k_key_place(const SysDesc *sd, const int *n_dev, const Blk *blk, const int *bbase, unsigned *keys,
+                int *vals, unsigned *keys2, int *vals2, const unsigned *rank,
+                const unsigned *start, unsigned *tsum, int ntile, int N, const int *list,
+                int nlist, long long *bbmin, long long *bbmax, int rs, int *flags,
+                unsigned cap) {
+  __shared__ unsigned base[256];
+  const int nthr = (int)gridDim.x * GR_BLOCK, me = (int)blockIdx.x * GR_BLOCK + threadIdx.x;
+  for (int k = me; k < ntile * KT_REP; k += nthr) tsum[k] = 0u;
+  for (int t = me; t < nlist * 3 * GR_BB_REP; t += nthr) {
+    const int r = t / (nlist * 3), e = t % (nlist * 3);
+    const int at = (r + 1) * rs + list[e / 3] * 3 + e % 3;
+    bbmin[at] = LLONG_MAX;
+    bbmax[at] = LLONG_MIN;
+  }
+  if (flags[0] == 0) return;
+  if ((unsigned)flags[2] > cap) {
+    if (blockIdx.x == 0 && threadIdx.x < 64) radix_one_wave(keys, vals, keys2, vals2, N, base);
+    return;
+  }
+  const Blk b = blk[blockIdx.x];
+  const int s = b.item;
+  const int i = b.first + threadIdx.x;
+  if (i >= n_dev[s]) return;
+  const int p = bbase[s] + i;
+  const unsigned key = keys[p];
+  const unsigned slot = start[key] + rank[p];
+  // the counts place every particle below N; a slot beyond it is reported,
+  // never written
+  if (slot >= (unsigned)N) {
+    atomicOr(&flags[1], 16);
+    return;
+  }
+  keys2[slot] = key;
+  vals2[slot] = (int)(sd[s].off + i);
+}
+
+// Slot p of the sorted order: the particle placed there (its pool index) and
+// the slot its rank in the cell gives it.
+__device__ __forceinline__ int key_slot(int p, const int *vals, const unsigned *keys2,
+                                        const int *vals2, const unsigned *start, const int *flags,
+                                        unsigned cap, int &slot) {
+  slot = p;
+  if ((unsigned)flags[2] > cap) return vals[p];
+  const int v = vals2[p];
+  const unsigned k = keys2[p];
+  const int a = (int)start[k], e = (int)start[k + 1];
+  int r = 0;
+  for (int j = a; j < e; j += KT_RANKS) {
+    int u[KT_RANKS];
+#pragma unroll
+    for (int q = 0; q < KT_RANKS; ++q) u[q] = vals2[j + q < e ? j + q : e - 1];
+#pragma unroll
+    for (int q = 0; q < KT_RANKS; ++q) r += j + q < e && u[q] < v ? 1 : 0;
+  }
+  slot = a + r;
+  return v;
+}
+
+// ---------------------------------------------------------------------------
 // Permutation of real systems (src/Sorting.jl:88-105): pool A → pool B for
 // every real particle; identity where the system is not sorted this step.
 // ---------------------------------------------------------------------------
@@ -582,19 +934,29 @@ __device__ inline double eos_p(int kind, double rho, double rho0, double gamma, 
 // mult ½): one pass over the particles instead of two.  PACK (FP32, with
 // HALF): their compact partner records too, as k_pack writes them from the
 // half-step state (1: ρ and p, 2: 1/ρ and p/ρ²).
-template <typename R, int D, bool HALF, int PACK = 0>
+// TAB: the order comes from the counting sort (each thread takes the particle
+// of one slot to its place in the cell), else from the radix sort.
+template <typename R, int D, bool HALF, int PACK = 0, bool TAB = false>
 __global__ void k_permute_real(Pool<R> A, Pool<R> B, const SysDesc *sd, const Blk *blk,
                                const int *bbase, const int *vals, const int *vals2,
                                const int *flags, int vadj, const StepSys *st,
-                               const int *halfsys) {
+                               const int *halfsys, KeyTable kt) {
   const Blk b = blk[blockIdx.x];
   const int s = b.item;
   const int i = b.first + threadIdx.x;
   const SysDesc S = sd[s];
   if (i >= S.cap) return;
-  const int64_t dst = S.off + i;
+  int64_t dst = S.off + i;
   int64_t src = dst;
-  if (flags[0] != 0 && bbase[s] >= 0) src = radix_sorted_vals(vals, vals2, flags)[bbase[s] + i];
+  if constexpr (TAB) {
+    if (flags[0] != 0 && bbase[s] >= 0 && kt.krange[s * 3] != 0u) {  // not a faulted system
+      int slot;
+      src = key_slot(bbase[s] + i, vals, kt.keys2, vals2, kt.start, flags, kt.cap, slot);
+      dst = S.off + (slot - bbase[s]);
+    }
+  } else {
+    if (flags[0] != 0 && bbase[s] >= 0) src = radix_sorted_vals(vals, vals2, flags)[bbase[s] + i];
+  }
   const bool half = HALF && halfsys[s] != 0;
   // fields this step overwrites before reading them are not moved (only with
   // the half step, which has read the old rates here)
@@ -710,7 +1072,8 @@ __device__ inline bool ghost_qualifies(const double *xi, const Bnd &B, double gc
 template <int D>
 __global__ void __launch_bounds__(GR_BLOCK)
     k_ghost_count(XP x, const SysDesc *sd, const Bnd *bnd, const Blk *blk, const int *gslot,
-                  int *cnt) {
+                  int *cnt, int *flags) {
+  if (flags && blockIdx.x == 0 && threadIdx.x == 0) flags[0] = 0;  // for the ghosts' sort
   const Blk b = blk[blockIdx.x];
   const int g = b.item;
   const SysDesc G = sd[g];
@@ -730,15 +1093,31 @@ __global__ void __launch_bounds__(GR_BLOCK)
   }
 }
 
+// Sum of v[0 .. n) by the workgroup.
+__device__ inline int block_sum(const int *v, int n, int *wsum) {
+  const int t = threadIdx.x, lane = t & 63, w = t >> 6;
+  int a = 0;
+  for (int k = t; k < n; k += GR_BLOCK) a += v[k];
+  for (int o = 32; o > 0; o >>= 1) a += __shfl_xor(a, o, 64);
+  if (lane == 0) wsum[w] = a;
+  __syncthreads();
+  int r = 0;
+  for (int q = 0; q < GR_BLOCK / 64; ++q) r += wsum[q];
+  __syncthreads();
+  return r;
+}
+
 // Mirrored position, source index, boundary index, and the boundary whose
 // normal slot k keeps (normals are not permuted by the ghost sort,
-// src/Sorting.jl:33-40).
+// src/Sorting.jl:33-40); also the ghosts' position bounds.  `scan`: the
+// exclusive scan of the slots, or null: a workgroup that holds ghosts adds up
+// the slots before its own (a ghost system has a few hundred).
 template <int D>
 __global__ void __launch_bounds__(GR_BLOCK)
     k_ghost_scatter(XP x, XPW gx, int *gidx, int *gbnd, int *gnrm, const SysDesc *sd,
-                    const Bnd *bnd, const Blk *blk, const int *gslot, const int *scan,
-                    int *n_dev) {
-  __shared__ int wc[GR_BLOCK / 64];
+                    const Bnd *bnd, const Blk *blk, const int *gslot, const int *cnt,
+                    const int *scan, int *n_dev, long long *bbmin, long long *bbmax, int rs) {
+  __shared__ int wc[GR_BLOCK / 64], wsum[GR_BLOCK / 64];
   const Blk b = blk[blockIdx.x];
   const int g = b.item;
   const SysDesc G = sd[g];
@@ -752,8 +1131,17 @@ __global__ void __launch_bounds__(GR_BLOCK)
   for (int d = 0; d < D; ++d) xi[d] = x[d][gi];
   const int nsb = (S.cap + GR_BLOCK - 1) / GR_BLOCK, sb = b.first / GR_BLOCK;
   const int s0 = gslot[g];
-  const int first = scan[s0];
-  if (sb == 0 && threadIdx.x == 0) n_dev[g] = scan[s0 + G.nb * nsb] - first;
+  if (sb == 0) {
+    const int tot = scan ? scan[s0 + G.nb * nsb] - scan[s0] : block_sum(cnt + s0, G.nb * nsb, wsum);
+    if (threadIdx.x == 0) n_dev[g] = tot;
+  }
+  long long mn[D], mx[D];
+#pragma unroll
+  for (int d = 0; d < D; ++d) {
+    mn[d] = LLONG_MAX;
+    mx[d] = LLONG_MIN;
+  }
+  bool any = false;
   for (int bi = 0; bi < G.nb; ++bi) {
     const Bnd B = bnd[G.bnd + bi];
     double da;
@@ -761,37 +1149,75 @@ __global__ void __launch_bounds__(GR_BLOCK)
     const unsigned long long bal = __ballot(q);
     if (lane == 0) wc[w] = __popcll(bal);
     __syncthreads();
-    int woff = 0;
-    for (int v = 0; v < w; ++v) woff += wc[v];
+    int woff = 0, tot = 0;
+    for (int v = 0; v < GR_BLOCK / 64; ++v) {
+      woff += v < w ? wc[v] : 0;
+      tot += wc[v];
+    }
     __syncthreads();  // wc is written again for the next boundary
+    if (tot == 0) continue;  // uniform over the workgroup
+    any = true;
+    const int k0 = scan ? scan[s0 + bi * nsb + sb] - scan[s0]
+                        : block_sum(cnt + s0, bi * nsb + sb, wsum);
     if (q) {
-      const int k = scan[s0 + bi * nsb + sb] - first + woff +
-                    __popcll(bal & ((1ull << lane) - 1ull));
+      const int k = k0 + woff + __popcll(bal & ((1ull << lane) - 1ull));
       const int64_t go = G.off + k;
 #pragma unroll
-      for (int d = 0; d < D; ++d) gx[d][go] = xi[d] - (2.0 * da) * B.n[d];
+      for (int d = 0; d < D; ++d) {
+        const double xm = xi[d] - (2.0 * da) * B.n[d];
+        gx[d][go] = xm;
+        const long long o = ord_d(xm);
+        mn[d] = o < mn[d] ? o : mn[d];
+        mx[d] = o > mx[d] ? o : mx[d];
+      }
       gidx[go] = i;
       gbnd[go] = bi;
       gnrm[go] = bi;
+    }
+  }
+  if (!bbmin || !any) return;
+  bbmin += (1 + blockIdx.x % GR_BB_REP) * rs;
+  bbmax += (1 + blockIdx.x % GR_BB_REP) * rs;
+#pragma unroll
+  for (int d = 0; d < D; ++d) {
+    const long long a = wave_red_ll<false>(mn[d]), z = wave_red_ll<true>(mx[d]);
+    if (lane == 0 && a != LLONG_MAX) {
+      if (a < ld_dev(&bbmin[g * 3 + d])) atomicMin(&bbmin[g * 3 + d], a);
+      if (z > ld_dev(&bbmax[g * 3 + d])) atomicMax(&bbmax[g * 3 + d], z);
     }
   }
 }
 
 // Ghost sort permutation: generation scratch → pool (x, idx_original,
 // idx_boundary).
-template <int D>
+template <int D, bool TAB>
 __global__ void k_permute_ghost(XP gxs, const int *gidx_s, const int *gbnd_s, XPW x, int *gidx,
                                 int *gbnd, const SysDesc *sd, const int *n_dev, const Blk *blk,
                                 const int *bbase, const int *vals, const int *vals2,
-                                const int *flags) {
+                                const int *flags, KeyTable kt) {
   const Blk b = blk[blockIdx.x];
   const int g = b.item;
   const int k = b.first + threadIdx.x;
   const SysDesc G = sd[g];
   if (k >= n_dev[g]) return;
-  const int64_t dst = G.off + k;
+  int64_t dst = G.off + k;
   int64_t src = dst;
-  if (flags[0] != 0) src = radix_sorted_vals(vals, vals2, flags)[bbase[g] + k];
+  if constexpr (TAB) {
+    if (flags[0] != 0 && kt.krange[g * 3] != 0u) {
+      // the live ghosts of the systems listed before this one
+      int p0 = 0;
+      if ((unsigned)flags[2] > kt.cap) {
+        for (int q = 0; q < kt.nlist && kt.list[q] != g; ++q) p0 += n_dev[kt.list[q]];
+      } else {
+        p0 = (int)kt.start[kt.kbase[g]];
+      }
+      int slot;
+      src = key_slot(p0 + k, vals, kt.keys2, vals2, kt.start, flags, kt.cap, slot);
+      dst = G.off + (slot - p0);
+    }
+  } else {
+    if (flags[0] != 0) src = radix_sorted_vals(vals, vals2, flags)[bbase[g] + k];
+  }
 #pragma unroll
   for (int d = 0; d < D; ++d) x[d][dst] = gxs[d][src];
   gidx[dst] = gidx_s[src];
@@ -1762,16 +2188,16 @@ static inline unsigned nb_of(long long n, int per) { return (unsigned)((n + per 
 
 void launch_key_minmax(hipStream_t s, XP xs, const SysDesc *sd, const int *n, const Blk *blk,
                        int nblk, int D, long long *bbmin, long long *bbmax, int rs,
-                       const int *list, int nlist, bool fold) {
+                       const int *list, int nlist, bool fold, int *flags) {
   if (nblk > 0) {
     // 8 table entries (2048 particles) per workgroup: enough workgroups to
     // fill the chip, few enough that the per-system atomics stay cheap
     constexpr int per = 8;
     const unsigned g = nb_of(nblk, per);
     if (D == 2)
-      k_key_minmax<2, per><<<g, GR_BLOCK, 0, s>>>(xs, sd, n, blk, nblk, bbmin, bbmax, rs);
+      k_key_minmax<2, per><<<g, GR_BLOCK, 0, s>>>(xs, sd, n, blk, nblk, bbmin, bbmax, rs, flags);
     else
-      k_key_minmax<3, per><<<g, GR_BLOCK, 0, s>>>(xs, sd, n, blk, nblk, bbmin, bbmax, rs);
+      k_key_minmax<3, per><<<g, GR_BLOCK, 0, s>>>(xs, sd, n, blk, nblk, bbmin, bbmax, rs, flags);
   }
   if (fold && nlist > 0)
     k_bb_fold<<<nb_of(nlist * 3, GR_BLOCK), GR_BLOCK, 0, s>>>(list, nlist, bbmin, bbmax, rs);
@@ -1786,7 +2212,50 @@ void launch_key_base(hipStream_t s, const int *list, int nlist, int D, int pad, 
                      const StepSys *st, long long *bbmin, long long *bbmax, int rs, int *kmin,
                      int *kmax, unsigned *kbase, unsigned *krange, int *flags, int *sysfault) {
   k_key_base<<<1, KB_THREADS, 0, s>>>(list, nlist, D, pad, n, st, bbmin, bbmax, rs, kmin, kmax,
-                                      kbase, krange, flags, sysfault);
+                                      kbase, krange, flags, sysfault, 0);
+}
+size_t key_table_bytes(int64_t ntile) {
+  return (size_t)ntile * (KT_TILE * 2 + KT_REP) * sizeof(unsigned);
+}
+int key_table_tile() { return KT_TILE; }
+void launch_key_sort(hipStream_t s, XP xs, const SysDesc *sd, const int *n, const StepSys *st,
+                     const Blk *blk, int nblk, const int *bbase, int D, const int *list, int nlist,
+                     int N, long long *bbmin, long long *bbmax, int rs, int *kmin, int *kmax,
+                     unsigned *krange, unsigned *kbase, unsigned *keys, int *vals,
+                     unsigned *keys2, int *vals2, unsigned *rank, int *flags, int *sysfault,
+                     unsigned *table, int tiles, int ntile) {
+  if (nblk <= 0) return;
+  unsigned *count = table, *start = table + (size_t)tiles * KT_TILE;
+  unsigned *tsum = table + (size_t)tiles * KT_TILE * 2;
+  const unsigned cap = (unsigned)ntile * KT_TILE - 1u;
+  const int inl = nlist <= KC_SYSTEMS && nblk <= KC_BLOCKS;
+  if (!inl)
+    k_key_base<<<1, KB_THREADS, 0, s>>>(list, nlist, D, 0, n, st, bbmin, bbmax, rs, kmin, kmax,
+                                        kbase, krange, flags, sysfault, 1);
+  if (D == 2)
+    k_key_count<2><<<nblk, GR_BLOCK, 0, s>>>(xs, sd, n, st, blk, bbase, list, nlist, bbmin, bbmax,
+                                             rs, kmin, kmax, krange, kbase, keys, vals, rank,
+                                             flags, sysfault, count, tsum, cap, inl);
+  else
+    k_key_count<3><<<nblk, GR_BLOCK, 0, s>>>(xs, sd, n, st, blk, bbase, list, nlist, bbmin, bbmax,
+                                             rs, kmin, kmax, krange, kbase, keys, vals, rank,
+                                             flags, sysfault, count, tsum, cap, inl);
+  k_key_scan<<<ntile, GR_BLOCK, 0, s>>>(count, tsum, start, flags, cap);
+  k_key_place<<<nblk, GR_BLOCK, 0, s>>>(sd, n, blk, bbase, keys, vals, keys2, vals2, rank, start,
+                                        tsum, ntile, N, list, nlist, bbmin, bbmax, rs, flags, cap);
+}
+KeyTable key_table_view(unsigned *table, int tiles, int ntile, const unsigned *keys2,
+                        const unsigned *krange, const unsigned *kbase, const int *list,
+                        int nlist) {
+  KeyTable kt;
+  kt.keys2 = keys2;
+  kt.start = table + (size_t)tiles * KT_TILE;
+  kt.krange = krange;
+  kt.kbase = kbase;
+  kt.list = list;
+  kt.nlist = nlist;
+  kt.cap = (unsigned)ntile * KT_TILE - 1u;
+  return kt;
 }
 void launch_key_write(hipStream_t s, XP xs, const SysDesc *sd, const int *n, const StepSys *st,
                       const Blk *blk, int nblk, const int *bbase, int D, const int *kmin,
@@ -1821,54 +2290,58 @@ template <typename R>
 void launch_permute_real(hipStream_t s, const Pool<R> &A, const Pool<R> &B, const SysDesc *sd,
                          const Blk *blk, int nblk, const int *bbase, const int *vals,
                          const int *vals2, const int *flags, int vadj, int D, const StepSys *st,
-                         const int *halfsys, int pack) {
+                         const int *halfsys, int pack, const KeyTable *kt) {
   if (nblk <= 0) return;
-  if (halfsys) {
-    auto go = [&](auto dc, auto pc) {
-      constexpr int DD = decltype(dc)::value, PP = decltype(pc)::value;
-      k_permute_real<R, DD, true, PP><<<nblk, GR_BLOCK, 0, s>>>(A, B, sd, blk, bbase, vals,
-                                                                vals2, flags, vadj, st, halfsys);
-    };
-    using I2 = std::integral_constant<int, 2>;
-    using I3 = std::integral_constant<int, 3>;
-    using P0 = std::integral_constant<int, 0>;
-    using P1 = std::integral_constant<int, 1>;
-    using P2 = std::integral_constant<int, 2>;
-    if (sizeof(R) != 4) pack = 0;
-    if (D == 2) {
-      if (pack == 2) go(I2{}, P2{});
-      else if (pack == 1) go(I2{}, P1{});
-      else go(I2{}, P0{});
-    } else {
-      if (pack == 2) go(I3{}, P2{});
-      else if (pack == 1) go(I3{}, P1{});
-      else go(I3{}, P0{});
-    }
-    return;
-  }
-  if (D == 2)
-    k_permute_real<R, 2, false><<<nblk, GR_BLOCK, 0, s>>>(A, B, sd, blk, bbase, vals, vals2,
-                                                          flags, vadj, st, halfsys);
+  using I2 = std::integral_constant<int, 2>;
+  using I3 = std::integral_constant<int, 3>;
+  using P0 = std::integral_constant<int, 0>;
+  using P1 = std::integral_constant<int, 1>;
+  using P2 = std::integral_constant<int, 2>;
+  auto go = [&](auto dc, auto pc, auto hc, auto tc) {
+    constexpr int DD = decltype(dc)::value, PP = decltype(pc)::value;
+    constexpr bool H = decltype(hc)::value, T = decltype(tc)::value;
+    k_permute_real<R, DD, H, PP, T><<<nblk, GR_BLOCK, 0, s>>>(
+        A, B, sd, blk, bbase, vals, vals2, flags, vadj, st, halfsys, kt ? *kt : KeyTable{});
+  };
+  auto tab = [&](auto dc, auto pc, auto hc) {
+    if (kt)
+      go(dc, pc, hc, std::true_type{});
+    else
+      go(dc, pc, hc, std::false_type{});
+  };
+  auto dim = [&](auto pc, auto hc) {
+    if (D == 2)
+      tab(I2{}, pc, hc);
+    else
+      tab(I3{}, pc, hc);
+  };
+  if (sizeof(R) != 4) pack = 0;
+  if (!halfsys)
+    dim(P0{}, std::false_type{});
+  else if (pack == 2)
+    dim(P2{}, std::true_type{});
+  else if (pack == 1)
+    dim(P1{}, std::true_type{});
   else
-    k_permute_real<R, 3, false><<<nblk, GR_BLOCK, 0, s>>>(A, B, sd, blk, bbase, vals, vals2,
-                                                          flags, vadj, st, halfsys);
+    dim(P0{}, std::true_type{});
 }
 template void launch_permute_real<float>(hipStream_t, const Pool<float> &, const Pool<float> &,
                                          const SysDesc *, const Blk *, int, const int *,
                                          const int *, const int *, const int *, int, int,
-                                         const StepSys *, const int *, int);
+                                         const StepSys *, const int *, int, const KeyTable *);
 template void launch_permute_real<double>(hipStream_t, const Pool<double> &,
                                           const Pool<double> &, const SysDesc *, const Blk *,
                                           int, const int *, const int *, const int *, const int *,
-                                          int, int, const StepSys *, const int *, int);
+                                          int, int, const StepSys *, const int *, int,
+                                          const KeyTable *);
 
 void launch_ghost_count(hipStream_t s, XP x, const SysDesc *sd, const Bnd *bnd, const Blk *blk,
-                        int nblk, const int *gslot, int D, int *cnt) {
+                        int nblk, const int *gslot, int D, int *cnt, int *flags) {
   if (nblk <= 0) return;
   if (D == 2)
-    k_ghost_count<2><<<nblk, GR_BLOCK, 0, s>>>(x, sd, bnd, blk, gslot, cnt);
+    k_ghost_count<2><<<nblk, GR_BLOCK, 0, s>>>(x, sd, bnd, blk, gslot, cnt, flags);
   else
-    k_ghost_count<3><<<nblk, GR_BLOCK, 0, s>>>(x, sd, bnd, blk, gslot, cnt);
+    k_ghost_count<3><<<nblk, GR_BLOCK, 0, s>>>(x, sd, bnd, blk, gslot, cnt, flags);
 }
 void launch_scan(hipStream_t s, const int *in, int *out, int *bsum, int N) {
   const int nb = (int)nb_of(N > 0 ? N : 1, SCAN_TILE);
@@ -1879,26 +2352,36 @@ void launch_scan(hipStream_t s, const int *in, int *out, int *bsum, int N) {
 int scan_block_count(int N) { return (int)nb_of(N > 0 ? N : 1, SCAN_TILE); }
 void launch_ghost_scatter(hipStream_t s, XP x, XPW gx, int *gidx, int *gbnd, int *gnrm,
                           const SysDesc *sd, const Bnd *bnd, const Blk *blk, int nblk,
-                          const int *gslot, const int *scan, int D, int *n) {
+                          const int *gslot, const int *cnt, const int *scan, int D, int *n,
+                          long long *bbmin, long long *bbmax, int rs) {
   if (nblk <= 0) return;
   if (D == 2)
     k_ghost_scatter<2><<<nblk, GR_BLOCK, 0, s>>>(x, gx, gidx, gbnd, gnrm, sd, bnd, blk, gslot,
-                                                 scan, n);
+                                                 cnt, scan, n, bbmin, bbmax, rs);
   else
     k_ghost_scatter<3><<<nblk, GR_BLOCK, 0, s>>>(x, gx, gidx, gbnd, gnrm, sd, bnd, blk, gslot,
-                                                 scan, n);
+                                                 cnt, scan, n, bbmin, bbmax, rs);
 }
 void launch_permute_ghost(hipStream_t s, XP gxs, const int *gidx_s, const int *gbnd_s, XPW x,
                           int *gidx, int *gbnd, const SysDesc *sd, const int *n, const Blk *blk,
                           int nblk, const int *bbase, const int *vals, const int *vals2,
-                          const int *flags, int D) {
+                          const int *flags, int D, const KeyTable *kt) {
   if (nblk <= 0) return;
-  if (D == 2)
-    k_permute_ghost<2><<<nblk, GR_BLOCK, 0, s>>>(gxs, gidx_s, gbnd_s, x, gidx, gbnd, sd, n, blk,
-                                                 bbase, vals, vals2, flags);
+  auto go = [&](auto dc, auto tc) {
+    k_permute_ghost<decltype(dc)::value, decltype(tc)::value><<<nblk, GR_BLOCK, 0, s>>>(
+        gxs, gidx_s, gbnd_s, x, gidx, gbnd, sd, n, blk, bbase, vals, vals2, flags,
+        kt ? *kt : KeyTable{});
+  };
+  auto dim = [&](auto tc) {
+    if (D == 2)
+      go(std::integral_constant<int, 2>{}, tc);
+    else
+      go(std::integral_constant<int, 3>{}, tc);
+  };
+  if (kt)
+    dim(std::true_type{});
   else
-    k_permute_ghost<3><<<nblk, GR_BLOCK, 0, s>>>(gxs, gidx_s, gbnd_s, x, gidx, gbnd, sd, n, blk,
-                                                 bbase, vals, vals2, flags);
+    dim(std::false_type{});
 }
 template <typename R>
 void launch_ghost_kin(hipStream_t s, const Pool<R> &P, const SysDesc *sd, const Bnd *bnd,

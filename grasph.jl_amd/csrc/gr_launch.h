@@ -43,14 +43,14 @@ struct NlistArgs {
   int span = 2;   // lanes whose ranges start within span·(widest range) group
 };
 
-// Position bounds per system and dimension are kept in GR_BB_REP replicas
-// of `rs` entries each (the key pass's atomics are spread over them); replica
-// 0 holds the folded bounds that every reader uses.  launch_key_minmax folds
-// them itself when `fold`, launch_key_base always does.
+// Position bounds per system and dimension: replicas 1 .. GR_BB_REP of `rs`
+// entries each take the bounds pass's atomics, replica 0 holds the folded
+// bounds that every reader uses.  launch_key_minmax folds them itself when
+// `fold`, launch_key_base and launch_key_sort always do.
 #define GR_BB_REP 8
 void launch_key_minmax(hipStream_t s, XP xs, const SysDesc *sd, const int *n, const Blk *blk,
                        int nblk, int D, long long *bbmin, long long *bbmax, int rs,
-                       const int *list, int nlist, bool fold);
+                       const int *list, int nlist, bool fold, int *flags = nullptr);
 void launch_minmax_reset(hipStream_t s, const int *list, int nlist, long long *bbmin,
                          long long *bbmax, int rs);
 void launch_key_base(hipStream_t s, const int *list, int nlist, int D, int pad, const int *n,
@@ -69,26 +69,54 @@ void launch_key_write(hipStream_t s, XP xs, const SysDesc *sd, const int *n,
 void launch_radix_sort(hipStream_t s, unsigned *keys, int *vals, unsigned *keys2, int *vals2,
                        unsigned *rscr, int N, int *flags);
 size_t radix_scratch_bytes(int N);
+// The counting sort of a step (keys, table, placement) after the bounds pass:
+// `table` of key_table_bytes(tiles) bytes, zeroed when allocated, of which this
+// sort uses ntile <= tiles tiles (ntile·key_table_tile() - 1 keys; the layout
+// goes by `tiles`, as sorts of different sizes share the table).  flags[0] must
+// be clear; the permutations take the order by key_table_view.  Replicas 1..
+// of the listed systems' bounds are reset.
+size_t key_table_bytes(int64_t ntile);
+int key_table_tile();
+void launch_key_sort(hipStream_t s, XP xs, const SysDesc *sd, const int *n, const StepSys *st,
+                     const Blk *blk, int nblk, const int *bbase, int D, const int *list, int nlist,
+                     int N, long long *bbmin, long long *bbmax, int rs, int *kmin, int *kmax,
+                     unsigned *krange, unsigned *kbase, unsigned *keys, int *vals,
+                     unsigned *keys2, int *vals2, unsigned *rank, int *flags, int *sysfault,
+                     unsigned *table, int tiles, int ntile);
+struct KeyTable {  // what the permutations read of the counting sort
+  const unsigned *keys2, *start, *krange, *kbase;
+  const int *list;
+  int nlist;
+  unsigned cap;
+};
+KeyTable key_table_view(unsigned *table, int tiles, int ntile, const unsigned *keys2,
+                        const unsigned *krange, const unsigned *kbase, const int *list,
+                        int nlist);
 template <typename R>
 void launch_permute_real(hipStream_t s, const Pool<R> &A, const Pool<R> &B, const SysDesc *sd,
                          const Blk *blk, int nblk, const int *bbase, const int *vals,
                          const int *vals2, const int *flags, int vadj, int D,
                          const StepSys *st = nullptr, const int *halfsys = nullptr,
-                         int pack = 0);
+                         int pack = 0, const KeyTable *kt = nullptr);
 // ghost generation: per-(boundary, source block) counts at gslot[g] + ...,
-// then the scatter at the counts' exclusive scan
+// then the scatter at the counts' exclusive scan (`scan` null: each workgroup
+// adds up the counts itself); bbmin/bbmax: also the ghosts' bounds; flags: also
+// clear the sort's flags
 void launch_ghost_count(hipStream_t s, XP x, const SysDesc *sd, const Bnd *bnd,
-                        const Blk *blk, int nblk, const int *gslot, int D, int *cnt);
+                        const Blk *blk, int nblk, const int *gslot, int D, int *cnt,
+                        int *flags = nullptr);
 void launch_scan(hipStream_t s, const int *in, int *out, int *bsum, int N);
 int scan_block_count(int N);
 void launch_ghost_scatter(hipStream_t s, XP x, XPW gx, int *gidx,
                           int *gbnd, int *gnrm, const SysDesc *sd, const Bnd *bnd, const Blk *blk,
-                          int nblk, const int *gslot, const int *scan, int D, int *n);
+                          int nblk, const int *gslot, const int *cnt, const int *scan, int D,
+                          int *n, long long *bbmin = nullptr, long long *bbmax = nullptr,
+                          int rs = 0);
 void launch_permute_ghost(hipStream_t s, XP gxs, const int *gidx_s,
                           const int *gbnd_s, XPW x, int *gidx, int *gbnd,
                           const SysDesc *sd, const int *n, const Blk *blk, int nblk,
                           const int *bbase, const int *vals, const int *vals2, const int *flags,
-                          int D);
+                          int D, const KeyTable *kt = nullptr);
 template <typename R>
 void launch_ghost_kin(hipStream_t s, const Pool<R> &P, const SysDesc *sd, const Bnd *bnd,
                       const int *n, const Blk *blk, int nblk, int D);
