@@ -403,15 +403,15 @@ struct gr_ctx {
   DBuf d_sysfault;  // per system: GR_FAULT_* bits raised by the step's kernels
   int bb_rs = 0;  // entries per replica of d_bbmin / d_bbmax (GR_BB_REP + 1 replicas)
   bool bb_valid = false;  // d_bbmin / d_bbmax hold the bounds of a step's key pass
-  DBuf d_grids, d_carr, d_cellsz, d_inter_sys, d_inter_carr, cells;
+  DBuf d_grids, d_carr, d_cellsz, d_inter_sys, d_inter_carr, cells, ctile;
   std::vector<CellArr> carr;
   int64_t cells_cap = 0;
   std::vector<StepSys> stepsys;
   // sort / scan scratch
-  DBuf keys, vals, keys2, vals2, krank, hist, cand, cand_scan, scan_bsum, bagg;
+  DBuf keys, vals, keys2, vals2, krank, hist, cand, cand_scan, scan_bsum;
   DBuf ktable;          // the counting sort's table (key_table_bytes)
   int ktable_tiles = 0;
-  int64_t sort_cap = 0, cand_cap = 0, cellblk_cap = 0;
+  int64_t sort_cap = 0, cand_cap = 0;
   DBuf d_pairs;
   DBuf lidx, lcnt;
   int64_t lidx_cap = 0, lcnt_cap = 0;
@@ -1130,6 +1130,14 @@ void drop_graphs(gr_ctx *c) {
       }
 }
 
+// The cell pool and its tile flags, as large as the arrays in use.
+void size_cells(gr_ctx *c) {
+  const size_t n = (size_t)std::max<int64_t>(c->cells_cap, 1);
+  const size_t nt = (size_t)cell_tiles((int64_t)n);
+  if (n * 4 > c->cells.bytes) c->cells.alloc(n * 4);
+  if (nt * 4 > c->ctile.bytes) c->ctile.alloc(nt * 4);
+}
+
 // Allocate cell arrays of the interactions that have none yet.
 void ensure_cells(gr_ctx *c, const std::vector<int> &inters, const std::vector<int> &union_sys) {
   bool any = false;
@@ -1175,8 +1183,7 @@ void ensure_cells(gr_ctx *c, const std::vector<int> &inters, const std::vector<i
   // grow the cell pool (grids are rebuilt every step, so no copy); captured
   // graphs of other plans hold the old table and pool pointers
   drop_graphs(c);
-  if ((size_t)std::max<int64_t>(c->cells_cap, 1) * 4 > c->cells.bytes)
-    c->cells.alloc(std::max<int64_t>(c->cells_cap, 1) * 4);
+  size_cells(c);
   c->d_carr.upload(c->carr, c->stream);
   const int ni = (int)c->inter.size();
   std::vector<int2> isys(ni), icarr(ni);
@@ -1235,10 +1242,6 @@ void plan_grids(gr_ctx *c, Plan &P, const std::vector<int> &inters,
   P.blk_mark.upload(mb, c->stream);
   P.nblk_cells = (int)cb.size();
   P.nblk_mark = (int)mb.size();
-  if ((int64_t)cb.size() + 1 > c->cellblk_cap) {
-    c->bagg.alloc((cb.size() + 1) * 4);
-    c->cellblk_cap = cb.size() + 1;
-  }
 }
 
 void plan_sort_real(gr_ctx *c, Plan &P, const std::vector<int> &systems) {
@@ -1757,9 +1760,37 @@ void all_real(gr_ctx *c, const Blk *&blk, int &nblk) {
 // Step phases
 // ---------------------------------------------------------------------------
 
+CellsArgs cells_args(gr_ctx *c, const Plan &P) {
+  CellsArgs A;
+  A.cells = c->cells.as<int>();
+  A.tflag = c->ctile.as<int>();
+  A.carr = c->d_carr.as<CellArr>();
+  A.cblk = P.blk_cells.as<Blk>();
+  A.ncblk = P.nblk_cells;
+  A.inter_list = P.d_inter_list.as<int>();
+  A.n_inter = (int)P.inters.size();
+  A.inter_sys = c->d_inter_sys.as<int2>();
+  A.inter_carr = c->d_inter_carr.as<int2>();
+  A.cellsz = c->d_cellsz.as<double>();
+  A.bbmin = c->d_bbmin.as<long long>();
+  A.bbmax = c->d_bbmax.as<long long>();
+  A.n_dev = c->d_n.as<int>();
+  A.grids = c->d_grids.as<Grid>();
+  A.D = c->D;
+  return A;
+}
+
+// Whether the real or ghost sort of a step prepares its cells: the last one,
+// where it is a counting sort.
+bool sort_preps_cells(const Plan &P, bool ghost) {
+  if (P.real_list.empty() || ghost == P.ghost_list.empty()) return false;
+  return (ghost ? P.tiles_ghost : P.tiles_real) > 0;
+}
+
 // The counting sort of a step's real or ghost systems (after their bounds).
-void key_sort(gr_ctx *c, const XP &xs, const DBuf &blk, int nblk, const DBuf &bbase,
-              const DBuf &list, int nlist, int n, int tiles) {
+void key_sort(gr_ctx *c, const Plan &P, const XP &xs, const DBuf &blk, int nblk, const DBuf &bbase,
+              const DBuf &list, int nlist, int n, int tiles, bool cells) {
+  const CellsArgs A = cells_args(c, P);
   launch_key_sort(c->stream, xs, c->d_sd.as<SysDesc>(), c->d_n.as<int>(), c->d_st.as<StepSys>(),
                   blk.as<Blk>(), nblk, bbase.as<int>(), c->D, list.as<int>(), nlist, n,
                   c->d_bbmin.as<long long>(), c->d_bbmax.as<long long>(), c->bb_rs,
@@ -1767,7 +1798,7 @@ void key_sort(gr_ctx *c, const XP &xs, const DBuf &blk, int nblk, const DBuf &bb
                   c->d_kbase.as<unsigned>(), c->keys.as<unsigned>(), c->vals.as<int>(),
                   c->keys2.as<unsigned>(), c->vals2.as<int>(), c->krank.as<unsigned>(),
                   c->d_flags.as<int>(), c->d_sysfault.as<int>(), c->ktable.as<unsigned>(),
-                  c->ktable_tiles, tiles);
+                  c->ktable_tiles, tiles, cells ? &A : nullptr);
 }
 
 // half: also take the leapfrog half step of the plan's integrated systems
@@ -1784,8 +1815,8 @@ void phase_sort_real(gr_ctx *c, Plan &P, bool half = false, int pack = 0) {
                       P.nblk_real, c->D, c->d_bbmin.as<long long>(), c->d_bbmax.as<long long>(),
                       c->bb_rs, P.d_real_list.as<int>(), (int)P.real_list.size(), false,
                       c->d_flags.as<int>());
-    key_sort(c, xs, P.blk_real, P.nblk_real, P.d_bbase_real, P.d_real_list,
-             (int)P.real_list.size(), P.n_real, P.tiles_real);
+    key_sort(c, P, xs, P.blk_real, P.nblk_real, P.d_bbase_real, P.d_real_list,
+             (int)P.real_list.size(), P.n_real, P.tiles_real, sort_preps_cells(P, false));
     all_real(c, arb, arn);
     const KeyTable kt =
         key_table_view(c->ktable.as<unsigned>(), c->ktable_tiles, P.tiles_real, c->keys2.as<unsigned>(),
@@ -1847,8 +1878,8 @@ void phase_ghosts(gr_ctx *c, Plan &P, bool generate, bool sort) {
   }
   if (table) {  // a step: counting sort (the bounds' replicas are reset already)
     const XP gx = xp_gxs(c);
-    key_sort(c, gx, P.blk_ghost, P.nblk_ghost, P.d_bbase_ghost, P.d_ghost_list,
-             (int)P.ghost_list.size(), P.n_ghost, P.tiles_ghost);
+    key_sort(c, P, gx, P.blk_ghost, P.nblk_ghost, P.d_bbase_ghost, P.d_ghost_list,
+             (int)P.ghost_list.size(), P.n_ghost, P.tiles_ghost, sort_preps_cells(P, true));
     const KeyTable kt =
         key_table_view(c->ktable.as<unsigned>(), c->ktable_tiles, P.tiles_ghost, c->keys2.as<unsigned>(),
                        c->d_krange.as<unsigned>(), c->d_kbase.as<unsigned>(),
@@ -1896,18 +1927,14 @@ void mark_grids(gr_ctx *c, const Plan &P) {
   }
 }
 
-void phase_grids(gr_ctx *c, Plan &P) {
+// prepared: the last sort of the step has found the grids and cleared the
+// plan's cell arrays.
+void phase_grids(gr_ctx *c, Plan &P, bool prepared = false) {
   if (P.inters.empty()) return;
-  hipStream_t s = c->stream;
-  launch_grid_params(s, P.d_inter_list.as<int>(), (int)P.inters.size(), c->d_inter_sys.as<int2>(),
-                     c->d_cellsz.as<double>(), c->d_bbmin.as<long long>(),
-                     c->d_bbmax.as<long long>(), c->d_n.as<int>(), c->d_grids.as<Grid>(),
-                     c->d_inter_carr.as<int2>(), c->d_carr.as<CellArr>(), c->D, c->d_flags.as<int>(),
-                     c->d_sysfault.as<int>());
-  launch_cells_build(s, xp_pool(c, c->cur), c->cells.as<int>(),
-                     c->d_carr.as<CellArr>(), c->d_grids.as<Grid>(), c->d_cellsz.as<double>(),
-                     c->d_sd.as<SysDesc>(), c->d_n.as<int>(), P.blk_cells.as<Blk>(), P.nblk_cells,
-                     P.blk_mark.as<Blk>(), P.nblk_mark, c->bagg.as<int>(), c->D);
+  const CellsArgs A = cells_args(c, P);
+  if (!prepared) launch_cells_prep(c->stream, A, c->d_flags.as<int>(), c->d_sysfault.as<int>());
+  launch_cells_build(c->stream, xp_pool(c, c->cur), A, c->d_sd.as<SysDesc>(), P.blk_mark.as<Blk>(),
+                     P.nblk_mark);
 }
 
 template <typename R>
@@ -2099,8 +2126,7 @@ bool grow_cells(gr_ctx *c, const Plan &P) {
   drop_graphs(c);
   c->plans.clear();
   if (!grew) return true;  // the next plan takes larger key tables
-  if ((size_t)std::max<int64_t>(c->cells_cap, 1) * 4 > c->cells.bytes)
-    c->cells.alloc(std::max<int64_t>(c->cells_cap, 1) * 4);
+  size_cells(c);
   c->d_carr.upload(c->carr, c->stream);
   std::fill(c->carr_valid.begin(), c->carr_valid.end(), 0);
   return true;
@@ -2149,7 +2175,7 @@ void run_step(gr_ctx *c, Plan &P, bool cnt, std::vector<hipEvent_t> *ev) {
   rec(1);
   phase_ghosts<R>(c, P, true, true);
   rec(2);
-  phase_grids(c, P);
+  phase_grids(c, P, sort_preps_cells(P, !P.ghost_list.empty()));
   rec(3);
   Pool<R> A = pool_view<R>(c, c->cur);
   if (P.nblk_list > 0) {

@@ -616,6 +616,78 @@ __device__ __forceinline__ const int *radix_sorted_vals(const int *vals, const i
 }
 
 // ---------------------------------------------------------------------------
+// Grids of a step's interactions and its cleared cell arrays (CellsArgs)
+// ---------------------------------------------------------------------------
+
+// Cells of the pool per tile flag: k_cells_mark sets the flags of the tiles it
+// writes to, so that k_cells_fill passes over empty regions a tile at a time.
+#define CELL_TILE 1024
+#define CELL_SHIFT 10
+static_assert(CELL_TILE == 4 * GR_BLOCK && CELL_TILE == 1 << CELL_SHIFT, "cell tile");
+
+// Grid of interaction `it` from the bounding boxes of its systems; cell arrays
+// checked against their capacity.
+__device__ inline void grid_of(const CellsArgs &A, int it, int *flags, int *sysfault) {
+  const int2 ab = A.inter_sys[it];
+  const double cutoff = A.cellsz[it];
+  Grid G;
+  double cells = 1.0;  // exact below 2^53, far beyond any capacity
+  for (int d = 0; d < 3; ++d) {
+    G.ming[d] = 0.0;
+    G.ng[d] = 1;
+    if (d >= A.D) continue;
+    double mn = unord_d(A.bbmin[ab.x * 3 + d]), mx = unord_d(A.bbmax[ab.x * 3 + d]);
+    if (ab.y >= 0 && A.n_dev[ab.y] > 0) {
+      double mnb = unord_d(A.bbmin[ab.y * 3 + d]), mxb = unord_d(A.bbmax[ab.y * 3 + d]);
+      mn = mnb < mn ? mnb : mn;
+      mx = mxb > mx ? mxb : mx;
+    }
+    G.ming[d] = floor((mn - 2.0 * cutoff) / cutoff) * cutoff;  // _snap_to_grid :191
+    double maxg = mx + 2.0 * cutoff;
+    double ngd = floor((maxg - G.ming[d]) / cutoff) + 1.0;  // :179
+    if (!(ngd >= 1.0) || ngd > 1.0e9) ngd = 1.0e9;
+    G.ng[d] = (int)ngd;
+    cells *= ngd;
+  }
+  const int2 ca = A.inter_carr[it];
+  long long cap = A.carr[ca.x].cap;
+  if (ca.y >= 0 && A.carr[ca.y].cap < cap) cap = A.carr[ca.y].cap;
+  G.ok = cells + 1.0 <= (double)cap;
+  if (!G.ok) {
+    // an empty grid: the sweeps find no partner for these systems; the
+    // systems are faulted, the other systems' grids are unaffected
+    atomicOr(&flags[1], 2);
+    atomicOr(&sysfault[ab.x], GR_FAULT_DOMAIN);
+    if (ab.y >= 0) atomicOr(&sysfault[ab.y], GR_FAULT_DOMAIN);
+  }
+  G.ncells = G.ok ? (int)cells : 0;
+  G.pad = 0;
+  A.grids[it] = G;
+}
+
+// Workgroup k of cells_prep_blocks(A): the grids of GR_BLOCK interactions, or
+// CELL_TILE cells cleared with the flags of the tiles they touch.
+__device__ inline void cells_prep(const CellsArgs &A, int k, int *flags, int *sysfault) {
+  const int ng = (A.n_inter + GR_BLOCK - 1) / GR_BLOCK, t = threadIdx.x;
+  if (k < ng) {
+    const int q = k * GR_BLOCK + t;
+    if (q < A.n_inter) grid_of(A, A.inter_list[q], flags, sysfault);
+    return;
+  }
+  const Blk b = A.cblk[k - ng];
+  const CellArr C = A.carr[b.item];
+  for (int c = b.first + t; c < C.cap && c < b.first + CELL_TILE; c += GR_BLOCK)
+    A.cells[C.off + c] = 0;
+  if (t < 2) {
+    const int c = t == 0 ? b.first : min(b.first + CELL_TILE, C.cap) - 1;
+    if (c >= 0) A.tflag[(C.off + c) >> CELL_SHIFT] = 0;
+  }
+}
+__global__ void __launch_bounds__(GR_BLOCK) k_cells_prep(CellsArgs A, int *flags, int *sysfault) {
+  cells_prep(A, blockIdx.x, flags, sysfault);
+}
+
+// ---------------------------------------------------------------------------
 // Counting sort of the step: one table entry per key
 //
 // The keys of a step are cells, a few per 100 particles, so they are sorted by
@@ -862,15 +934,22 @@ __device__ void radix_one_wave(unsigned *k0, int *v0, unsigned *k1, int *v1, int
 }
 
 // Every particle to its cell's slots (former place and key); also the tile
-// sums and the listed systems' bounds back to their initial values.
+// sums and the listed systems' bounds back to their initial values.  The
+// first nprep workgroups prepare the step's cell arrays (A): a longer chain of
+// dependent loads than the others', so they start first.
 __global__ void __launch_bounds__(GR_BLOCK)
     k_key_place(const SysDesc *sd, const int *n_dev, const Blk *blk, const int *bbase, unsigned *keys,
                 int *vals, unsigned *keys2, int *vals2, const unsigned *rank,
                 const unsigned *start, unsigned *tsum, int ntile, int N, const int *list,
                 int nlist, long long *bbmin, long long *bbmax, int rs, int *flags,
-                unsigned cap) {
+                unsigned cap, int nprep, CellsArgs A, int *sysfault) {
+  if ((int)blockIdx.x < nprep) {
+    cells_prep(A, (int)blockIdx.x, flags, sysfault);
+    return;
+  }
   __shared__ unsigned base[256];
-  const int nthr = (int)gridDim.x * GR_BLOCK, me = (int)blockIdx.x * GR_BLOCK + threadIdx.x;
+  const int bid = (int)blockIdx.x - nprep;
+  const int nthr = ((int)gridDim.x - nprep) * GR_BLOCK, me = bid * GR_BLOCK + threadIdx.x;
   for (int k = me; k < ntile * KT_REP; k += nthr) tsum[k] = 0u;
   for (int t = me; t < nlist * 3 * GR_BB_REP; t += nthr) {
     const int r = t / (nlist * 3), e = t % (nlist * 3);
@@ -880,10 +959,10 @@ __global__ void __launch_bounds__(GR_BLOCK)
   }
   if (flags[0] == 0) return;
   if ((unsigned)flags[2] > cap) {
-    if (blockIdx.x == 0 && threadIdx.x < 64) radix_one_wave(keys, vals, keys2, vals2, N, base);
+    if (bid == 0 && threadIdx.x < 64) radix_one_wave(keys, vals, keys2, vals2, N, base);
     return;
   }
-  const Blk b = blk[blockIdx.x];
+  const Blk b = blk[bid];
   const int s = b.item;
   const int i = b.first + threadIdx.x;
   if (i >= n_dev[s]) return;
@@ -1399,59 +1478,6 @@ __global__ void k_scan_add(int *out, const int *bsum, int N) {
 // Grid / CSR (src/Interaction.jl:123-236)
 // ---------------------------------------------------------------------------
 
-// Grid of each listed interaction from the bounding boxes of its systems.
-// inter_sys[2q] = a, inter_sys[2q+1] = b (or -1); cell arrays checked
-// against their capacity.
-__global__ void k_grid_params(const int *inter_list, int n, const int2 *inter_sys,
-                              const double *cellsz, const long long *bbmin,
-                              const long long *bbmax, const int *n_dev, Grid *grids,
-                              const int2 *inter_carr, const CellArr *carr, int D, int *flags,
-                              int *sysfault) {
-  int q = blockIdx.x * blockDim.x + threadIdx.x;
-  if (q >= n) return;
-  const int it = inter_list[q];
-  const int2 ab = inter_sys[it];
-  const double cutoff = cellsz[it];
-  Grid G;
-  long long ncells = 1;
-  for (int d = 0; d < D; ++d) {
-    double mn = double_of(bbmin[ab.x * 3 + d]), mx = double_of(bbmax[ab.x * 3 + d]);
-    if (ab.y >= 0 && n_dev[ab.y] > 0) {
-      double mnb = double_of(bbmin[ab.y * 3 + d]), mxb = double_of(bbmax[ab.y * 3 + d]);
-      mn = mnb < mn ? mnb : mn;
-      mx = mxb > mx ? mxb : mx;
-    }
-    G.ming[d] = floor((mn - 2.0 * cutoff) / cutoff) * cutoff;  // _snap_to_grid :191
-    double maxg = mx + 2.0 * cutoff;
-    double ngd = floor((maxg - G.ming[d]) / cutoff) + 1.0;  // :179
-    if (!(ngd >= 1.0) || ngd > 1.0e9) ngd = 1.0e9;
-    G.ng[d] = (int)ngd;
-    // saturate at 2^40 cells (far beyond any capacity): three factors of up
-    // to 1e9 would overflow a 64-bit product
-    ncells = ncells > (1LL << 40) / G.ng[d] ? (1LL << 40) : ncells * (long long)G.ng[d];
-  }
-  for (int d = D; d < 3; ++d) {
-    G.ming[d] = 0.0;
-    G.ng[d] = 1;
-  }
-  G.ok = 1;
-  const int2 ca = inter_carr[it];
-  long long cap = carr[ca.x].cap;
-  if (ca.y >= 0 && carr[ca.y].cap < cap) cap = carr[ca.y].cap;
-  if (ncells + 1 > cap || ncells < 1) {
-    // an empty grid: the sweeps find no partner for these systems; the
-    // systems are faulted, the other systems' grids are unaffected
-    G.ok = 0;
-    atomicOr(&flags[1], 2);
-    atomicOr(&sysfault[ab.x], GR_FAULT_DOMAIN);
-    if (ab.y >= 0) atomicOr(&sysfault[ab.y], GR_FAULT_DOMAIN);
-    ncells = 0;
-  }
-  G.ncells = (int)ncells;
-  G.pad = 0;
-  grids[it] = G;
-}
-
 template <int D>
 __device__ inline int cell_flat0(XP x, int64_t gi, const Grid &G,
                                  double cell) {  // _cell_1idx − 1 (:197-206)
@@ -1465,24 +1491,17 @@ __device__ inline int cell_flat0(XP x, int64_t gi, const Grid &G,
   return (int)flat;
 }
 
-// Zero the cells and write the sentinel n + 1 (:228).
-__global__ void k_cells_clear(int *cells, const CellArr *carr, const Grid *grids,
-                              const int *n_dev, const Blk *blk) {
-  const Blk b = blk[blockIdx.x];
-  const CellArr C = carr[b.item];
-  const int ncells = grids[C.grid].ncells;
-  for (int q = 0; q < 4; ++q) {
-    int c = b.first + q * GR_BLOCK + threadIdx.x;
-    if (c < C.cap && c <= ncells) cells[C.off + c] = (c == ncells) ? n_dev[C.sys] + 1 : 0;
-  }
-}
+// Three launches, or two in a step, whose last sort prepares the cells
+// (cells_prep): a launch costs 2.5 to 4 us in a scene of 20k particles whatever
+// it does.  The five before them (grids, clearing, marks and two for the fill)
+// took 13 us there and 43 at 1M particles; these two 5 to 7 and 24.
 
 // First particle of each run of equal cells (forward pass :219-226); the
 // last run of a cell wins, as the serial loop's last write does.
 template <int D>
-__global__ void k_cells_mark(XP x, int *cells, const CellArr *carr, const Grid *grids,
-                             const double *cellsz, const SysDesc *sd, const int *n_dev,
-                             const Blk *blk) {
+__global__ void __launch_bounds__(GR_BLOCK)
+    k_cells_mark(XP x, int *cells, int *tflag, const CellArr *carr, const Grid *grids,
+                 const double *cellsz, const SysDesc *sd, const int *n_dev, const Blk *blk) {
   const Blk b = blk[blockIdx.x];
   const CellArr C = carr[b.item];
   const int i = b.first + threadIdx.x;
@@ -1503,30 +1522,81 @@ __global__ void k_cells_mark(XP x, int *cells, const CellArr *carr, const Grid *
   __syncthreads();
   int prev = __shfl_up(c, 1, 64);
   if (lane == 0) prev = w > 0 ? cw[w - 1] : c0;
-  if (live && c != prev && c >= 0 && c < G.ncells) atomicMax(&cells[C.off + c], i + 1);
+  if (live && c != prev && c >= 0 && c < G.ncells) {
+    atomicMax(&cells[C.off + c], i + 1);
+    // (the first lane of a run of one tile: the flag's line is shared widely)
+    const int64_t T = (C.off + c) >> CELL_SHIFT;
+    if (lane == 0 || prev < 0 || (C.off + prev) >> CELL_SHIFT != T) tflag[T] = 1;
+  }
 }
 
 // Backward pass (:231-235): every empty cell takes the first non-empty start
-// to its right.  Two kernels: block-local suffix (with the block's first
-// non-empty start as its aggregate), then each block finds the first
-// non-empty aggregate among the blocks after it and applies it.
-#define FILL_TILE (GR_BLOCK * 4)
+// to its right, the end of the array (the sentinel n + 1, :228) one after its
+// last.  A workgroup fills its tile from the right; cells after its last start
+// take the first start beyond the tile, which it finds for itself, whole tiles
+// without a start passed over by their flags.  A cell that another workgroup
+// has filled meanwhile holds that same start, so either reading is right.
 
 __device__ inline int first_nz(int a, int b) { return a != 0 ? a : b; }
 
-__global__ void k_fill_local(int *cells, const CellArr *carr, const Grid *grids, const Blk *blk,
-                             int *bagg) {
-  __shared__ int s[GR_BLOCK / 64];
+// First start at or after cell p of the pool, below `lim`; `end` if none.
+__device__ inline int next_start(const int *cells, const int *tflag, int64_t p, int64_t lim,
+                                 int end) {
+  const int lane = threadIdx.x & 63;
+  while (p < lim) {
+    const int64_t last = (lim - 1) >> CELL_SHIFT;
+    int64_t T = -1;
+    for (int64_t k0 = p >> CELL_SHIFT; k0 <= last; k0 += 256) {
+      int first = 4;
+#pragma unroll
+      for (int q = 3; q >= 0; --q) {
+        const int64_t k = k0 + lane * 4 + q;
+        if (k <= last && tflag[k] != 0) first = q;
+      }
+      const unsigned long long m = __ballot(first < 4);
+      if (m != 0ull) {
+        const int l = __ffsll((long long)m) - 1;
+        T = k0 + l * 4 + __shfl(first, l, 64);
+        break;
+      }
+    }
+    if (T < 0) return end;
+    const int64_t t0 = T << CELL_SHIFT;
+    for (int64_t c0 = p > t0 ? p : t0; c0 < t0 + CELL_TILE; c0 += 256) {
+      int v[4];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int64_t c = c0 + q * 64 + lane;
+        v[q] = c < lim && c < t0 + CELL_TILE ? ld_dev(&cells[c]) : 0;
+      }
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const unsigned long long m = __ballot(v[q] != 0);
+        if (m != 0ull) return __shfl(v[q], __ffsll((long long)m) - 1, 64);
+      }
+    }
+    p = t0 + CELL_TILE;
+  }
+  return end;
+}
+
+__global__ void __launch_bounds__(GR_BLOCK)
+    k_cells_fill(int *cells, const int *tflag, const CellArr *carr, const Grid *grids,
+                 const int *n_dev, const Blk *blk) {
+  __shared__ int s[GR_BLOCK / 64], s_last, s_carry;
   const Blk b = blk[blockIdx.x];
   const CellArr C = carr[b.item];
   const int ncells = grids[C.grid].ncells;
+  if (b.first > ncells) return;  // uniform: no cell of this block is in the grid
   const int t = threadIdx.x, lane = t & 63, w = t >> 6;
+  const int end = n_dev[C.sys] + 1;
   const int c0 = b.first + t * 4;
   int v[4];
   for (int q = 0; q < 4; ++q) {
-    int c = c0 + q;
-    v[q] = (c < C.cap && c <= ncells) ? cells[C.off + c] : 0;
+    const int c = c0 + q;
+    v[q] = c < ncells ? cells[C.off + c] : end;
   }
+  if (t == GR_BLOCK - 1) s_last = v[3];
   // thread-local suffix, then the wavefront's (lanes lane..63) by shuffles
   for (int q = 2; q >= 0; --q) v[q] = first_nz(v[q], v[q + 1]);
   int a = v[0];
@@ -1536,60 +1606,22 @@ __global__ void k_fill_local(int *cells, const CellArr *carr, const Grid *grids,
   }
   if (lane == 0) s[w] = a;
   __syncthreads();
-  int rw = 0;  // first non-zero in the wavefronts after this one
+  int rw = 0;  // first start after this wavefront
+  if (s_last == 0) {  // uniform over the workgroup
+    if (w == 0) {
+      const int u =
+          next_start(cells, tflag, C.off + b.first + CELL_TILE, C.off + ncells, end);
+      if (lane == 0) s_carry = u;
+    }
+    __syncthreads();
+    rw = s_carry;
+  }
   for (int q = GR_BLOCK / 64 - 1; q > w; --q) rw = first_nz(s[q], rw);
   const int nx = __shfl_down(a, 1, 64);
   const int right = first_nz(lane < 63 ? nx : 0, rw);
   for (int q = 0; q < 4; ++q) {
-    int c = c0 + q;
+    const int c = c0 + q;
     if (c < C.cap && c <= ncells) cells[C.off + c] = first_nz(v[q], right);
-  }
-  if (t == 0) bagg[blockIdx.x] = first_nz(a, rw);
-}
-
-// The carry of a block is the first non-zero aggregate among the following
-// blocks of its cell array (consecutive in the table, `first` restarting at 0
-// for the next array), found 256 blocks at a time by each wavefront (4 per
-// lane, loads independent of each other).  The array's sentinel cell (n + 1)
-// is non-zero, so the search ends at the latest in the sentinel's block.
-__global__ void k_fill_apply(int *cells, const CellArr *carr, const Grid *grids, const Blk *blk,
-                             int nblk, const int *bagg) {
-  const Blk b = blk[blockIdx.x];
-  const CellArr C = carr[b.item];
-  const int ncells = grids[C.grid].ncells;
-  if (b.first > ncells) return;  // uniform: no cell of this block is in the grid
-  const int lane = threadIdx.x & 63;
-  int cr = 0;
-  for (int k0 = blockIdx.x + 1; k0 < nblk; k0 += 256) {
-    Blk bk[4];
-    int g[4];
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const int k = k0 + lane * 4 + q;
-      bk[q] = k < nblk ? blk[k] : Blk{-1, 0};
-      g[q] = k < nblk ? bagg[k] : 0;
-    }
-    // this lane's first stop (end of the array or a non-zero aggregate)
-    bool stop = false;
-    int gs = 0;
-#pragma unroll
-    for (int q = 3; q >= 0; --q) {
-      const bool same = bk[q].item == b.item && bk[q].first != 0;
-      if (!same || g[q] != 0) {
-        stop = true;
-        gs = same ? g[q] : 0;
-      }
-    }
-    const unsigned long long m = __ballot(stop);
-    if (m != 0ull) {
-      cr = __shfl(gs, __ffsll((long long)m) - 1, 64);  // 0 when the array ended first
-      break;
-    }
-  }
-  if (cr == 0) return;
-  for (int q = 0; q < 4; ++q) {
-    int c = b.first + threadIdx.x * 4 + q;
-    if (c < C.cap && c <= ncells && cells[C.off + c] == 0) cells[C.off + c] = cr;
   }
 }
 
@@ -2214,6 +2246,10 @@ void launch_key_base(hipStream_t s, const int *list, int nlist, int D, int pad, 
   k_key_base<<<1, KB_THREADS, 0, s>>>(list, nlist, D, pad, n, st, bbmin, bbmax, rs, kmin, kmax,
                                       kbase, krange, flags, sysfault, 0);
 }
+static int cells_prep_blocks(const CellsArgs &A) { return nb_of(A.n_inter, GR_BLOCK) + A.ncblk; }
+void launch_cells_prep(hipStream_t s, const CellsArgs &A, int *flags, int *sysfault) {
+  if (A.n_inter > 0) k_cells_prep<<<cells_prep_blocks(A), GR_BLOCK, 0, s>>>(A, flags, sysfault);
+}
 size_t key_table_bytes(int64_t ntile) {
   return (size_t)ntile * (KT_TILE * 2 + KT_REP) * sizeof(unsigned);
 }
@@ -2223,8 +2259,11 @@ void launch_key_sort(hipStream_t s, XP xs, const SysDesc *sd, const int *n, cons
                      int N, long long *bbmin, long long *bbmax, int rs, int *kmin, int *kmax,
                      unsigned *krange, unsigned *kbase, unsigned *keys, int *vals,
                      unsigned *keys2, int *vals2, unsigned *rank, int *flags, int *sysfault,
-                     unsigned *table, int tiles, int ntile) {
-  if (nblk <= 0) return;
+                     unsigned *table, int tiles, int ntile, const CellsArgs *cells) {
+  if (nblk <= 0) {
+    if (cells) launch_cells_prep(s, *cells, flags, sysfault);
+    return;
+  }
   unsigned *count = table, *start = table + (size_t)tiles * KT_TILE;
   unsigned *tsum = table + (size_t)tiles * KT_TILE * 2;
   const unsigned cap = (unsigned)ntile * KT_TILE - 1u;
@@ -2241,8 +2280,11 @@ void launch_key_sort(hipStream_t s, XP xs, const SysDesc *sd, const int *n, cons
                                              rs, kmin, kmax, krange, kbase, keys, vals, rank,
                                              flags, sysfault, count, tsum, cap, inl);
   k_key_scan<<<ntile, GR_BLOCK, 0, s>>>(count, tsum, start, flags, cap);
-  k_key_place<<<nblk, GR_BLOCK, 0, s>>>(sd, n, blk, bbase, keys, vals, keys2, vals2, rank, start,
-                                        tsum, ntile, N, list, nlist, bbmin, bbmax, rs, flags, cap);
+  const CellsArgs A = cells ? *cells : CellsArgs{};
+  const int nprep = cells_prep_blocks(A);
+  k_key_place<<<nblk + nprep, GR_BLOCK, 0, s>>>(
+      sd, n, blk, bbase, keys, vals, keys2, vals2, rank, start, tsum, ntile, N, list, nlist, bbmin,
+      bbmax, rs, flags, cap, nprep, A, sysfault);
 }
 KeyTable key_table_view(unsigned *table, int tiles, int ntile, const unsigned *keys2,
                         const unsigned *krange, const unsigned *kbase, const int *list,
@@ -2409,30 +2451,19 @@ template void launch_ghost_copy<double>(hipStream_t, const Pool<double> &, const
                                         const Bnd *, const int *, const Blk *, int,
                                         const int2 *, int);
 
-void launch_grid_params(hipStream_t s, const int *inter_list, int n, const int2 *inter_sys,
-                        const double *cellsz, const long long *bbmin, const long long *bbmax,
-                        const int *n_dev, Grid *grids, const int2 *inter_carr,
-                        const CellArr *carr, int D, int *flags, int *sysfault) {
-  if (n > 0)
-    k_grid_params<<<nb_of(n, 64), 64, 0, s>>>(inter_list, n, inter_sys, cellsz, bbmin, bbmax,
-                                              n_dev, grids, inter_carr, carr, D, flags,
-                                              sysfault);
-}
-void launch_cells_build(hipStream_t s, XP x, int *cells, const CellArr *carr,
-                        const Grid *grids, const double *cellsz, const SysDesc *sd,
-                        const int *n_dev, const Blk *cblk, int ncblk, const Blk *mblk,
-                        int nmblk, int *bagg, int D) {
-  if (ncblk > 0) k_cells_clear<<<ncblk, GR_BLOCK, 0, s>>>(cells, carr, grids, n_dev, cblk);
+int64_t cell_tiles(int64_t cells) { return (cells + CELL_TILE - 1) / CELL_TILE; }
+void launch_cells_build(hipStream_t s, XP x, const CellsArgs &A, const SysDesc *sd, const Blk *mblk,
+                        int nmblk) {
   if (nmblk > 0) {
-    if (D == 2)
-      k_cells_mark<2><<<nmblk, GR_BLOCK, 0, s>>>(x, cells, carr, grids, cellsz, sd, n_dev, mblk);
+    if (A.D == 2)
+      k_cells_mark<2><<<nmblk, GR_BLOCK, 0, s>>>(x, A.cells, A.tflag, A.carr, A.grids, A.cellsz, sd,
+                                                 A.n_dev, mblk);
     else
-      k_cells_mark<3><<<nmblk, GR_BLOCK, 0, s>>>(x, cells, carr, grids, cellsz, sd, n_dev, mblk);
+      k_cells_mark<3><<<nmblk, GR_BLOCK, 0, s>>>(x, A.cells, A.tflag, A.carr, A.grids, A.cellsz, sd,
+                                                 A.n_dev, mblk);
   }
-  if (ncblk > 0) {
-    k_fill_local<<<ncblk, GR_BLOCK, 0, s>>>(cells, carr, grids, cblk, bagg);
-    k_fill_apply<<<ncblk, GR_BLOCK, 0, s>>>(cells, carr, grids, cblk, ncblk, bagg);
-  }
+  if (A.ncblk > 0)
+    k_cells_fill<<<A.ncblk, GR_BLOCK, 0, s>>>(A.cells, A.tflag, A.carr, A.grids, A.n_dev, A.cblk);
 }
 
 template <typename R>

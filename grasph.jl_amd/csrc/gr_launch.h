@@ -69,12 +69,31 @@ void launch_key_write(hipStream_t s, XP xs, const SysDesc *sd, const int *n,
 void launch_radix_sort(hipStream_t s, unsigned *keys, int *vals, unsigned *keys2, int *vals2,
                        unsigned *rscr, int N, int *flags);
 size_t radix_scratch_bytes(int N);
+// Interactions whose grids a step finds (from the bounds in replica 0) and the
+// cell arrays it builds: cblk lists them 4·GR_BLOCK cells at a time, tflag holds
+// a flag per that many cells of the pool (cell_tiles).
+struct CellsArgs {
+  int *cells, *tflag;
+  const CellArr *carr;
+  const Blk *cblk;
+  int ncblk;
+  const int *inter_list;
+  int n_inter;
+  const int2 *inter_sys;  // systems a and b (or -1) of an interaction
+  const int2 *inter_carr;
+  const double *cellsz;
+  const long long *bbmin, *bbmax;
+  const int *n_dev;
+  Grid *grids;
+  int D;
+};
 // The counting sort of a step (keys, table, placement) after the bounds pass:
 // `table` of key_table_bytes(tiles) bytes, zeroed when allocated, of which this
 // sort uses ntile <= tiles tiles (ntile·key_table_tile() - 1 keys; the layout
 // goes by `tiles`, as sorts of different sizes share the table).  flags[0] must
 // be clear; the permutations take the order by key_table_view.  Replicas 1..
-// of the listed systems' bounds are reset.
+// of the listed systems' bounds are reset, and `cells` prepared (as
+// launch_cells_prep does).
 size_t key_table_bytes(int64_t ntile);
 int key_table_tile();
 void launch_key_sort(hipStream_t s, XP xs, const SysDesc *sd, const int *n, const StepSys *st,
@@ -82,7 +101,7 @@ void launch_key_sort(hipStream_t s, XP xs, const SysDesc *sd, const int *n, cons
                      int N, long long *bbmin, long long *bbmax, int rs, int *kmin, int *kmax,
                      unsigned *krange, unsigned *kbase, unsigned *keys, int *vals,
                      unsigned *keys2, int *vals2, unsigned *rank, int *flags, int *sysfault,
-                     unsigned *table, int tiles, int ntile);
+                     unsigned *table, int tiles, int ntile, const CellsArgs *cells = nullptr);
 struct KeyTable {  // what the permutations read of the counting sort
   const unsigned *keys2, *start, *krange, *kbase;
   const int *list;
@@ -123,14 +142,12 @@ void launch_ghost_kin(hipStream_t s, const Pool<R> &P, const SysDesc *sd, const 
 template <typename R>
 void launch_ghost_copy(hipStream_t s, const Pool<R> &P, const SysDesc *sd, const Bnd *bnd,
                        const int *n, const Blk *blk, int nblk, const int2 *copy, int D);
-void launch_grid_params(hipStream_t s, const int *inter_list, int n, const int2 *inter_sys,
-                        const double *cellsz, const long long *bbmin, const long long *bbmax,
-                        const int *n_dev, Grid *grids, const int2 *inter_carr,
-                        const CellArr *carr, int D, int *flags, int *sysfault);
-void launch_cells_build(hipStream_t s, XP x, int *cells, const CellArr *carr,
-                        const Grid *grids, const double *cellsz, const SysDesc *sd,
-                        const int *n_dev, const Blk *cblk, int ncblk, const Blk *mblk,
-                        int nmblk, int *bagg, int D);
+int64_t cell_tiles(int64_t cells);
+// The grids, and the arrays cleared: once the bounds are there.
+void launch_cells_prep(hipStream_t s, const CellsArgs &A, int *flags, int *sysfault);
+// The arrays, after that.
+void launch_cells_build(hipStream_t s, XP x, const CellsArgs &A, const SysDesc *sd, const Blk *mblk,
+                        int nmblk);
 template <typename R>
 void launch_halfstep(hipStream_t s, const Pool<R> &P, const SysDesc *sd, const StepSys *st,
                      const Blk *blk, int nblk, int D, double mult, int keep);
