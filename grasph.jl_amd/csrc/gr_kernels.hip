@@ -150,14 +150,60 @@ __device__ inline void radix_add_runs(unsigned bin, bool valid, unsigned *cnt) {
 // replicas 1 .. GR_BB_REP of the bounds (stride `rs`), one for the workgroups
 // of each XCD, and folded into replica 0 afterwards (key_space, k_bb_fold).
 // `flags`: also clear the sort's inversion flag for the key pass that follows.
+//
+// In small scenes the kernel that advances the positions takes their bounds
+// for the next step instead (k_fullstep, k_rk4_apply with BB), which saves the
+// launch (step_bounds).
+template <int D>
+__device__ inline void bb_flush(const long long *mn, const long long *mx, int s, long long *bbmin,
+                                long long *bbmax) {
+  __shared__ long long red[2][GR_BLOCK / 64][3];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+#pragma unroll
+  for (int d = 0; d < D; ++d) {
+    const long long a = wave_red_ll<false>(mn[d]), bq = wave_red_ll<true>(mx[d]);
+    if (lane == 0) {
+      red[0][w][d] = a;
+      red[1][w][d] = bq;
+    }
+  }
+  __syncthreads();
+  if (threadIdx.x < D) {
+    const int d = threadIdx.x;
+    long long a = LLONG_MAX, bq = LLONG_MIN;
+    for (int q = 0; q < GR_BLOCK / 64; ++q) {
+      a = red[0][q][d] < a ? red[0][q][d] : a;
+      bq = red[1][q][d] > bq ? red[1][q][d] : bq;
+    }
+    // every workgroup of a system reduces into the same few words; only
+    // a partial result that improves on the current value takes the atomic
+    if (a != LLONG_MAX) {
+      if (a < ld_dev(&bbmin[s * 3 + d])) atomicMin(&bbmin[s * 3 + d], a);
+      if (bq > ld_dev(&bbmax[s * 3 + d])) atomicMax(&bbmax[s * 3 + d], bq);
+    }
+  }
+  __syncthreads();
+}
+// Bounds of one workgroup's particles, all of system s, for the next step.
+template <int D>
+__device__ inline void bb_block(const double *x, bool live, int s, const StepBounds &B) {
+  long long mn[D], mx[D];
+#pragma unroll
+  for (int d = 0; d < D; ++d) {
+    mn[d] = live ? ord_d(x[d]) : LLONG_MAX;
+    mx[d] = live ? ord_d(x[d]) : LLONG_MIN;
+  }
+  const int r = (1 + blockIdx.x % GR_BB_REP) * B.rs;
+  bb_flush<D>(mn, mx, s, B.bbmin + r, B.bbmax + r);
+  if (blockIdx.x == 0 && threadIdx.x == 0) B.flags[0] = 0;  // for the next step's keys
+}
+
 template <int D, int PER>
 __global__ void k_key_minmax(XP xs, const SysDesc *sd, const int *n_dev, const Blk *blk, int nblk,
                              long long *bbmin, long long *bbmax, int rs, int *flags) {
   if (flags && blockIdx.x == 0 && threadIdx.x == 0) flags[0] = 0;
   bbmin += (1 + blockIdx.x % GR_BB_REP) * rs;
   bbmax += (1 + blockIdx.x % GR_BB_REP) * rs;
-  __shared__ long long red[2][GR_BLOCK / 64][3];
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int b0 = blockIdx.x * PER;
   int item[PER];
   bool live[PER];
@@ -180,32 +226,7 @@ __global__ void k_key_minmax(XP xs, const SysDesc *sd, const int *n_dev, const B
       mx[d] = LLONG_MIN;
     }
   };
-  auto flush = [&](int s) {
-#pragma unroll
-    for (int d = 0; d < D; ++d) {
-      const long long a = wave_red_ll<false>(mn[d]), bq = wave_red_ll<true>(mx[d]);
-      if (lane == 0) {
-        red[0][w][d] = a;
-        red[1][w][d] = bq;
-      }
-    }
-    __syncthreads();
-    if (threadIdx.x < D) {
-      const int d = threadIdx.x;
-      long long a = LLONG_MAX, bq = LLONG_MIN;
-      for (int q = 0; q < GR_BLOCK / 64; ++q) {
-        a = red[0][q][d] < a ? red[0][q][d] : a;
-        bq = red[1][q][d] > bq ? red[1][q][d] : bq;
-      }
-      // every workgroup of a system reduces into the same few words; only
-      // a partial result that improves on the current value takes the atomic
-      if (a != LLONG_MAX) {
-        if (a < ld_dev(&bbmin[s * 3 + d])) atomicMin(&bbmin[s * 3 + d], a);
-        if (bq > ld_dev(&bbmax[s * 3 + d])) atomicMax(&bbmax[s * 3 + d], bq);
-      }
-    }
-    __syncthreads();
-  };
+  auto flush = [&](int s) { bb_flush<D>(mn, mx, s, bbmin, bbmax); };
   reset();
   int cur = item[0];
 #pragma unroll
@@ -1494,7 +1515,7 @@ __device__ inline int cell_flat0(XP x, int64_t gi, const Grid &G,
 // Three launches, or two in a step, whose last sort prepares the cells
 // (cells_prep): a launch costs 2.5 to 4 us in a scene of 20k particles whatever
 // it does.  The five before them (grids, clearing, marks and two for the fill)
-// took 13 us there and 43 at 1M particles; these two 5 to 7 and 24.
+// took 13 us there and 43 at 1.4M particles; these two 5 to 7 and 24.
 
 // First particle of each run of equal cells (forward pass :219-226); the
 // last run of a cell wins, as the serial loop's last write does.
@@ -1736,51 +1757,67 @@ __global__ void k_rk4_acc(Pool<R> P, const SysDesc *sd, const StepSys *st, const
 }
 
 // q = q0 + dt·acc, then x += dt·v (_apply_acc_all!, _update_positions_all!).
-template <typename R, int D>
+// BB: and the bounds of x for the next step's sort.
+template <typename R, int D, bool BB>
 __global__ void k_rk4_apply(Pool<R> P, const SysDesc *sd, const StepSys *st, const Blk *blk,
-                            int pos) {
+                            int pos, StepBounds B) {
   const Blk b = blk[blockIdx.x];
   const int s = b.item;
   const int i = b.first + threadIdx.x;
   const SysDesc S = sd[s];
-  if (i >= S.cap) return;
-  const StepSys T = st[s];
-  const int64_t g = S.off + i;
+  const bool live = i < S.cap;
+  double x[D] = {};
+  if (live) {
+    const StepSys T = st[s];
+    const int64_t g = S.off + i;
 #pragma unroll
-  for (int d = 0; d < D; ++d) {
-    const double vn = P.v[d][g] + T.dt * P.acc[d][g];
-    P.v[d][g] = vn;
-    if (pos) P.x[d][g] = P.x[d][g] + T.dt * vn;
+    for (int d = 0; d < D; ++d) {
+      const double vn = P.v[d][g] + T.dt * P.acc[d][g];
+      P.v[d][g] = vn;
+      if (pos) {
+        x[d] = P.x[d][g] + T.dt * vn;
+        P.x[d][g] = x[d];
+      }
+    }
+    P.rho[g] = fma(T.dt, P.acc[3][g], P.rho[g]);
   }
-  P.rho[g] = fma(T.dt, P.acc[3][g], P.rho[g]);
+  if constexpr (BB) bb_block<D>(x, live && i < B.n_dev[s], s, B);
 }
 
 // _apply_damping_all! (:251-271), _fullstep_q_all! (:227-232),
 // _update_positions_all! (:235-240).  v and x use separate products and sums
 // (SVector arithmetic is outside @fastmath); ρ uses the fused axpy.
-template <typename R, int D>
+// BB: and the bounds of x for the next step's sort.
+template <typename R, int D, bool BB>
 __global__ void k_fullstep(Pool<R> P, const SysDesc *sd, const StepSys *st, const Blk *blk,
-                           int pos) {
+                           int pos, StepBounds B) {
   const Blk b = blk[blockIdx.x];
   const int s = b.item;
   const int i = b.first + threadIdx.x;
   const SysDesc S = sd[s];
-  if (i >= S.cap) return;
-  const StepSys T = st[s];
-  const int64_t g = S.off + i;
+  const bool live = i < S.cap;
+  double x[D] = {};
+  if (live) {
+    const StepSys T = st[s];
+    const int64_t g = S.off + i;
 #pragma unroll
-  for (int d = 0; d < D; ++d) {
-    double a = (double)P.dvdt[d][g];
-    if (T.damping) {
-      a = a - T.gdt * (double)P.vs[d][g];
-      P.dvdt[d][g] = (R)a;
-      a = (double)P.dvdt[d][g];
+    for (int d = 0; d < D; ++d) {
+      double a = (double)P.dvdt[d][g];
+      if (T.damping) {
+        a = a - T.gdt * (double)P.vs[d][g];
+        P.dvdt[d][g] = (R)a;
+        a = (double)P.dvdt[d][g];
+      }
+      double vn = P.v[d][g] + T.dt * a;
+      P.v[d][g] = vn;
+      if (pos) {
+        x[d] = P.x[d][g] + T.dt * vn;
+        P.x[d][g] = x[d];
+      }
     }
-    double vn = P.v[d][g] + T.dt * a;
-    P.v[d][g] = vn;
-    if (pos) P.x[d][g] = P.x[d][g] + T.dt * vn;
+    P.rho[g] = fma(T.dt, (double)P.drhodt[g], P.rho[g]);
   }
-  P.rho[g] = fma(T.dt, (double)P.drhodt[g], P.rho[g]);
+  if constexpr (BB) bb_block<D>(x, live && i < B.n_dev[s], s, B);
 }
 
 // _xsph_correction! (src/TimeIntegration.jl:423-436) around the XSPH sweep.
@@ -2484,23 +2521,34 @@ void launch_rk4_acc(hipStream_t s, const Pool<R> &P, const SysDesc *sd, const St
   else
     k_rk4_acc<R, 3><<<nblk, GR_BLOCK, 0, s>>>(P, sd, st, blk, w, first);
 }
+template <typename F>
+static void dispatch_bb(int D, bool bb, F go) {
+  using T = std::true_type;
+  using N = std::false_type;
+  if (D == 2)
+    bb ? go(std::integral_constant<int, 2>{}, T{}) : go(std::integral_constant<int, 2>{}, N{});
+  else
+    bb ? go(std::integral_constant<int, 3>{}, T{}) : go(std::integral_constant<int, 3>{}, N{});
+}
 template <typename R>
 void launch_rk4_apply(hipStream_t s, const Pool<R> &P, const SysDesc *sd, const StepSys *st,
-                      const Blk *blk, int nblk, int D, int pos) {
+                      const Blk *blk, int nblk, int D, int pos, const StepBounds *bb) {
   if (nblk <= 0) return;
-  if (D == 2)
-    k_rk4_apply<R, 2><<<nblk, GR_BLOCK, 0, s>>>(P, sd, st, blk, pos);
-  else
-    k_rk4_apply<R, 3><<<nblk, GR_BLOCK, 0, s>>>(P, sd, st, blk, pos);
+  const StepBounds B = bb ? *bb : StepBounds{};
+  dispatch_bb(D, bb != nullptr, [&](auto d, auto q) {
+    k_rk4_apply<R, decltype(d)::value, decltype(q)::value>
+        <<<nblk, GR_BLOCK, 0, s>>>(P, sd, st, blk, pos, B);
+  });
 }
 template <typename R>
 void launch_fullstep(hipStream_t s, const Pool<R> &P, const SysDesc *sd, const StepSys *st,
-                     const Blk *blk, int nblk, int D, int pos) {
+                     const Blk *blk, int nblk, int D, int pos, const StepBounds *bb) {
   if (nblk <= 0) return;
-  if (D == 2)
-    k_fullstep<R, 2><<<nblk, GR_BLOCK, 0, s>>>(P, sd, st, blk, pos);
-  else
-    k_fullstep<R, 3><<<nblk, GR_BLOCK, 0, s>>>(P, sd, st, blk, pos);
+  const StepBounds B = bb ? *bb : StepBounds{};
+  dispatch_bb(D, bb != nullptr, [&](auto d, auto q) {
+    k_fullstep<R, decltype(d)::value, decltype(q)::value>
+        <<<nblk, GR_BLOCK, 0, s>>>(P, sd, st, blk, pos, B);
+  });
 }
 template <typename R>
 void launch_xsph(hipStream_t s, const Pool<R> &P, const SysDesc *sd, const StepSys *st,
@@ -2539,9 +2587,11 @@ void launch_updaters(hipStream_t s, const Pool<R> &P, const SysDesc *sd, const S
   template void launch_rk4_acc<R>(hipStream_t, const Pool<R> &, const SysDesc *,               \
                                   const StepSys *, const Blk *, int, int, double, int);        \
   template void launch_rk4_apply<R>(hipStream_t, const Pool<R> &, const SysDesc *,             \
-                                    const StepSys *, const Blk *, int, int, int);              \
+                                    const StepSys *, const Blk *, int, int, int,               \
+                                    const StepBounds *);                                       \
   template void launch_fullstep<R>(hipStream_t, const Pool<R> &, const SysDesc *,              \
-                                   const StepSys *, const Blk *, int, int, int);               \
+                                   const StepSys *, const Blk *, int, int, int,                \
+                                   const StepBounds *);                                        \
   template void launch_xsph<R>(hipStream_t, const Pool<R> &, const SysDesc *, const StepSys *, \
                                const int *, const Blk *, int, int, int);                       \
   template void launch_updaters<R>(hipStream_t, const Pool<R> &, const SysDesc *,              \

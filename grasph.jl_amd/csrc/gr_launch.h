@@ -48,6 +48,12 @@ struct NlistArgs {
 // bounds that every reader uses.  launch_key_minmax folds them itself when
 // `fold`, launch_key_base and launch_key_sort always do.
 #define GR_BB_REP 8
+struct StepBounds {  // where the end of a step takes the bounds of the next
+  const int *n_dev;
+  long long *bbmin, *bbmax;
+  int rs;
+  int *flags;  // [0] is cleared
+};
 void launch_key_minmax(hipStream_t s, XP xs, const SysDesc *sd, const int *n, const Blk *blk,
                        int nblk, int D, long long *bbmin, long long *bbmax, int rs,
                        const int *list, int nlist, bool fold, int *flags = nullptr);
@@ -156,10 +162,12 @@ void launch_rk4_acc(hipStream_t s, const Pool<R> &P, const SysDesc *sd, const St
                     const Blk *blk, int nblk, int D, double w, int first);
 template <typename R>
 void launch_rk4_apply(hipStream_t s, const Pool<R> &P, const SysDesc *sd, const StepSys *st,
-                      const Blk *blk, int nblk, int D, int pos);
+                      const Blk *blk, int nblk, int D, int pos,
+                     const StepBounds *bb = nullptr);
 template <typename R>
 void launch_fullstep(hipStream_t s, const Pool<R> &P, const SysDesc *sd, const StepSys *st,
-                     const Blk *blk, int nblk, int D, int pos);
+                     const Blk *blk, int nblk, int D, int pos,
+                     const StepBounds *bb = nullptr);
 template <typename R>
 void launch_xsph(hipStream_t s, const Pool<R> &P, const SysDesc *sd, const StepSys *st,
                  const int *n, const Blk *blk, int nblk, int D, int mode);

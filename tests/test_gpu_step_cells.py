@@ -66,3 +66,31 @@ def test_step_cells_equal_oracle(name, D):
     for a, b in zip(*got):
         for u, v in zip(a, b):
             assert np.array_equal(u, v)
+
+
+# one workgroup per 256 particles: 1024 of them take the next step's bounds as
+# they advance the positions, more leave them to a pass of their own
+@pytest.mark.parametrize("scheme", ["LeapFrogTimeIntegrator", "RK4TimeIntegrator"])
+@pytest.mark.parametrize("n", [1, 257, 262144, 262145])
+def test_bounds_follow_the_particles(n, scheme):
+    """The box of a cloud that closes in on its centre, over steps of one call:
+    the last step's cells and order are the oracle's."""
+    x = _random(2, n, max(1.0, 0.02 * n ** 0.5))
+    got = []
+    for scene in (M.Session(2, "f64").scene, oracle_scene(2)):
+        ps = M.FluidParticleSystem("a", n, 2, 1e-3, 10.0, state_updater=M.TaitEOSUpdater(1000.0))
+        ps.x[:] = x
+        ps.v[:] = 0.4 * (x.mean(axis=0) - x)
+        ps.rho[:] = 1000.0
+        si = M.SystemInteraction(M.WenlandC2Kernel(0.01, ndims=2), M.NeighborCounterPfn(), ps)
+        lf = getattr(M, scheme)([ps], [si])
+        h = scene.integrator(lf)
+        scene.upload_all(lf)
+        scene.be.step(h, 3, 0.25)
+        scene.download_all(lf)
+        hi = scene.interaction(si)
+        ming, ng, ncells = scene.be.get_grid(hi, 2)
+        got.append([ps.id.copy(), ps.x.copy(), ming, ng,
+                    scene.be.get_cell_start(hi, 0, ncells + 1)])
+    for u, v in zip(*got):
+        assert np.array_equal(u, v)
