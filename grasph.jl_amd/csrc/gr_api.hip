@@ -1953,25 +1953,26 @@ void phase_grids(gr_ctx *c, Plan &P, bool prepared = false) {
                      P.nblk_mark);
 }
 
+// kin: the ghosts' kinematics are still to be done (stage 0).
 template <typename R>
-void phase_stage(gr_ctx *c, Plan &P, int k, bool cnt, hipEvent_t *mid, bool real_packed = false) {
+void phase_stage(gr_ctx *c, Plan &P, int k, bool cnt, hipEvent_t *mid, bool real_packed, bool kin) {
   hipStream_t s = c->stream;
   StagePlan &S = *P.stages[k];
   Pool<R> A = pool_view<R>(c, c->cur);
-  launch_updaters<R>(s, A, c->d_sd.as<SysDesc>(), c->d_st.as<StepSys>(), S.blk_upd.as<Blk>(),
-                     S.nblk_upd, S.urange.as<int2>(), S.upd.as<UpdDesc>(), c->D, S.upd_kinds);
-  launch_ghost_copy<R>(s, A, c->d_sd.as<SysDesc>(), c->d_bnd.as<Bnd>(), c->d_n.as<int>(),
-                       S.blk_gcopy.as<Blk>(), S.nblk_gcopy, S.gcopy.as<int2>(), c->D);
-  if (mid) HIPCHK(hipEventRecord(*mid, s));
+  const SysDesc *sd = c->d_sd.as<SysDesc>();
+  const int *n = c->d_n.as<int>();
+  const Bnd *bnd = c->d_bnd.as<Bnd>();
   // a stage whose only sweeps are FP32 force and strain-rate sweeps reads the
   // compact records alone
   const bool c_only = sizeof(R) == 4 && S.fam[FAM_INTERP].nblk == 0 &&
                       S.fam[FAM_COUNT].nblk == 0;
-  // the partner stress records only for stages with Cauchy force sweeps
-  const bool with_s = S.fam[FAM_FORCE].cauchy;
   // records of 1/ρ and p/ρ² when the stage's only sweeps are FluidPfn S = 2
   // force sweeps without δ-SPH or surface tension
   const bool inv = c_only && S.fam[FAM_FORCE].inv && S.fam[FAM_STRAIN].nblk == 0;
+  // the partner stress records only for stages with Cauchy force sweeps
+  const bool with_s = S.fam[FAM_FORCE].cauchy;
+  const int mode = (c_only ? GR_REC_C : 0) | (with_s ? GR_REC_S : 0) |
+                   (inv && !with_s ? GR_REC_INV : 0);
   // the compact records of the real systems packed for the previous stage
   // still hold when they are of the same kind and nothing in between wrote
   // x, v, ρ or p: the stage's only updaters are Drucker-Prager (stress and
@@ -1986,25 +1987,44 @@ void phase_stage(gr_ctx *c, Plan &P, int k, bool cnt, hipEvent_t *mid, bool real
   const bool keep_c = k > 0 && P.nblk_virt == 0 && rec_kind(S) != 0 &&
                       rec_kind(S) == rec_kind(*P.stages[k - 1]) &&
                       (S.upd_kinds & ~(1 << GR_UPD_EP | 1 << GR_UPD_NOTHING)) == 0;
-  auto pack = [&]() {
-    if (!real_packed)
-      launch_pack<R>(s, A, c->d_sd.as<SysDesc>(), c->d_n.as<int>(), P.blk_real.as<Blk>(),
-                     P.nblk_real, c->D, c_only, with_s, inv, keep_c);
-    launch_pack<R>(s, A, c->d_sd.as<SysDesc>(), c->d_n.as<int>(), P.blk_ghost.as<Blk>(),
-                   P.nblk_ghost, c->D, c_only, with_s, inv);
-  };
   const int nother = S.fam[FAM_FORCE].nblk + S.fam[FAM_COUNT].nblk + S.fam[FAM_STRAIN].nblk;
-  if (nother + S.fam[FAM_INTERP].nblk > 0) pack();
+  // the real systems' records, if any are to be written
+  const bool real = !real_packed && !(keep_c && !with_s);
+  const int rmode = mode | (keep_c ? GR_REC_S_ONLY : 0);
+  // In a stage with sweeps and no interpolation the records are written as soon
+  // as their fields are there: the real systems' by the updaters (none of which
+  // writes what the ghosts' kinematics read), the ghosts' with their kinematics
+  // and copies.
+  const bool fuse = nother > 0 && S.fam[FAM_INTERP].nblk == 0;
+  const bool with_upd = fuse && real && S.nblk_upd > 0;
+  if (kin && !fuse)
+    launch_ghost_kin<R>(s, A, sd, bnd, n, P.blk_ghost.as<Blk>(), P.nblk_ghost, c->D);
+  launch_updaters<R>(s, A, sd, c->d_st.as<StepSys>(), (with_upd ? P.blk_real : S.blk_upd).as<Blk>(),
+                     with_upd ? P.nblk_real : S.nblk_upd, S.urange.as<int2>(),
+                     S.upd.as<UpdDesc>(), c->D, S.upd_kinds, with_upd ? rmode : -1);
+  if (!fuse)
+    launch_ghost_copy<R>(s, A, sd, bnd, n, S.blk_gcopy.as<Blk>(), S.nblk_gcopy,
+                         S.gcopy.as<int2>(), c->D);
+  auto pack = [&](bool rl, const int2 *copy, bool kn) {
+    launch_pack<R>(s, A, sd, n, P.blk_real.as<Blk>(), rl ? P.nblk_real : 0, rmode,
+                   P.blk_ghost.as<Blk>(), P.nblk_ghost, mode, bnd, copy, kn, c->D);
+  };
+  if (fuse)
+    pack(real && !with_upd, S.nblk_gcopy > 0 ? S.gcopy.as<int2>() : nullptr, kin);
+  else if (nother + S.fam[FAM_INTERP].nblk > 0)
+    pack(real, nullptr, false);
+  if (mid) HIPCHK(hipEventRecord(*mid, s));
   // interpolation into virtual systems runs first; the functors of the same
   // stage then see the interpolated fields
   for (int fam : {FAM_INTERP, FAM_FORCE, FAM_COUNT, FAM_STRAIN}) {
     FamPlan &F = S.fam[fam];
     if (F.nblk == 0) continue;
-    if (fam == FAM_FORCE && S.fam[FAM_INTERP].nblk > 0) pack();
-    if (fam == FAM_COUNT && S.fam[FAM_INTERP].nblk > 0 && S.fam[FAM_FORCE].nblk == 0) pack();
+    if (fam == FAM_FORCE && S.fam[FAM_INTERP].nblk > 0) pack(real, nullptr, false);
+    if (fam == FAM_COUNT && S.fam[FAM_INTERP].nblk > 0 && S.fam[FAM_FORCE].nblk == 0)
+      pack(real, nullptr, false);
     if (fam == FAM_STRAIN && S.fam[FAM_INTERP].nblk > 0 && S.fam[FAM_FORCE].nblk == 0 &&
         S.fam[FAM_COUNT].nblk == 0)
-      pack();
+      pack(real, nullptr, false);
     SweepArgs a;
     a.sd = c->d_sd.as<SysDesc>();
     a.n = c->d_n.as<int>();
@@ -2039,9 +2059,9 @@ void phase_xsph(gr_ctx *c, Plan &P) {
   launch_xsph<R>(s, A, sd, st, c->d_n.as<int>(), P.blk_int.as<Blk>(), P.nblk_int, c->D, 0);
   if (P.xsph.nblk > 0 || !P.xsph_al.empty()) {
     launch_xsph<R>(s, A, sd, st, c->d_n.as<int>(), P.blk_virt.as<Blk>(), P.nblk_virt, c->D, 1);
-    launch_pack<R>(s, A, sd, c->d_n.as<int>(), P.blk_real.as<Blk>(), P.nblk_real, c->D);
-    if (!P.xsph_alias.empty())
-      launch_pack<R>(s, A, sd, c->d_n.as<int>(), P.blk_ghost.as<Blk>(), P.nblk_ghost, c->D);
+    launch_pack<R>(s, A, sd, c->d_n.as<int>(), P.blk_real.as<Blk>(), P.nblk_real, GR_REC_S,
+                   P.blk_ghost.as<Blk>(), P.xsph_alias.empty() ? 0 : P.nblk_ghost, GR_REC_S,
+                   nullptr, nullptr, false, c->D);
     SweepArgs a;
     a.sd = sd;
     a.n = c->d_n.as<int>();
@@ -2222,13 +2242,17 @@ void run_step(gr_ctx *c, Plan &P, bool cnt, std::vector<hipEvent_t> *ev) {
   const StepSys *st = c->d_st.as<StepSys>();
   // the stage loop of one pass (_sweep_all_stages!) after the stage state
   auto pass = [&]() {
-    launch_ghost_kin<R>(s, A, sd, c->d_bnd.as<Bnd>(), c->d_n.as<int>(), P.blk_ghost.as<Blk>(),
-                        P.nblk_ghost, c->D);
+    // (stage 0 may do the ghosts' kinematics along with their records, where no
+    // virtual system is zeroed in between)
+    const bool kin = nst > 0 && P.nblk_virt == 0 && P.nblk_ghost > 0;
+    if (!kin)
+      launch_ghost_kin<R>(s, A, sd, c->d_bnd.as<Bnd>(), c->d_n.as<int>(), P.blk_ghost.as<Blk>(),
+                          P.nblk_ghost, c->D);
     launch_virtual<R>(s, A, sd, st, c->d_n.as<int>(), P.blk_virt.as<Blk>(), P.nblk_virt, 0, c->D);
     rec(5);
     for (int k = 0; k < nst; ++k) {
       phase_stage<R>(c, P, k, cnt, ev ? &(*ev)[6 + 2 * k] : nullptr,
-                     k == 0 && pack_in_sort != 0);
+                     k == 0 && pack_in_sort != 0, k == 0 && kin);
       rec(7 + 2 * k);
     }
   };
@@ -2457,7 +2481,7 @@ void pack_systems(gr_ctx *c, const std::vector<int> &systems) {
   DBuf b;
   b.upload(v, c->stream);
   launch_pack<R>(c->stream, pool_view<R>(c, c->cur), c->d_sd.as<SysDesc>(), c->d_n.as<int>(),
-                 b.as<Blk>(), (int)v.size(), c->D);
+                 b.as<Blk>(), (int)v.size(), GR_REC_S, nullptr, 0, 0, nullptr, nullptr, false, c->D);
   HIPCHK(hipStreamSynchronize(c->stream));
 }
 

@@ -1324,29 +1324,120 @@ __global__ void k_permute_ghost(XP gxs, const int *gidx_s, const int *gbnd_s, XP
   gbnd[dst] = gbnd_s[src];
 }
 
+// Partner records of a particle (positions, shadows of density and velocity,
+// pressure, stress), read by the pair sweeps; which of them by GR_REC_* flags.
+template <typename R>
+struct Rec {
+  double x[3];
+  R v[3], rho, p;
+  float s[8];
+};
+template <typename R>
+__device__ inline void rec_load_stress(const Pool<R> &P, const SysDesc &S, int64_t g, Rec<R> &r) {
+#pragma unroll
+  for (int k = 0; k < 8; ++k) r.s[k] = 0.0f;
+  if (S.kind >= GR_SYS_STRESS) {
+#pragma unroll
+    for (int k = 0; k < GR_MAXNS; ++k)
+      if (k < S.ns) r.s[k] = (float)P.stress_s[k][g];
+  }
+}
+template <typename R>
+__device__ inline void rec_load(const Pool<R> &P, const SysDesc &S, int64_t g, int D, int mode,
+                                Rec<R> &r) {
+  if (!(mode & GR_REC_S_ONLY)) {
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+      r.x[d] = d < D ? P.x[d][g] : 0.0;
+      r.v[d] = d < D ? P.vs[d][g] : (R)0;
+    }
+    r.rho = P.rhos[g];
+    r.p = P.p[g];
+  }
+  if (sizeof(R) == 4 && (mode & GR_REC_S)) rec_load_stress(P, S, g, r);
+}
+template <typename R>
+__device__ inline void rec_store(const Pool<R> &P, int64_t g, int D, int mode, const Rec<R> &r) {
+  if (!(mode & GR_REC_S_ONLY)) {
+    if (sizeof(R) == 8 || !(mode & GR_REC_C)) {
+      RecA<R> a;
+      RecB<R> b;
+#pragma unroll
+      for (int d = 0; d < 3; ++d) {
+        a.x[d] = r.x[d];
+        b.v[d] = r.v[d];
+      }
+      a.rho = r.rho;
+      if constexpr (sizeof(R) == 4) {
+        a.p = r.p;
+        b.pad = 0.0f;
+      } else {
+        b.p = r.p;
+      }
+      P.ra[g] = a;
+      P.rb[g] = b;
+    }
+    if constexpr (sizeof(R) == 4) {
+      RecC c;
+#pragma unroll
+      for (int d = 0; d < 3; ++d) {
+        c.xq[d] = d < D ? (int32_t)quant_of(r.x[d], P.iqs) : 0;
+        c.v[d] = r.v[d];
+      }
+      if (mode & GR_REC_INV) {  // 1/ρ and p/ρ² (the FluidPfn S = 2 force sweep)
+        const float ir = __builtin_amdgcn_rcpf(r.rho);
+        c.rho = ir;
+        c.p = r.p * (ir * ir);
+      } else {
+        c.rho = r.rho;
+        c.p = r.p;
+      }
+      P.rc[g] = c;
+    }
+  }
+  if constexpr (sizeof(R) == 4) {
+    if (mode & GR_REC_S) {  // stages with Cauchy sweeps
+      // the whole record also in 2D, where the sweeps read only its first half:
+      // writing half of every 32-byte record measured slower (partial lines)
+      RecS q;
+      q.a = make_float4(r.s[0], r.s[1], r.s[2], r.s[3]);
+      q.b = make_float4(r.s[4], r.s[5], r.s[6], r.s[7]);
+      P.rs[g] = q;
+    }
+  }
+}
+
 // update_ghost_kinematics! (:404-421): reflected half-step velocity of the
-// source and its density, with the normal of slot k.
-template <typename R, int D>
+// source and its density, with the normal of the ghost's slot.
+template <typename R>
+__device__ inline void ghost_kin(const Pool<R> &P, int64_t si, int64_t go, const Bnd &B, int D,
+                                 Rec<R> &r) {
+  R vr[3];
+#pragma unroll
+  for (int d = 0; d < 3; ++d) vr[d] = d < D ? P.vs[d][si] : (R)0;
+  R dd = vr[0] * (R)B.n[0];
+#pragma unroll
+  for (int d = 1; d < 3; ++d)
+    if (d < D) dd = dd + vr[d] * (R)B.n[d];
+#pragma unroll
+  for (int d = 0; d < 3; ++d) {
+    r.v[d] = d < D ? vr[d] - (R)2 * dd * (R)B.n[d] : (R)0;
+    if (d < D) P.vs[d][go] = r.v[d];
+  }
+  r.rho = P.rhos[si];
+  P.rhos[go] = r.rho;
+}
+template <typename R>
 __global__ void k_ghost_kin(Pool<R> P, const SysDesc *sd, const Bnd *bnd, const int *n_dev,
-                            const Blk *blk) {
+                            const Blk *blk, int D) {
   const Blk b = blk[blockIdx.x];
   const int g = b.item;
   const int k = b.first + threadIdx.x;
   const SysDesc G = sd[g];
   if (k >= n_dev[g]) return;
-  const SysDesc S = sd[G.src];
   const int64_t go = G.off + k;
-  const int64_t si = S.off + P.gidx[go];
-  const Bnd B = bnd[G.bnd + P.gnrm[go]];
-  R vr[D];
-#pragma unroll
-  for (int d = 0; d < D; ++d) vr[d] = P.vs[d][si];
-  R dd = vr[0] * (R)B.n[0];
-#pragma unroll
-  for (int d = 1; d < D; ++d) dd = dd + vr[d] * (R)B.n[d];
-#pragma unroll
-  for (int d = 0; d < D; ++d) P.vs[d][go] = vr[d] - (R)2 * dd * (R)B.n[d];
-  P.rhos[go] = P.rhos[si];
+  Rec<R> r;
+  ghost_kin(P, sd[G.src].off + P.gidx[go], go, bnd[G.bnd + P.gnrm[go]], D, r);
 }
 
 // _apply_mode(σ, HouseholderReflect(), n̂) (:66-110) in FP64, one function
@@ -1396,8 +1487,8 @@ __device__ inline void householder6(double *s, const double *n) {
 // GhostCopier of one stage (:112-129): copy p, copy or reflect stress.
 // copy[g] = {copy_p, stress_mode (-1 none, 0 plain, 1 Householder)}.
 template <typename R, int NS>
-__device__ __forceinline__ void ghost_copy_stress(Pool<R> P, int64_t si, int64_t go, int mode,
-                                         const double *n) {
+__device__ __forceinline__ void ghost_copy_stress(const Pool<R> &P, int64_t si, int64_t go, int mode,
+                                                  const double *n, Rec<R> &r) {
   double s[NS];
 #pragma unroll
   for (int q = 0; q < NS; ++q) s[q] = P.stress[q][si];
@@ -1407,9 +1498,24 @@ __device__ __forceinline__ void ghost_copy_stress(Pool<R> P, int64_t si, int64_t
     if (NS == 6) householder6(s, n);
   }
 #pragma unroll
-  for (int q = 0; q < NS; ++q) P.stress_s[q][go] = (R)s[q];
+  for (int q = 0; q < NS; ++q) {
+    P.stress_s[q][go] = (R)s[q];
+    r.s[q] = (float)(R)s[q];
+  }
 }
-
+template <typename R>
+__device__ inline void ghost_copy(const Pool<R> &P, const SysDesc &S, int64_t si, int64_t go,
+                                  int2 cp, const Bnd &B, Rec<R> &r) {
+  if (cp.x) {
+    r.p = P.p[si];
+    P.p[go] = r.p;
+  }
+  if (cp.y >= 0) {
+    if (S.ns == 3) ghost_copy_stress<R, 3>(P, si, go, cp.y, B.n, r);
+    if (S.ns == 4) ghost_copy_stress<R, 4>(P, si, go, cp.y, B.n, r);
+    if (S.ns == 6) ghost_copy_stress<R, 6>(P, si, go, cp.y, B.n, r);
+  }
+}
 template <typename R>
 __global__ void k_ghost_copy(Pool<R> P, const SysDesc *sd, const Bnd *bnd, const int *n_dev,
                              const Blk *blk, const int2 *copy) {
@@ -1418,17 +1524,37 @@ __global__ void k_ghost_copy(Pool<R> P, const SysDesc *sd, const Bnd *bnd, const
   const int k = b.first + threadIdx.x;
   const SysDesc G = sd[g];
   if (k >= n_dev[g]) return;
-  const SysDesc S = sd[G.src];
   const int64_t go = G.off + k;
-  const int64_t si = S.off + P.gidx[go];
-  const int2 cp = copy[g];
-  if (cp.x) P.p[go] = P.p[si];
-  if (cp.y >= 0) {
-    const Bnd B = bnd[G.bnd + P.gnrm[go]];
-    if (S.ns == 3) ghost_copy_stress<R, 3>(P, si, go, cp.y, B.n);
-    if (S.ns == 4) ghost_copy_stress<R, 4>(P, si, go, cp.y, B.n);
-    if (S.ns == 6) ghost_copy_stress<R, 6>(P, si, go, cp.y, B.n);
+  Rec<R> r;
+  ghost_copy(P, sd[G.src], sd[G.src].off + P.gidx[go], go, copy[g], bnd[G.bnd + P.gnrm[go]], r);
+}
+
+// Partner records: of the particles of `blk` (mode < 0: none), then of the
+// ghosts of `gblk`, with their kinematics and the stage's copies where asked.
+// One launch for what took up to four (kinematics, copies, two packs), each 2.5
+// to 4.5 us in a small scene and a chain of dependent loads: step of a 2D column
+// of 13k particles 122 -> 118 us with it and the records written by the
+// updaters, in FP64 of 2.3k 116 -> 110, 3D column of 179k 376 -> 371.
+template <typename R>
+__global__ void __launch_bounds__(GR_BLOCK)
+    k_pack(Pool<R> P, const SysDesc *sd, const int *n_dev, const Blk *blk, int nblk, int mode,
+           const Blk *gblk, int gmode, const Bnd *bnd, const int2 *copy, int kin, int D) {
+  const bool ghost = (int)blockIdx.x >= nblk;
+  const Blk b = ghost ? gblk[(int)blockIdx.x - nblk] : blk[blockIdx.x];
+  const int i = b.first + threadIdx.x;
+  if (i >= n_dev[b.item]) return;
+  const SysDesc S = sd[b.item];
+  const int64_t g = S.off + i;
+  Rec<R> r;
+  rec_load(P, S, g, D, ghost ? gmode : mode, r);
+  if (ghost && (kin || copy)) {
+    const SysDesc F = sd[S.src];
+    const int64_t si = F.off + P.gidx[g];
+    const Bnd B = bnd[S.bnd + P.gnrm[g]];
+    if (kin) ghost_kin(P, si, g, B, D, r);
+    if (copy) ghost_copy(P, F, si, g, copy[b.item], B, r);
   }
+  rec_store(P, g, D, ghost ? gmode : mode, r);
 }
 
 // ---------------------------------------------------------------------------
@@ -2013,7 +2139,7 @@ __device__ __forceinline__ void vpmc_update(Pool<R> P, int64_t g, int NS, double
 // Drucker-Prager updaters does not carry the registers of the others.
 template <typename R, int KM>
 __global__ void k_updaters(Pool<R> P, const SysDesc *sd, const StepSys *st, const Blk *blk,
-                           const int2 *urange, const UpdDesc *ud, int D) {
+                           const int2 *urange, const UpdDesc *ud, int D, int rec) {
   const Blk b = blk[blockIdx.x];
   const int s = b.item;
   const int i = b.first + threadIdx.x;
@@ -2115,6 +2241,11 @@ __global__ void k_updaters(Pool<R> P, const SysDesc *sd, const StepSys *st, cons
         break;
     }
   }
+  if (rec >= 0) {  // the partner records of the updated particle
+    Rec<R> w;
+    rec_load(P, S, g0, D, rec, w);
+    rec_store(P, g0, D, rec, w);
+  }
 }
 
 // Virtual systems: mode 0 refreshes the shadows of velocity and density
@@ -2183,70 +2314,6 @@ __global__ void k_virtual(Pool<R> P, const SysDesc *sd, const StepSys *st, const
 __global__ void k_fill_i32(int *p, int v, long long n) {
   long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) p[i] = v;
-}
-
-// Partner records of the live particles of the block's system (positions,
-// shadows of density and velocity, pressure), read by the pair sweeps.
-// S_ONLY: the stress records alone (the compact records of the previous
-// stage still hold: nothing in between wrote x, v, ρ or p).
-template <typename R, int D, bool C_ONLY, bool WITH_S, bool INV = false, bool S_ONLY = false>
-__global__ void k_pack(Pool<R> P, const SysDesc *sd, const int *n_dev, const Blk *blk) {
-  const Blk b = blk[blockIdx.x];
-  const int i = b.first + threadIdx.x;
-  if (i >= n_dev[b.item]) return;
-  const int64_t g = sd[b.item].off + i;
-  if constexpr (!S_ONLY) {
-  RecA<R> a;
-  RecB<R> r;
-#pragma unroll
-  for (int d = 0; d < 3; ++d) {
-    a.x[d] = d < D ? P.x[d][g] : 0.0;
-    r.v[d] = d < D ? P.vs[d][g] : (R)0;
-  }
-  a.rho = P.rhos[g];
-  if constexpr (sizeof(R) == 4) {
-    a.p = P.p[g];
-    r.pad = 0.0f;
-  } else {
-    r.p = P.p[g];
-  }
-  if (!C_ONLY) {
-    P.ra[g] = a;
-    P.rb[g] = r;
-  }
-  if constexpr (sizeof(R) == 4) {
-    RecC cc;
-#pragma unroll
-    for (int d = 0; d < 3; ++d) {
-      cc.xq[d] = d < D ? (int32_t)quant_of(a.x[d], P.iqs) : 0;
-      cc.v[d] = r.v[d];
-    }
-    if constexpr (INV) {  // 1/ρ and p/ρ² (the FluidPfn S = 2 force sweep)
-      const float ir = __builtin_amdgcn_rcpf(a.rho);
-      cc.rho = ir;
-      cc.p = a.p * (ir * ir);
-    } else {
-      cc.rho = a.rho;
-      cc.p = a.p;
-    }
-    P.rc[g] = cc;
-  }
-  }
-  if constexpr (sizeof(R) == 4 && WITH_S) {  // stages with Cauchy sweeps
-    const SysDesc S = sd[b.item];
-    float sv[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-    if (S.kind >= GR_SYS_STRESS) {
-#pragma unroll
-      for (int k = 0; k < GR_MAXNS; ++k)
-        if (k < S.ns) sv[k] = (float)P.stress_s[k][g];
-    }
-    // the whole record also in 2D, where the sweeps read only its first half:
-    // writing half of every 32-byte record measured slower (partial lines)
-    RecS rs;
-    rs.a = make_float4(sv[0], sv[1], sv[2], sv[3]);
-    rs.b = make_float4(sv[4], sv[5], sv[6], sv[7]);
-    P.rs[g] = rs;
-  }
 }
 
 // ---------------------------------------------------------------------------
@@ -2466,10 +2533,7 @@ template <typename R>
 void launch_ghost_kin(hipStream_t s, const Pool<R> &P, const SysDesc *sd, const Bnd *bnd,
                       const int *n, const Blk *blk, int nblk, int D) {
   if (nblk <= 0) return;
-  if (D == 2)
-    k_ghost_kin<R, 2><<<nblk, GR_BLOCK, 0, s>>>(P, sd, bnd, n, blk);
-  else
-    k_ghost_kin<R, 3><<<nblk, GR_BLOCK, 0, s>>>(P, sd, bnd, n, blk);
+  k_ghost_kin<R><<<nblk, GR_BLOCK, 0, s>>>(P, sd, bnd, n, blk, D);
 }
 template void launch_ghost_kin<float>(hipStream_t, const Pool<float> &, const SysDesc *,
                                       const Bnd *, const int *, const Blk *, int, int);
@@ -2562,13 +2626,14 @@ void launch_xsph(hipStream_t s, const Pool<R> &P, const SysDesc *sd, const StepS
 template <typename R>
 void launch_updaters(hipStream_t s, const Pool<R> &P, const SysDesc *sd, const StepSys *st,
                      const Blk *blk, int nblk, const int2 *urange, const UpdDesc *ud, int D,
-                     int kinds) {
+                     int kinds, int rec) {
   if (nblk <= 0) return;
   constexpr int Z = 1 << GR_UPD_ZERO | 1 << GR_UPD_NOTHING;
   constexpr int K_EP = Z | 1 << GR_UPD_EP, K_VPMC = Z | 1 << GR_UPD_VPMC,
                 K_EOS = Z | 1 << GR_UPD_TAIT | 1 << GR_UPD_LINEAR, K_HOOKE = Z | 1 << GR_UPD_HOOKE;
   auto go = [&](auto km) {
-    k_updaters<R, decltype(km)::value><<<nblk, GR_BLOCK, 0, s>>>(P, sd, st, blk, urange, ud, D);
+    k_updaters<R, decltype(km)::value><<<nblk, GR_BLOCK, 0, s>>>(P, sd, st, blk, urange, ud, D,
+                                                              rec);
   };
   if ((kinds & ~K_EP) == 0)
     go(std::integral_constant<int, K_EP>{});
@@ -2596,7 +2661,7 @@ void launch_updaters(hipStream_t s, const Pool<R> &P, const SysDesc *sd, const S
                                const int *, const Blk *, int, int, int);                       \
   template void launch_updaters<R>(hipStream_t, const Pool<R> &, const SysDesc *,              \
                                    const StepSys *, const Blk *, int, const int2 *,            \
-                                   const UpdDesc *, int, int);
+                                   const UpdDesc *, int, int, int);
 INST(float)
 INST(double)
 #undef INST
@@ -2615,48 +2680,20 @@ template void launch_virtual<float>(hipStream_t, const Pool<float> &, const SysD
 template void launch_virtual<double>(hipStream_t, const Pool<double> &, const SysDesc *,
                                      const StepSys *, const int *, const Blk *, int, int, int);
 
-template <typename R, bool C_ONLY, bool WITH_S>
-static void launch_pack_d(hipStream_t s, const Pool<R> &P, const SysDesc *sd, const int *n,
-                          const Blk *blk, int nblk, int D) {
-  if (D == 2)
-    k_pack<R, 2, C_ONLY, WITH_S><<<nblk, GR_BLOCK, 0, s>>>(P, sd, n, blk);
-  else
-    k_pack<R, 3, C_ONLY, WITH_S><<<nblk, GR_BLOCK, 0, s>>>(P, sd, n, blk);
-}
-
 template <typename R>
 void launch_pack(hipStream_t s, const Pool<R> &P, const SysDesc *sd, const int *n, const Blk *blk,
-                 int nblk, int D, bool c_only, bool with_s, bool inv, bool s_only) {
-  if (nblk <= 0) return;
-  c_only = c_only && sizeof(R) == 4;
-  if (s_only) {  // FP32 compact records only
-    if (!(c_only && with_s)) return;
-    if (D == 2)
-      k_pack<R, 2, true, true, false, true><<<nblk, GR_BLOCK, 0, s>>>(P, sd, n, blk);
-    else
-      k_pack<R, 3, true, true, false, true><<<nblk, GR_BLOCK, 0, s>>>(P, sd, n, blk);
-    return;
-  }
-  if (inv && c_only && !with_s && sizeof(R) == 4) {
-    if (D == 2)
-      k_pack<R, 2, true, false, true><<<nblk, GR_BLOCK, 0, s>>>(P, sd, n, blk);
-    else
-      k_pack<R, 3, true, false, true><<<nblk, GR_BLOCK, 0, s>>>(P, sd, n, blk);
-    return;
-  }
-  if (c_only && with_s)
-    launch_pack_d<R, true, true>(s, P, sd, n, blk, nblk, D);
-  else if (c_only)
-    launch_pack_d<R, true, false>(s, P, sd, n, blk, nblk, D);
-  else if (with_s)
-    launch_pack_d<R, false, true>(s, P, sd, n, blk, nblk, D);
-  else
-    launch_pack_d<R, false, false>(s, P, sd, n, blk, nblk, D);
+                 int nblk, int mode, const Blk *gblk, int ngblk, int gmode, const Bnd *bnd,
+                 const int2 *copy, bool kin, int D) {
+  if (nblk + ngblk > 0)
+    k_pack<R><<<nblk + ngblk, GR_BLOCK, 0, s>>>(P, sd, n, blk, nblk, mode, gblk, gmode, bnd, copy,
+                                                kin ? 1 : 0, D);
 }
 template void launch_pack<float>(hipStream_t, const Pool<float> &, const SysDesc *, const int *,
-                                 const Blk *, int, int, bool, bool, bool, bool);
+                                 const Blk *, int, int, const Blk *, int, int, const Bnd *,
+                                 const int2 *, bool, int);
 template void launch_pack<double>(hipStream_t, const Pool<double> &, const SysDesc *, const int *,
-                                  const Blk *, int, int, bool, bool, bool, bool);
+                                  const Blk *, int, int, const Blk *, int, int, const Bnd *,
+                                  const int2 *, bool, int);
 
 // Probe slot id[i] − 1 takes the position of mirror particle i
 // (_measure_probes!, src/TimeIntegration.jl:469-479).

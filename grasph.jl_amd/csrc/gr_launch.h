@@ -172,20 +172,29 @@ template <typename R>
 void launch_xsph(hipStream_t s, const Pool<R> &P, const SysDesc *sd, const StepSys *st,
                  const int *n, const Blk *blk, int nblk, int D, int mode);
 template <typename R>
-// kinds: the set of updater kinds (bit GR_UPD_x) in ud
+// kinds: the set of updater kinds (bit GR_UPD_x) in ud; rec: the partner
+// records written of every particle of blk after its updates, -1: none
 void launch_updaters(hipStream_t s, const Pool<R> &P, const SysDesc *sd, const StepSys *st,
                      const Blk *blk, int nblk, const int2 *urange, const UpdDesc *ud, int D,
-                     int kinds);
+                     int kinds, int rec = -1);
 template <typename R>
 void launch_sweep(hipStream_t s, const Pool<R> &P, const SweepArgs &a, int D, int fam, bool cnt);
 template <typename R>
 void launch_virtual(hipStream_t s, const Pool<R> &P, const SysDesc *sd, const StepSys *st,
                     const int *n, const Blk *blk, int nblk, int mode, int D);
+// Which partner records are written (FP64 pools: always RecA and RecB alone).
+enum {
+  GR_REC_C = 1,       // the compact records alone
+  GR_REC_S = 2,       // the stress records
+  GR_REC_INV = 4,     // compact records of 1/ρ and p/ρ²
+  GR_REC_S_ONLY = 8,  // the stress records alone (the compact ones still hold)
+};
+// Records `mode` of the particles of blk, `gmode` of the ghosts of gblk; the
+// latter after the kinematics (kin) and the copies of a stage (copy) if asked.
 template <typename R>
-// s_only: the FP32 stress records alone (the compact records still hold)
 void launch_pack(hipStream_t s, const Pool<R> &P, const SysDesc *sd, const int *n, const Blk *blk,
-                 int nblk, int D, bool c_only = false, bool with_s = true, bool inv = false,
-                 bool s_only = false);
+                 int nblk, int mode, const Blk *gblk, int ngblk, int gmode, const Bnd *bnd,
+                 const int2 *copy, bool kin, int D);
 template <typename R>
 void launch_nlist(hipStream_t s, const Pool<R> &P, const NlistArgs &a, int D);
 void launch_fill_i32(hipStream_t s, int *p, int v, long long n);
