@@ -2316,6 +2316,43 @@ __global__ void k_fill_i32(int *p, int v, long long n) {
   if (i < n) p[i] = v;
 }
 
+// Fields between the caller's layout (particle-major FP64, staged in pinned host
+// memory) and the pool's component arrays: element e of `host` is component
+// e % nc of particle e / nc.  The kernels read and write the host memory over
+// the bus themselves, so a transfer is one launch, in whole lines both ways.
+__global__ void __launch_bounds__(GR_BLOCK)
+    k_field_in(const double *host, int64_t count, int nc, int64_t cap, int64_t off, FieldSets F) {
+  const int64_t e = (int64_t)blockIdx.x * GR_BLOCK + threadIdx.x;
+  if (e >= count) return;
+  const double v = host[e];
+  const int64_t at = (e % nc) * cap + off + e / nc;
+  for (int q = 0; q < F.n; ++q) {
+    if (F.esz[q] == 8)
+      static_cast<double *>(F.p[q])[at] = v;
+    else
+      static_cast<float *>(F.p[q])[at] = (float)v;
+  }
+}
+__global__ void __launch_bounds__(GR_BLOCK)
+    k_field_out(double *host, int64_t count, int nc, int64_t cap, int64_t off, FieldSets F) {
+  const int64_t e = (int64_t)blockIdx.x * GR_BLOCK + threadIdx.x;
+  if (e >= count) return;
+  const int64_t at = (e % nc) * cap + off + e / nc;
+  host[e] = F.esz[0] == 8 ? static_cast<const double *>(F.p[0])[at]
+                          : (double)static_cast<const float *>(F.p[0])[at];
+}
+// 32-bit indices, the caller's being 64-bit and `add` larger.
+__global__ void __launch_bounds__(GR_BLOCK)
+    k_index_in(const int64_t *host, int64_t count, int64_t off, int add, int *dst) {
+  const int64_t e = (int64_t)blockIdx.x * GR_BLOCK + threadIdx.x;
+  if (e < count) dst[off + e] = (int)(host[e] - add);
+}
+__global__ void __launch_bounds__(GR_BLOCK)
+    k_index_out(int64_t *host, int64_t count, int64_t off, int add, const int *src) {
+  const int64_t e = (int64_t)blockIdx.x * GR_BLOCK + threadIdx.x;
+  if (e < count) host[e] = (int64_t)src[off + e] + add;
+}
+
 // ---------------------------------------------------------------------------
 // Host launchers
 // ---------------------------------------------------------------------------
@@ -2665,6 +2702,23 @@ void launch_updaters(hipStream_t s, const Pool<R> &P, const SysDesc *sd, const S
 INST(float)
 INST(double)
 #undef INST
+
+void launch_field(hipStream_t s, bool in, double *host, int64_t count, int nc, int64_t cap,
+                  int64_t off, const FieldSets &F) {
+  if (count <= 0) return;
+  if (in)
+    k_field_in<<<nb_of(count, GR_BLOCK), GR_BLOCK, 0, s>>>(host, count, nc, cap, off, F);
+  else
+    k_field_out<<<nb_of(count, GR_BLOCK), GR_BLOCK, 0, s>>>(host, count, nc, cap, off, F);
+}
+void launch_index(hipStream_t s, bool in, int64_t *host, int64_t count, int64_t off, int add,
+                  int *dev) {
+  if (count <= 0) return;
+  if (in)
+    k_index_in<<<nb_of(count, GR_BLOCK), GR_BLOCK, 0, s>>>(host, count, off, add, dev);
+  else
+    k_index_out<<<nb_of(count, GR_BLOCK), GR_BLOCK, 0, s>>>(host, count, off, add, dev);
+}
 
 template <typename R>
 void launch_virtual(hipStream_t s, const Pool<R> &P, const SysDesc *sd, const StepSys *st,

@@ -197,6 +197,18 @@ void launch_pack(hipStream_t s, const Pool<R> &P, const SysDesc *sd, const int *
                  const int2 *copy, bool kin, int D);
 template <typename R>
 void launch_nlist(hipStream_t s, const Pool<R> &P, const NlistArgs &a, int D);
+// A field's arrays on the device (component k at k·cap): the field itself, and
+// on the way in the shadows that follow it.
+struct FieldSets {
+  void *p[3];
+  int esz[3];  // 8: double, 4: float
+  int n;
+};
+// `count` elements between pinned host memory and the particles from `off` on.
+void launch_field(hipStream_t s, bool in, double *host, int64_t count, int nc, int64_t cap,
+                  int64_t off, const FieldSets &F);
+void launch_index(hipStream_t s, bool in, int64_t *host, int64_t count, int64_t off, int add,
+                  int *dev);
 void launch_fill_i32(hipStream_t s, int *p, int v, long long n);
 void launch_alias_check(hipStream_t s, const int *n, int ghost, int src_n, int *flags);
 template <typename R>
