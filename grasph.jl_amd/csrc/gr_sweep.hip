@@ -710,8 +710,14 @@ __global__ void __launch_bounds__(GR_BLOCK)
 // start within span·wmax of the lowest pending start form a group (targets
 // in one cell column); the group's union of ranges is staged in LDS, WIN
 // candidates at a time, with coalesced loads, and every lane walks its own
-// range from LDS in ascending order, so it tests each candidate once with the
-// walk's FP64 expression and sets the candidate's bit: no per-partner store.
+// range from LDS in ascending order and sets the bits of the candidates that
+// pass the walk's test: no per-partner store.  The staged candidates are FP32
+// offsets, on which all but the closest calls are decided exactly (Screen).
+// The search is bound by its vector instructions (the loads of a strip hide
+// behind the tests of the wavefronts next to it): testing all in FP64 took 8 FP64
+// operations a candidate, a comparison and the bit's insertion, 307 us in the
+// 3D dam break of 1.4M particles and 84 for 64 2D columns; the screen, 8 FP32
+// operations in all, takes 214 and 74.
 // WIN and span change only which lanes load together, never a lane's tests
 // or their order: every choice gives the same lists.
 // Wave-wide minimum / maximum (all 64 lanes active): DPP within each row of
@@ -727,6 +733,100 @@ __device__ inline int wave_red_dpp(int v) {
             op(__builtin_amdgcn_readlane(v, 32), __builtin_amdgcn_readlane(v, 48)));
 }
 
+// The walk's test r² < c² (FP64) screened in FP32: candidates and target as
+// offsets from a point O near the wavefront's targets, r = Σ(x − x_j)² − c² by
+// three subtractions and three FMAs, whose sign is the answer wherever |r|
+// exceeds the FP32 error bound `tol`; the others are tested in FP64.
+//
+// Bound, with u = 2⁻²⁴, X the target's largest offset and c the cell (c² >=
+// cutoff²).  A candidate of the cells around the target's differs from it by
+// a <= 2c in each dimension: both offsets round by at most u(2X + 2c) together,
+// their difference by ua, so r errs by 2Σa·u(2X + 4c) <= u(24cX + 48c²), and by
+// 3u·12c² in the sums and uc² in c².  A candidate farther than 2c (of cells out
+// of the sort's order) has r >= 3/4 a² and an error of u(12aX + 22a²), too
+// small to change its sign while X <= 1e5 c; beyond that all are tested.
+template <int D>
+struct Screen {
+  float xf[D], c2, tol;
+  bool finite;
+  __device__ inline void set(const double *xi, const double *O) {
+    finite = true;
+#pragma unroll
+    for (int d = 0; d < D; ++d) {
+      xf[d] = (float)(xi[d] - O[d]);
+      finite = finite && fabsf(xf[d]) < 3.0e38f;  // a non-finite target has no partner
+    }
+  }
+  __device__ inline void source(double cutoff2, double cell) {
+    float X = fabsf(xf[0]);
+#pragma unroll
+    for (int d = 1; d < D; ++d) X = fmaxf(X, fabsf(xf[d]));
+    const float c = (float)cell;
+    c2 = (float)cutoff2;
+    tol = 6.1e-8f * (c * (24.0f * X + 96.0f * c));
+    if (!(X <= 1.0e5f * c) || !(cutoff2 <= cell * cell * (1.0 + 1e-9))) tol = __builtin_inff();
+  }
+  // a staged coordinate; a non-finite one is far from every target
+  static __device__ inline float stage(double x, double o) {
+    const float f = (float)(x - o);
+    return fabsf(f) < 3.0e38f ? f : 3.0e38f;
+  }
+};
+// A point near the wavefront's targets (uniform): the first lane's.
+template <int D>
+__device__ inline void screen_origin(const double *xi, double *O) {
+#pragma unroll
+  for (int d = 0; d < D; ++d) {
+    const unsigned long long b = (unsigned long long)__double_as_longlong(xi[d]);
+    const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)b);
+    const unsigned hi = __builtin_amdgcn_readfirstlane((unsigned)(b >> 32));
+    O[d] = __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+    if (!(fabs(O[d]) < 1.0e300)) O[d] = 0.0;
+  }
+}
+
+// Screened signs of the four candidates staged at t, the first one's highest, in
+// the low bits of `cur` (shifted up); returns the smallest |r| less `tol`.
+template <int D, int W>
+__device__ __forceinline__ float screen4(const Screen<D> &scr, const float (*sf)[W], int t,
+                                         unsigned &cur) {
+  float r[4];
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    const float a0 = scr.xf[0] - sf[0][t + u];
+    r[u] = fmaf(a0, a0, -scr.c2);
+  }
+#pragma unroll
+  for (int k = 1; k < D; ++k)
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const float ak = scr.xf[k] - sf[k][t + u];
+      r[u] = fmaf(ak, ak, r[u]);
+    }
+#pragma unroll
+  for (int u = 0; u < 4; ++u) cur = __builtin_amdgcn_alignbit(cur, __float_as_uint(r[u]), 31);
+  return fminf(fminf(fabsf(r[0]), fabsf(r[1])), fminf(fabsf(r[2]), fabsf(r[3]))) - scr.tol;
+}
+// The walk's own test of pool indices g .. g + 3 (none beyond `last` is read).
+template <int D, typename R>
+__device__ inline unsigned exact4(const Pool<R> &P, const double *xi, double c2, int64_t g,
+                                  int64_t last) {
+  unsigned ex = 0u;
+#pragma unroll 1  // seldom run: registers count
+  for (int u = 0; u < 4; ++u) {
+    const int64_t j = g + u < last ? g + u : last;
+    const double a0 = xi[0] - P.x[0][j];
+    double r2 = a0 * a0;
+#pragma unroll
+    for (int k = 1; k < D; ++k) {
+      const double ak = xi[k] - P.x[k][j];
+      r2 = r2 + ak * ak;
+    }
+    ex = (ex << 1) | (unsigned)(r2 < c2);
+  }
+  return ex;
+}
+
 template <int D, typename R, int WIN>
 __global__ void __launch_bounds__(64)
     k_nlist(Pool<R> P, const SysDesc *__restrict__ sd, const int *__restrict__ n_dev,
@@ -735,7 +835,7 @@ __global__ void __launch_bounds__(64)
             const int *__restrict__ cells, const Blk *__restrict__ blk, int nblk, int *lcnt,
             int *lidx, const long long *__restrict__ bbmin,
             const long long *__restrict__ bbmax, int span) {
-  __shared__ double sx[D][WIN];
+  __shared__ float sf[D][WIN + 4];
   const Blk b = blk[xcd_block(nblk)];
   const LTask L = lt[b.item];
   const int lane = threadIdx.x;
@@ -748,6 +848,10 @@ __global__ void __launch_bounds__(64)
   for (int d = 0; d < D; ++d) xi[d] = P.x[d][gi];
   int2 *emask = reinterpret_cast<int2 *>(lidx + L.list_off) + i;
   int *ebase = lidx + L.list_off + 2 * (int64_t)L.maxnb * L.cap + i;
+  double O[D];
+  Screen<D> scr;
+  screen_origin<D>(xi, O);
+  scr.set(xi, O);
   int ne = 0;  // entries of this target
   int cq = 0;  // entries of the current source
   for (int q = L.src_begin; q < L.src_end; ++q) {
@@ -764,7 +868,8 @@ __global__ void __launch_bounds__(64)
       // a dynamic boundary (a sorted real system, its bounds taken this
       // step) more than a cutoff from the target along some axis holds no
       // partner: the margin keeps every FP64 r² of such a pair above c2
-      bool act = live;
+      bool act = live && scr.finite;
+      scr.source(c2, Q.cell);
       if (Q.pk == PK_DYNAMIC && bbmin) {
 #pragma unroll
         for (int d = 0; d < D; ++d) {
@@ -824,7 +929,7 @@ __global__ void __launch_bounds__(64)
             __syncthreads();  // the previous window has been read
             for (int t = lane; t < w1 - w0; t += 64) {
 #pragma unroll
-              for (int k = 0; k < D; ++k) sx[k][t] = P.x[k][poff + w0 + t];
+              for (int k = 0; k < D; ++k) sf[k][t] = scr.stage(P.x[k][poff + w0 + t], O[k]);
             }
             __syncthreads();
             // this lane's candidates in the window end before je; base + d is
@@ -840,52 +945,24 @@ __global__ void __launch_bounds__(64)
               const int wsel = d >> 5;
               const int lim = je - base, wend = (d & ~31) + 32;
               const int dend = lim < wend ? lim : wend;
-              const int toff = base - w0;
-              unsigned cur = 0u;
-              // four, then two candidates per iteration (independent chains)
-              for (; d + 3 < dend; d += 4) {
-                const int t = d + toff;
-                double r[4];
-#pragma unroll
-                for (int u = 0; u < 4; ++u) {
-                  const double a0 = xi[0] - sx[0][t + u];
-                  r[u] = a0 * a0;
-                }
-#pragma unroll
-                for (int k = 1; k < D; ++k)
-#pragma unroll
-                  for (int u = 0; u < 4; ++u) {
-                    const double ak = xi[k] - sx[k][t + u];
-                    r[u] = r[u] + ak * ak;
-                  }
-                cur |= ((unsigned)(r[0] < c2) | ((unsigned)(r[1] < c2) << 1) |
-                        ((unsigned)(r[2] < c2) << 2) | ((unsigned)(r[3] < c2) << 3))
-                       << (d & 31);
+              // four at a time, the last four beyond the run's end if need be
+              // (read, never kept); nr has a bit for each four that hold one
+              // too close to call
+              const int n = dend - d, ng = (n + 3) >> 2, t0 = base - w0 + d;
+              unsigned cur = 0u, nr = 0u;
+              for (int t = t0; t < t0 + n; t += 4)
+                nr = __builtin_amdgcn_alignbit(
+                    nr, __float_as_uint(screen4<D>(scr, sf, t, cur)), 31);
+              while (nr != 0u) {
+                const int g = __builtin_ctz(nr);
+                nr &= nr - 1u;
+                cur &= ~(15u << (4 * g));
+                cur |= exact4<D>(P, xi, c2, poff + base + d + 4 * (ng - 1 - g), poff + w1 - 1)
+                       << (4 * g);
               }
-              for (; d + 1 < dend; d += 2) {
-                const int t = d + toff;
-                const double a0 = xi[0] - sx[0][t], b0 = xi[0] - sx[0][t + 1];
-                double ra = a0 * a0, rb = b0 * b0;
-#pragma unroll
-                for (int k = 1; k < D; ++k) {
-                  const double ak = xi[k] - sx[k][t], bk = xi[k] - sx[k][t + 1];
-                  ra = ra + ak * ak;
-                  rb = rb + bk * bk;
-                }
-                cur |= ((unsigned)(ra < c2) | ((unsigned)(rb < c2) << 1)) << (d & 31);
-              }
-              if (d < dend) {
-                const int t = d + toff;
-                const double a0 = xi[0] - sx[0][t];
-                double r2 = a0 * a0;
-#pragma unroll
-                for (int k = 1; k < D; ++k) {
-                  const double ak = xi[k] - sx[k][t];
-                  r2 = r2 + ak * ak;
-                }
-                cur |= (unsigned)(r2 < c2) << (d & 31);
-                ++d;
-              }
+              cur = (__brev(cur) >> (32 - 4 * ng)) & (~0u >> (32 - n));
+              cur <<= d & 31;
+              d = dend;
               // selects, not branches (here and when the target's own bit
               // is cleared): branches make the compiler index a pair
               // {lo, hi} kept in scratch memory
@@ -912,13 +989,13 @@ __device__ __forceinline__ unsigned quad_or(unsigned v) {
 }
 
 // The search with S lanes per target (64 / S targets per wavefront, S
-// wavefronts per entry of the block table): lane s of a target tests its
-// candidates j with j mod S = s, and the masks are the OR of the S lanes', so
+// wavefronts per entry of the block table): lane s of a target tests four of
+// every 16 of its candidates, and the masks are the OR of the S lanes', so
 // the lists are k_nlist's.  For launches of few targets, which latency bounds
 // (nlist_split_blocks): S times the wavefronts, each with 1/S of the tests and
 // about half the candidates to stage; a launch that fills the chip pays S
-// times k_nlist's work per strip instead (3D dam break of 1.4M: 441 us against
-// 309).
+// times k_nlist's work per strip instead (3D dam break of 512k: 217 us against
+// 132).
 template <int D, typename R, int WIN, int S_>
 __global__ void __launch_bounds__(64)
     k_nlist_split(Pool<R> P, const SysDesc *__restrict__ sd, const int *__restrict__ n_dev,
@@ -928,7 +1005,7 @@ __global__ void __launch_bounds__(64)
                   int *lidx, const long long *__restrict__ bbmin,
                   const long long *__restrict__ bbmax, int span) {
   static_assert(S_ == 4, "quad_or joins four lanes");
-  __shared__ double sx[D][WIN];
+  __shared__ float sf[D][WIN + 4];
   const int lb = xcd_block(nblk * S_);
   const Blk b = blk[lb / S_];
   const LTask L = lt[b.item];
@@ -943,6 +1020,10 @@ __global__ void __launch_bounds__(64)
   for (int d = 0; d < D; ++d) xi[d] = P.x[d][gi];
   int2 *emask = reinterpret_cast<int2 *>(lidx + L.list_off) + i;
   int *ebase = lidx + L.list_off + 2 * (int64_t)L.maxnb * L.cap + i;
+  double O[D];
+  Screen<D> scr;
+  screen_origin<D>(xi, O);
+  scr.set(xi, O);
   int ne = 0;  // entries of this target
   int cq = 0;  // entries of the current source
   for (int q = L.src_begin; q < L.src_end; ++q) {
@@ -954,7 +1035,8 @@ __global__ void __launch_bounds__(64)
       const int self_j = Q.pk == PK_SELF ? i : -1;
       const double c2 = Q.cutoff2;
       const int64_t poff = sd[Q.partner].off;
-      bool act = live;  // as in k_nlist
+      bool act = live && scr.finite;  // as in k_nlist
+      scr.source(c2, Q.cell);
       if (Q.pk == PK_DYNAMIC && bbmin) {
 #pragma unroll
         for (int d = 0; d < D; ++d) {
@@ -1014,7 +1096,7 @@ __global__ void __launch_bounds__(64)
               __syncthreads();  // the previous window has been read
               for (int t = lane; t < w1 - w0; t += 64) {
 #pragma unroll
-                for (int k = 0; k < D; ++k) sx[k][t] = P.x[k][poff + w0 + t];
+                for (int k = 0; k < D; ++k) sf[k][t] = scr.stage(P.x[k][poff + w0 + t], O[k]);
               }
               __syncthreads();
               // the target's candidates in the window, [js, je): the same for
@@ -1029,38 +1111,25 @@ __global__ void __launch_bounds__(64)
                 while (true) {
                   const int ce = je < base + 64 ? je : base + 64;
                   const int jb = js > base ? js : base;
-                  int d = jb - base + ((sl - jb) & (S_ - 1));
-                  const int t0 = base - w0, de = ce - base;
-                  unsigned long long cur = 0ull;
-                  for (; d + 3 * S_ < de; d += 4 * S_) {
-                    double r[4];
+                  // the four lanes take four candidates each in turn: lane sl
+                  // those at 4·sl of every 16
+                  const int n = ce - jb;
+                  unsigned part[4];
 #pragma unroll
-                    for (int u = 0; u < 4; ++u) {
-                      const double a0 = xi[0] - sx[0][t0 + d + u * S_];
-                      r[u] = a0 * a0;
+                  for (int m = 0; m < 4; ++m) {
+                    const int o = 16 * m + 4 * sl;
+                    unsigned sg = 0u;
+                    if (o < n) {
+                      if (screen4<D>(scr, sf, jb - w0 + o, sg) < 0.0f)
+                        sg = exact4<D>(P, xi, c2, poff + jb + o, poff + w1 - 1);
+                      sg = __brev(sg) >> 28;
                     }
-#pragma unroll
-                    for (int k = 1; k < D; ++k)
-#pragma unroll
-                      for (int u = 0; u < 4; ++u) {
-                        const double ak = xi[k] - sx[k][t0 + d + u * S_];
-                        r[u] = r[u] + ak * ak;
-                      }
-                    const unsigned m4 = (unsigned)(r[0] < c2) | ((unsigned)(r[1] < c2) << S_) |
-                                        ((unsigned)(r[2] < c2) << (2 * S_)) |
-                                        ((unsigned)(r[3] < c2) << (3 * S_));
-                    cur |= (unsigned long long)m4 << d;
+                    part[m] = sg << (4 * sl);
                   }
-                  for (; d < de; d += S_) {
-                    const double a0 = xi[0] - sx[0][t0 + d];
-                    double r2 = a0 * a0;
-#pragma unroll
-                    for (int k = 1; k < D; ++k) {
-                      const double ak = xi[k] - sx[k][t0 + d];
-                      r2 = r2 + ak * ak;
-                    }
-                    cur |= (unsigned long long)(unsigned)(r2 < c2) << d;
-                  }
+                  unsigned long long cur =
+                      ((unsigned long long)(part[2] | part[3] << 16) << 32) |
+                      (part[0] | part[1] << 16);
+                  cur = (cur & (~0ull >> (64 - n))) << (jb - base);
                   lo |= (unsigned)cur;
                   hi |= (unsigned)(cur >> 32);
                   if (base + 64 >= je) break;
@@ -1572,12 +1641,13 @@ template void launch_sweep<double>(hipStream_t, const Pool<double> &, const Swee
 // Up to this many blocks of 64 targets the search takes four lanes per target:
 // with one, such a launch has at most about two wavefronts per SIMD, and a
 // wavefront's own chain of loads and tests is the launch's time.  Measured, us
-// with one / four lanes: 3D dam breaks of 422 blocks 92 / 52, 1000 88 / 56,
-// 1954 101 / 89, 3375 121 / 122, 5593 163 / 181; 2D of 313 blocks 20 / 16,
-// 1250 19.7 / 18.8, 2552 24 / 28 (EP columns of 1600 blocks 21 / 24).
+// with one / four lanes: 3D dam breaks of 422 blocks 80 / 50, 1000 77 / 52,
+// 1954 81 / 82, 3375 88 / 110, 5593 122 / 167 (columns of 1500 blocks 73 / 65,
+// 2250 78 / 81); 2D of 313 blocks 19 / 16, 1250 19.1 / 19.4, 2552 23 / 31 (EP
+// columns of 1600 blocks 20 / 24).
 template <int D>
 constexpr int nlist_split_blocks() {
-  return D == 3 ? 2400 : 1200;
+  return D == 3 ? 1950 : 1200;
 }
 
 template <int D, typename R, int WIN>
