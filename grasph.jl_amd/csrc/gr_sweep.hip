@@ -1395,6 +1395,20 @@ struct Terms {
 // their list entry and the terms are exchanged (19 moves a round), so a launch
 // that fills the chip is slower with it (3D dam break of 1.4M: 456 us against
 // 349).
+// Entries of a target staged in LDS (a multiple of 4; the others are loaded as
+// they come up), and sources whose counts are.
+#define SPLIT_ENTRIES 24
+#define SPLIT_SOURCES 8
+// Where that pays: not in the 2D fluid sweeps, whose few entries (three strips a
+// source) come and go behind the walls' short sources.  Measured, us with the
+// entries loaded one ahead / staged: 2D column of 13k in FP32 25.2 / 13.8 (Cauchy
+// force), 3D dam break of 224k 74 / 69, 3D column of 16k 50.8 / 49.4, 2D dam break
+// of 13k in FP64 15.9 / 17.2.
+template <int D, int FAM>
+constexpr bool split_stages() {
+  return D == 3 || (FAM != FAM_FORCE_FLUID && FAM != FAM_FORCE_FLUID_INV);
+}
+
 template <int D, typename R, int FAM, bool CNT>
 __global__ void __launch_bounds__(64)
     k_sweep_split(Pool<R> P, const SysDesc *__restrict__ sd, const int *__restrict__ n_dev,
@@ -1419,23 +1433,66 @@ __global__ void __launch_bounds__(64)
   const int nls = L.src_end - L.src_begin;
   const bool overflow =
       live && (T.ltask < 0 || lcnt[L.cnt_off + (int64_t)nls * L.cap + i] != 0);
+  // the targets' entries come to LDS first, all loads in flight together: in
+  // the pair loop an entry's load would hold up the records behind it, and the
+  // search has just written the entries on other XCDs, so each is a miss of L2
+  constexpr bool STAGE = split_stages<D, FAM>();
+  constexpr int LE = STAGE ? SPLIT_ENTRIES : 4, LS = STAGE ? SPLIT_SOURCES : 1;
+  __shared__ unsigned long long s_mask[LE][16];
+  __shared__ int s_base[LE][16];
+  __shared__ int s_cnt[LS][16];
+  const int tg = threadIdx.x >> 2;
+  if (STAGE && live && !overflow) {
+    const unsigned long long *em =
+        reinterpret_cast<const unsigned long long *>(lidx + L.list_off) + i;
+    const int *eb = lidx + L.list_off + 2 * (int64_t)L.maxnb * L.cap + i;
+    int cnt[LS], tot = 0;
+#pragma unroll
+    for (int l = 0; l < LS; ++l)
+      cnt[l] = l < nls ? lcnt[L.cnt_off + (int64_t)l * L.cap + i] : 0;
+#pragma unroll
+    for (int l = 0; l < LS; ++l) {
+      tot += cnt[l];
+      if (sl == 0) s_cnt[l][tg] = cnt[l];
+    }
+    unsigned long long m[LE / 4];
+    int bs[LE / 4];
+#pragma unroll
+    for (int k = 0; k < LE / 4; ++k) {
+      const int e = 4 * k + sl;
+      m[k] = e < tot ? em[(int64_t)e * L.cap] : 0ull;
+      bs[k] = e < tot ? eb[(int64_t)e * L.cap] : 0;
+    }
+#pragma unroll
+    for (int k = 0; k < LE / 4; ++k) {
+      s_mask[4 * k + sl][tg] = m[k];
+      s_base[4 * k + sl][tg] = bs[k];
+    }
+  }
+  if (STAGE) __syncthreads();
   using TT = Terms<D, R, FAM>;
   double sum[TT::NG] = {};
   if (live && !overflow) {
     Gather<D, R, FAM, Term<R>> Gp;
     Gp.load(P, S, T, gi);
     constexpr bool CMP = Gather<D, R, FAM>::COMPACT;
-    const int2 *emask = reinterpret_cast<const int2 *>(lidx + L.list_off) + i;
+    const unsigned long long *emask =
+        reinterpret_cast<const unsigned long long *>(lidx + L.list_off) + i;
     const int *ebase = lidx + L.list_off + 2 * (int64_t)L.maxnb * L.cap + i;
     // -1 for each of the lanes before this one in the quad, as the addend
     // that drops a mask's lowest bit
     const unsigned c1 = sl > 0 ? ~0u : 0u, c2 = sl > 1 ? ~0u : 0u, c3 = sl > 2 ? ~0u : 0u;
+    // entries staged: all up to SPLIT_ENTRIES, if the sources' counts were
+    const int staged = STAGE && nls <= LS ? LE : 0;
     auto wide = [](unsigned c) { return ((unsigned long long)c << 32) | c; };
     for (int q = T.src_begin; q < T.src_end; ++q) {
       const SrcDesc Q = srcs[q];
+      auto count = [&](int l) {
+        return STAGE && l < LS ? s_cnt[l][tg] : lcnt[L.cnt_off + (int64_t)l * L.cap + i];
+      };
       int e = 0;
-      for (int l = 0; l < Q.lsrc; ++l) e += lcnt[L.cnt_off + (int64_t)l * L.cap + i];
-      const int eend = e + lcnt[L.cnt_off + (int64_t)Q.lsrc * L.cap + i];
+      for (int l = 0; l < Q.lsrc; ++l) e += count(l);
+      const int eend = e + count(Q.lsrc);
       if (e >= eend) continue;
       const int64_t poff = sd[Q.partner].off;
       SrcK<R> K;
@@ -1446,19 +1503,34 @@ __global__ void __launch_bounds__(64)
       unsigned long long m = 0ull;
       int base = 0, jn = 0;
       bool vn = false;
-      int2 mpre = emask[(int64_t)e * L.cap];
-      int bpre = ebase[(int64_t)e * L.cap];
+      unsigned long long mpre = 0ull;
+      int bpre = 0;
+      if (!STAGE) {
+        mpre = emask[(int64_t)e * L.cap];
+        bpre = ebase[(int64_t)e * L.cap];
+      }
       // the quad's next (up to four) partners: whether there are any, and
       // this lane's (jn, vn)
       auto next = [&]() -> bool {
         if (m == 0ull) {
           if (e >= eend) return false;
-          base = bpre;
-          m = ((unsigned long long)(unsigned)mpre.y << 32) | (unsigned)mpre.x;
-          ++e;
-          if (e < eend) {
-            mpre = emask[(int64_t)e * L.cap];
-            bpre = ebase[(int64_t)e * L.cap];
+          if constexpr (STAGE) {
+            if (e < staged) {
+              m = s_mask[e][tg];
+              base = s_base[e][tg];
+            } else {
+              m = emask[(int64_t)e * L.cap];
+              base = ebase[(int64_t)e * L.cap];
+            }
+            ++e;
+          } else {
+            base = bpre;
+            m = mpre;
+            ++e;
+            if (e < eend) {
+              mpre = emask[(int64_t)e * L.cap];
+              bpre = ebase[(int64_t)e * L.cap];
+            }
           }
         }
         unsigned long long w = m;
@@ -1489,8 +1561,9 @@ __global__ void __launch_bounds__(64)
         }
       };
       auto run = [&](auto dk) {
-        jn = bpre;  // a lane without a partner in the first round reads this one
+        // a lane without a partner in the first round reads the entry's base
         bool have = next();
+        if (!vn) jn = base;
         fetch();
         while (have) {
           const int64_t gj = poff + jn;
