@@ -1150,6 +1150,216 @@ __global__ void __launch_bounds__(64)
     lcnt[L.cnt_off + (int64_t)(L.src_end - L.src_begin) * L.cap + i] = ne > L.maxnb ? 1 : 0;
 }
 
+// k_nlist_split for launches smaller still (nlist_all_blocks): where the targets
+// of a wavefront share a cell column, and so the unions of their ranges are
+// short, all strips of a source are staged together, a memory latency or two
+// instead of one a strip.  It takes 221 registers in 3D, so a SIMD holds two
+// wavefronts.
+template <int D, typename R, int WIN>
+__global__ void __launch_bounds__(64)
+    k_nlist_small(Pool<R> P, const SysDesc *__restrict__ sd, const int *__restrict__ n_dev,
+                  const LTask *__restrict__ lt, const SrcDesc *__restrict__ srcs,
+                  const Grid *__restrict__ grids, const CellArr *__restrict__ carr,
+                  const int *__restrict__ cells, const Blk *__restrict__ blk, int nblk, int *lcnt,
+                  int *lidx, const long long *__restrict__ bbmin,
+                  const long long *__restrict__ bbmax, int span) {
+  constexpr int S_ = 4;
+  // one strip's window of candidates, or the short ones of all strips
+  constexpr int NST = (D == 3) ? 9 : 3;
+  constexpr int CAP = NST * 88 > WIN ? NST * 88 : WIN;
+  __shared__ float sf[D][CAP + 4];
+  const int lb = xcd_block(nblk * S_);
+  const Blk b = blk[lb / S_];
+  const LTask L = lt[b.item];
+  const int lane = threadIdx.x, sl = lane % S_;
+  const int i = b.first + (lb % S_) * (64 / S_) + lane / S_;
+  const SysDesc S = sd[L.sys];
+  const bool live = i < n_dev[L.sys];
+  if (__builtin_amdgcn_ballot_w64(live) == 0ull) return;
+  const int64_t gi = S.off + (live ? i : 0);
+  double xi[D];
+#pragma unroll
+  for (int d = 0; d < D; ++d) xi[d] = P.x[d][gi];
+  int2 *emask = reinterpret_cast<int2 *>(lidx + L.list_off) + i;
+  int *ebase = lidx + L.list_off + 2 * (int64_t)L.maxnb * L.cap + i;
+  double O[D];
+  Screen<D> scr;
+  screen_origin<D>(xi, O);
+  scr.set(xi, O);
+  int ne = 0;  // entries of this target
+  int cq = 0;  // entries of the current source
+  for (int q = L.src_begin; q < L.src_end; ++q) {
+    const SrcDesc Q = srcs[q];
+    const Grid G = grids[Q.grid];
+    cq = 0;
+    if (G.ncells > 0) {
+      const int *cs = cells + carr[Q.carr].off;
+      const int self_j = Q.pk == PK_SELF ? i : -1;
+      const double c2 = Q.cutoff2;
+      const int64_t poff = sd[Q.partner].off;
+      bool act = live && scr.finite;  // as in k_nlist
+      scr.source(c2, Q.cell);
+      if (Q.pk == PK_DYNAMIC && bbmin) {
+#pragma unroll
+        for (int d = 0; d < D; ++d) {
+          const double mn = double_of(bbmin[Q.partner * 3 + d]);
+          const double mx = double_of(bbmax[Q.partner * 3 + d]);
+          const double gap = mn - xi[d] > xi[d] - mx ? mn - xi[d] : xi[d] - mx;
+          act = act && !(gap > Q.cell * (1.0 + 1e-9));
+        }
+      }
+      int c[D];
+      target_cell<D>(xi, G, Q.cell, c);
+      if (__builtin_amdgcn_ballot_w64(act) != 0ull) {
+        // every strip's range up front: one latency instead of one a strip
+        int n0[NST], n1[NST];
+#pragma unroll
+        for (int st = 0; st < NST; ++st) {
+          n0[st] = n1[st] = 1;
+          if (act) {
+            const int sb = strip_base<D>(c, G, st);
+            n0[st] = cs[sb];
+            n1[st] = cs[sb + 3];
+          }
+        }
+        int base = 0;
+        unsigned lo = 0u, hi = 0u;
+        auto flush = [&]() {
+          lo = quad_or(lo);
+          hi = quad_or(hi);
+          const unsigned sdl = (unsigned)(self_j - base);
+          const unsigned sbit = 1u << (sdl & 31u);
+          lo &= sdl < 32u ? ~sbit : ~0u;
+          hi &= sdl - 32u < 32u ? ~sbit : ~0u;
+          if (live && (lo | hi) != 0u) {
+            if (ne < L.maxnb && sl == 0) {
+              emask[(int64_t)ne * L.cap] = make_int2((int)lo, (int)hi);
+              ebase[(int64_t)ne * L.cap] = base;
+            }
+            ++ne;
+            ++cq;
+          }
+          lo = hi = 0u;
+        };
+        // the target's candidates [js, je), staged from index js + o of sf on: the
+        // same for its S lanes, so they store a full mask together
+        auto walk = [&](int js, int je, int o, int64_t last) {
+          if (js >= base + 64) {
+            flush();
+            base += 64;
+          }
+          while (true) {
+            const int ce = je < base + 64 ? je : base + 64;
+            const int jb = js > base ? js : base;
+            // the four lanes take four candidates each in turn: lane sl those at
+            // 4·sl of every 16
+            const int n = ce - jb;
+            unsigned part[4];
+#pragma unroll
+            for (int m = 0; m < 4; ++m) {
+              const int t = 16 * m + 4 * sl;
+              unsigned sg = 0u;
+              if (t < n) {
+                if (screen4<D>(scr, sf, jb + o + t, sg) < 0.0f)
+                  sg = exact4<D>(P, xi, c2, poff + jb + t, last);
+                sg = __brev(sg) >> 28;
+              }
+              part[m] = sg << (4 * sl);
+            }
+            unsigned long long cur =
+                ((unsigned long long)(part[2] | part[3] << 16) << 32) | (part[0] | part[1] << 16);
+            cur = (cur & (~0ull >> (64 - n))) << (jb - base);
+            lo |= (unsigned)cur;
+            hi |= (unsigned)(cur >> 32);
+            if (base + 64 >= je) break;
+            flush();
+            base += 64;
+          }
+        };
+        // where the strips' unions of ranges are short (the targets of a wavefront
+        // in one cell column) all are staged together: a latency or two for the
+        // source instead of one a strip
+        int g0[NST], off[NST], tot = 0, most = 0;
+        unsigned g1[NST];  // lengths
+#pragma unroll
+        for (int st = 0; st < NST; ++st) {
+          const bool any = n0[st] < n1[st];
+          g0[st] = wave_red_dpp<false>(any ? n0[st] - 1 : INT_MAX);
+          const int e = wave_red_dpp<true>(any ? n1[st] - 1 : INT_MIN);
+          g1[st] = e > g0[st] ? (unsigned)(e - g0[st]) : 0u;  // 0: no range
+          off[st] = tot;
+          tot = g1[st] < (unsigned)CAP ? tot + (int)g1[st] : CAP + 1;
+          tot = tot < CAP ? tot : CAP + 1;
+          most = (int)g1[st] > most ? (int)g1[st] : most;
+        }
+        if (tot <= CAP && most <= 128) {
+          __syncthreads();  // the previous source's candidates have been read
+#pragma unroll
+          for (int h = 0; h < 128; h += 64) {
+            if (h >= most) break;
+            double x[NST][D];
+#pragma unroll
+            for (int st = 0; st < NST; ++st) {
+              const int t = h + lane < (int)g1[st] ? h + lane : 0;
+#pragma unroll
+              for (int k = 0; k < D; ++k)
+                x[st][k] = g1[st] != 0u ? P.x[k][poff + g0[st] + t] : 0.0;
+            }
+#pragma unroll
+            for (int st = 0; st < NST; ++st)
+              if (h + lane < (int)g1[st]) {
+#pragma unroll
+                for (int k = 0; k < D; ++k)
+                  sf[k][off[st] + h + lane] = scr.stage(x[st][k], O[k]);
+              }
+          }
+          __syncthreads();
+#pragma unroll
+          for (int st = 0; st < NST; ++st) {
+            if (g1[st] == 0u) continue;  // uniform
+            const int j0 = n0[st] - 1, j1 = n1[st] - 1;
+            base = j0;
+            if (j0 < j1) walk(j0, j1, off[st] - g0[st], poff + g0[st] + (int)g1[st] - 1);
+            flush();
+          }
+        } else {
+#pragma unroll
+          for (int st = 0; st < NST; ++st) {
+            const int j0 = n0[st] - 1, j1 = n1[st] - 1;
+            bool pend = j0 < j1;
+            if (__builtin_amdgcn_ballot_w64(pend) == 0ull) continue;
+            base = j0;
+            const int wmax = wave_red_dpp<true>(j1 - j0);
+            while (true) {
+              const int glo = wave_red_dpp<false>(pend ? j0 : INT_MAX);
+              if (glo == INT_MAX) break;
+              const bool mem = pend && j0 - glo <= span * wmax;
+              const int ghi = wave_red_dpp<true>(mem ? j1 : INT_MIN);
+              for (int w0 = glo; w0 < ghi; w0 += WIN) {
+                const int w1 = ghi - w0 < WIN ? ghi : w0 + WIN;
+                __syncthreads();  // the previous window has been read
+                for (int t = lane; t < w1 - w0; t += 64) {
+#pragma unroll
+                  for (int k = 0; k < D; ++k) sf[k][t] = scr.stage(P.x[k][poff + w0 + t], O[k]);
+                }
+                __syncthreads();
+                const int js = j0 > w0 ? j0 : w0;
+                const int je = mem ? (j1 < w1 ? j1 : w1) : 0;
+                if (js < je) walk(js, je, -w0, poff + w1 - 1);
+              }
+              if (mem) pend = false;
+            }
+            flush();
+          }
+        }
+      }
+    }
+    if (live && sl == 0) lcnt[L.cnt_off + (int64_t)(q - L.src_begin) * L.cap + i] = cq;
+  }
+  if (live && sl == 0)
+    lcnt[L.cnt_off + (int64_t)(L.src_end - L.src_begin) * L.cap + i] = ne > L.maxnb ? 1 : 0;
+}
+
 // Functors over the accepted partners of each target (one stage).
 template <int D, typename R, int FAM, bool CNT>
 __global__ void __launch_bounds__(GR_BLOCK)
@@ -1722,9 +1932,23 @@ template <int D>
 constexpr int nlist_split_blocks() {
   return D == 3 ? 1950 : 1200;
 }
+// Up to this many blocks the strips are staged together.  Measured, us strip by
+// strip / together: 2D dam breaks of 79 blocks 15.0 / 13.2, 640 16.2 / 14.0, 1155
+// 19.3 / 19.9; 3D of 125 41 / 38, 422 50 / 46, 615 48 / 53, 1000 52 / 65 (columns
+// of 500 blocks 40 / 34).
+template <int D>
+constexpr int nlist_all_blocks() {
+  return D == 3 ? 500 : 1000;
+}
 
 template <int D, typename R, int WIN>
 static void nlist_one(hipStream_t s, const Pool<R> &P, const NlistArgs &a) {
+  if (a.nblk <= nlist_all_blocks<D>()) {
+    k_nlist_small<D, R, WIN><<<a.nblk * 4, 64, 0, s>>>(P, a.sd, a.n, a.lt, a.srcs, a.grids, a.carr,
+                                                       a.cells, a.blk, a.nblk, a.lcnt, a.lidx,
+                                                       a.bbmin, a.bbmax, a.span);
+    return;
+  }
   if (a.nblk <= nlist_split_blocks<D>()) {
     k_nlist_split<D, R, WIN, 4><<<a.nblk * 4, 64, 0, s>>>(P, a.sd, a.n, a.lt, a.srcs, a.grids,
                                                           a.carr, a.cells, a.blk, a.nblk, a.lcnt,

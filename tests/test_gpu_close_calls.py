@@ -42,18 +42,20 @@ def _cloud(x, h, name):
 
 
 @pytest.mark.parametrize("prec", ["f32", "f64"])
-@pytest.mark.parametrize("lanes", [1, 4])
+# alone, or with a companion that takes the launch to each larger kernel (four
+# lanes per target strip by strip, one lane)
+@pytest.mark.parametrize("companion", [0, 1, 2])
 @pytest.mark.parametrize("D", [2, 3])
 @pytest.mark.parametrize("name", list(SCENES))
-def test_partner_counts(name, D, lanes, prec):
+def test_partner_counts(name, D, companion, prec):
     x, dx = SCENES[name](D)
     h = 1.5 * dx
     got = []
     for sc in (M.Session(D, prec).scene, oracle_scene(D)):
         ps, lf = _cloud(x, h, "a")
         lfs = [lf]
-        if lanes == 1 and not got:  # a companion large enough for the other kernel
-            n = 140000
+        if companion and not got:
+            n = (70000 if D == 2 else 60000) if companion == 1 else 140000
             y = np.random.default_rng(3).uniform(0.0, dx * n ** (1.0 / D), (n, D))
             lfs.append(_cloud(y, h, "b")[1])
         hs = [sc.integrator(f) for f in lfs]
