@@ -46,7 +46,7 @@ def parse():
     ap.add_argument("--start-step", type=int, default=300,
                     help="untimed steps of the dam break before tuning, warm-up and timing: "
                          "from rest no particle crosses a cell face and the sort skips its "
-                         "radix passes, which a flowing dam break does not")
+                         "placement, which a flowing dam break does not")
     ap.add_argument("--precision", default="f32", choices=["f32", "f64"])
     ap.add_argument("--cpu-steps", type=int, default=60,
                     help="timed oracle steps on the host (0 disables the CPU baseline)")
@@ -181,8 +181,8 @@ def sweep_bytes(cfg, grids):
 
 def sort_bytes(cfg, key_cells, precision):
     """Algorithmic bytes of the sort phase of one step: the key pass reads x
-    (8D) and writes a key (4), the ranking reads and writes a pool index (8),
-    the histogram and its scan touch 8 B per key cell, and the permutation
+    (8D) and writes a key (4), the placement reads and writes a pool index (8),
+    the counts and their scan touch 8 B per key cell, and the permutation
     reads and writes every per-particle array once (2·S_state: x 8D, v 8D,
     ρ 8, id 4, dvdt and drhodt in the state precision, p for fluids).  The
     leapfrog half step and stage 0's partner records are written by the same
@@ -417,9 +417,9 @@ def main():
                           "unit": "GB/s",
                           "frac": sort_gbs / HBM_PEAK_GBS if sort_gbs else None,
                           "algorithmic_bytes_per_step": bytes_sort, "phase_ms": phases[0],
-                          "kernels": "key min/max, key write (with the first pass's tile "
-                                     "counts), LSD radix (a scan and a scatter kernel per "
-                                     "8-bit digit), permutation of every per-particle array "
+                          "kernels": "key min/max, key count, starts of the cells, "
+                                     "placement in the cells (with the grids and the cleared "
+                                     "cell arrays), permutation of every per-particle array "
                                      "with the leapfrog half step and stage 0's partner "
                                      "records"},
         "cpu_baseline": cpu,
