@@ -1710,6 +1710,12 @@ __global__ void __launch_bounds__(64)
       const double da = (Q.pk == PK_DYNAMIC) ? Gp.da_of(Q) : 0.0;
       const bool nb = needs_b<FAM>(Q);
       const bool ns_a = CMP && needs_s<FAM>(Q), ns_b = ns_a && Gp.NS > 4;
+      // a functor without vorticity leaves those terms as the last source's
+      // pair left them
+      if constexpr (FAM == FAM_STRAIN) {
+#pragma unroll
+        for (int k = 0; k < 3; ++k) Gp.avo[k].t = (R)0;
+      }
       unsigned long long m = 0ull;
       int base = 0, jn = 0;
       bool vn = false;
