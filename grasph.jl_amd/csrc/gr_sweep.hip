@@ -744,17 +744,19 @@ __device__ inline int wave_red_dpp(int v) {
 // their difference by ua, so r errs by 2Σa·u(2X + 4c) <= u(24cX + 48c²), and by
 // 3u·12c² in the sums and uc² in c².  A candidate farther than 2c (of cells out
 // of the sort's order) has r >= 3/4 a² and an error of u(12aX + 22a²), too
-// small to change its sign while X <= 1e5 c; beyond that all are tested.
+// small to change its sign while X <= 1e5 c; beyond that all are tested, and
+// where c is so small or large that c² (or the tolerance's products) could
+// leave FP32's normal range (`all`).
 template <int D>
 struct Screen {
   float xf[D], c2, tol;
-  bool finite;
+  bool finite, all;
   __device__ inline void set(const double *xi, const double *O) {
     finite = true;
 #pragma unroll
     for (int d = 0; d < D; ++d) {
-      xf[d] = (float)(xi[d] - O[d]);
-      finite = finite && fabsf(xf[d]) < 3.0e38f;  // a non-finite target has no partner
+      xf[d] = stage(xi[d], O[d]);
+      finite = finite && fabs(xi[d]) <= 1.7976931348623157e308;  // else it has no partner
     }
   }
   __device__ inline void source(double cutoff2, double cell) {
@@ -765,8 +767,11 @@ struct Screen {
     c2 = (float)cutoff2;
     tol = 6.1e-8f * (c * (24.0f * X + 96.0f * c));
     if (!(X <= 1.0e5f * c) || !(cutoff2 <= cell * cell * (1.0 + 1e-9))) tol = __builtin_inff();
+    const unsigned e = (unsigned)((unsigned long long)__double_as_longlong(cell) >> 52);
+    all = e - (1023u - 40u) > 80u;  // (the exponent: scalar arithmetic)
   }
-  // a staged coordinate; a non-finite one is far from every target
+  // a staged coordinate; one beyond FP32's range (or not finite) is far from
+  // every target that is not tested in FP64 throughout
   static __device__ inline float stage(double x, double o) {
     const float f = (float)(x - o);
     return fabsf(f) < 3.0e38f ? f : 3.0e38f;
@@ -953,6 +958,7 @@ __global__ void __launch_bounds__(64)
               for (int t = t0; t < t0 + n; t += 4)
                 nr = __builtin_amdgcn_alignbit(
                     nr, __float_as_uint(screen4<D>(scr, sf, t, cur)), 31);
+              if (scr.all) nr = (1u << ng) - 1u;
               while (nr != 0u) {
                 const int g = __builtin_ctz(nr);
                 nr &= nr - 1u;
@@ -1120,7 +1126,7 @@ __global__ void __launch_bounds__(64)
                     const int o = 16 * m + 4 * sl;
                     unsigned sg = 0u;
                     if (o < n) {
-                      if (screen4<D>(scr, sf, jb - w0 + o, sg) < 0.0f)
+                      if (screen4<D>(scr, sf, jb - w0 + o, sg) < 0.0f || scr.all)
                         sg = exact4<D>(P, xi, c2, poff + jb + o, poff + w1 - 1);
                       sg = __brev(sg) >> 28;
                     }
@@ -1260,7 +1266,7 @@ __global__ void __launch_bounds__(64)
               const int t = 16 * m + 4 * sl;
               unsigned sg = 0u;
               if (t < n) {
-                if (screen4<D>(scr, sf, jb + o + t, sg) < 0.0f)
+                if (screen4<D>(scr, sf, jb + o + t, sg) < 0.0f || scr.all)
                   sg = exact4<D>(P, xi, c2, poff + jb + t, last);
                 sg = __brev(sg) >> 28;
               }
