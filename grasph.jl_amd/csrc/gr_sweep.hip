@@ -1688,7 +1688,14 @@ __global__ void __launch_bounds__(64)
   if (STAGE) __syncthreads();
   using TT = Terms<D, R, FAM>;
   double sum[TT::NG] = {};
-  if (live && !overflow) {
+  // OV: targets without a list (it overflowed, or there is none): the quad tests
+  // the candidates of the cell walk itself, 16 of every 64 a lane, and takes the
+  // partners of those as an entry's.  Sweep where every list overflows, with one
+  // lane of the four walking alone / with the quad / with one lane per target (us,
+  // 3D dam break functor in FP32, 400 particles a cell): 27k targets 4040 / 950 /
+  // 4410, 110k 9010 / 2500 / 4510.
+  auto sources = [&](auto ovc) {
+    constexpr bool OV = decltype(ovc)::value;
     Gather<D, R, FAM, Term<R>> Gp;
     Gp.load(P, S, T, gi);
     constexpr bool CMP = Gather<D, R, FAM>::COMPACT;
@@ -1706,10 +1713,12 @@ __global__ void __launch_bounds__(64)
       auto count = [&](int l) {
         return STAGE && l < LS ? s_cnt[l][tg] : lcnt[L.cnt_off + (int64_t)l * L.cap + i];
       };
-      int e = 0;
-      for (int l = 0; l < Q.lsrc; ++l) e += count(l);
-      const int eend = e + count(Q.lsrc);
-      if (e >= eend) continue;
+      int e = 0, eend = 0;
+      if constexpr (!OV) {
+        for (int l = 0; l < Q.lsrc; ++l) e += count(l);
+        eend = e + count(Q.lsrc);
+        if (e >= eend) continue;
+      }
       const int64_t poff = sd[Q.partner].off;
       SrcK<R> K;
       K.load(Q);
@@ -1727,15 +1736,50 @@ __global__ void __launch_bounds__(64)
       bool vn = false;
       unsigned long long mpre = 0ull;
       int bpre = 0;
-      if (!STAGE) {
+      if (!STAGE && !OV) {
         mpre = emask[(int64_t)e * L.cap];
         bpre = ebase[(int64_t)e * L.cap];
       }
+      // OV: the mask of the 64 candidates from `base` on, below `wend`
+      auto test = [&](int wend) {
+        const int self_j = Q.pk == PK_SELF ? i : -1;
+        unsigned h[2] = {0u, 0u};
+#pragma unroll
+        for (int w = 0; w < 2; ++w) {
+#pragma unroll 1
+          for (int b4 = 0; b4 < 32; b4 += 16) {
+            // four loads in flight; beyond the range's end its last one again
+            double r2[4];
+#pragma unroll
+            for (int d = 0; d < D; ++d) {
+              double xj[4];
+#pragma unroll
+              for (int u = 0; u < 4; ++u) {
+                const int j = base + 32 * w + b4 + 4 * u + sl;
+                xj[u] = P.x[d][poff + (j < wend ? j : wend - 1)];
+              }
+#pragma unroll
+              for (int u = 0; u < 4; ++u) {
+                const double dx = Gp.xi[d] - xj[u];
+                r2[u] = d == 0 ? dx * dx : r2[u] + dx * dx;
+              }
+            }
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+              const int j = base + 32 * w + b4 + 4 * u + sl;
+              h[w] |= (unsigned)(r2[u] < Q.cutoff2 && j < wend && j != self_j)
+                      << (b4 + 4 * u + sl);
+            }
+          }
+          h[w] = quad_or(h[w]);
+        }
+        m = ((unsigned long long)h[1] << 32) | h[0];
+      };
       // the quad's next (up to four) partners: whether there are any, and
       // this lane's (jn, vn)
       auto next = [&]() -> bool {
         if (m == 0ull) {
-          if (e >= eend) return false;
+          if (OV || e >= eend) return false;
           if constexpr (STAGE) {
             if (e < staged) {
               m = s_mask[e][tg];
@@ -1830,12 +1874,32 @@ __global__ void __launch_bounds__(64)
           }
         }
       };
-      if (Q.pk == PK_DYNAMIC)
+      if constexpr (OV) {
+        // (the quads of a wavefront test in step, then take their partners)
+        const Grid G = grids[Q.grid];
+        if (G.ncells <= 0) continue;
+        const int *cs = cells + carr[Q.carr].off;
+        int c[D];
+        target_cell<D>(Gp.xi, G, Q.cell, c);
+        for (int st = 0; st < (D == 3 ? 9 : 3); ++st) {
+          const int sb = strip_base<D>(c, G, st);
+          const int wend = cs[sb + 3] - 1;
+          for (base = cs[sb] - 1; base < wend; base += 64) {
+            test(wend);
+            if (m != 0ull) run(std::integral_constant<int, -1>{});
+          }
+        }
+      } else if (Q.pk == PK_DYNAMIC) {
         run(std::integral_constant<int, 1>{});
-      else
+      } else {
         run(std::integral_constant<int, 0>{});
+      }
     }
-  }
+  };
+  if (overflow)
+    sources(std::true_type{});
+  else if (live)
+    sources(std::false_type{});
   // every lane of the quad takes all its components
   double tot[TT::NG * 4];
 #pragma unroll
@@ -1846,8 +1910,6 @@ __global__ void __launch_bounds__(64)
     tot[4 * g + 3] = quad_mov<0xFF>(sum[g]);
   }
   TT::set(Gt, tot);
-  if (overflow && sl == 0)
-    gather_direct<D, R, FAM>(Gt, P, sd, T, srcs, grids, carr, cells, i, ns, no);
   count_pairs<CNT>(pair_count, ns, no);
   if (live && sl == 0) Gt.store(P, S, T, gi);
 }
