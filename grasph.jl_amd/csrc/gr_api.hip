@@ -431,7 +431,7 @@ struct gr_ctx {
   int64_t cells_cap = 0;
   std::vector<StepSys> stepsys;
   // sort / scan scratch
-  DBuf keys, vals, keys2, vals2, krank, hist, cand, cand_scan, scan_bsum;
+  DBuf keys, vals, keys2, vals2, krank, krun, hist, cand, cand_scan, scan_bsum;
   DBuf ktable;          // the counting sort's table (key_table_bytes)
   int ktable_tiles = 0;
   int64_t sort_cap = 0, cand_cap = 0;
@@ -734,6 +734,7 @@ void commit(gr_ctx *c) {
     c->keys2.alloc(sc * 4);
     c->vals2.alloc(sc * 4);
     c->krank.alloc(sc * 4);
+    c->krun.alloc(sc * 4);
     // the radix sort's tile counts start at zero (each sort leaves them so)
     c->hist.alloc(radix_scratch_bytes((int)sc));
     HIPCHK(hipMemsetAsync(c->hist.p, 0, c->hist.bytes, c->stream));
@@ -1147,15 +1148,15 @@ constexpr int kGrowMargin = 8;
 // wider than their bounds on every side; 0 beyond kMaxKeyTiles (8M keys, 68 MB
 // of table, whose scan would cost as much as the radix passes).  A ghost
 // system's bounds are its source's, widened by twice its cutoff (a mirror
-// moves a particle by at most that).  Also 0 where a system's cells hold more
-// than kKeyCellMean particles on average: the rank within the cell grows with
-// them (sort of 200k particles in motion, 3D: table 49 us at 32 a cell, 68 at
-// 128, 83 at 256, 105 at 512, radix kernels 74 to 87; 20k in 2D: 31, 35, 39,
-// 49 against 49 to 58).
+// moves a particle by at most that).  Also 0 where the particles times the mean
+// number in a cell of their system exceed kKeyRank: the rank within the cell
+// grows with them (sort of particles in motion, us, table / radix kernels, 2D:
+// 1M at 32 a cell 92 / 111, at 128 149 / 111; 200k at 128 57 / 80, at 200 73 / 75,
+// at 1024 76 / 75; 20k at 1024 33 / 51, at 4096 54 / 49).
 constexpr int kMaxKeyTiles = 8192;
-constexpr double kKeyCellMean = 256.0;
+constexpr double kKeyRank = 3.2e7;
 int key_tiles(gr_ctx *c, const std::vector<int> &systems, const HostBounds &h, int margin) {
-  double keys = 1.0;
+  double keys = 1.0, rank = 0.0;
   for (int s : systems) {
     const SysH &S = c->sys[s];
     const bool ghost = S.kind == GR_SYS_GHOST;
@@ -1169,8 +1170,9 @@ int key_tiles(gr_ctx *c, const std::vector<int> &systems, const HostBounds &h, i
     }
     keys += r;
     if (!(keys < 1e12)) return 0;
-    if (!ghost && (double)S.n > kKeyCellMean * cells) return 0;
+    if (!ghost) rank += (double)S.n * (double)S.n / cells;
   }
+  if (rank > kKeyRank) return 0;
   const double t = std::floor(keys / key_table_tile()) + 1.0;
   return t <= kMaxKeyTiles ? (int)t : 0;
 }
@@ -1872,8 +1874,8 @@ void key_sort(gr_ctx *c, const Plan &P, const XP &xs, const DBuf &blk, int nblk,
                   c->d_kmin.as<int>(), c->d_kmax.as<int>(), c->d_krange.as<unsigned>(),
                   c->d_kbase.as<unsigned>(), c->keys.as<unsigned>(), c->vals.as<int>(),
                   c->keys2.as<unsigned>(), c->vals2.as<int>(), c->krank.as<unsigned>(),
-                  c->d_flags.as<int>(), c->d_sysfault.as<int>(), c->ktable.as<unsigned>(),
-                  c->ktable_tiles, tiles, cells ? &A : nullptr);
+                  c->d_flags.as<int>(), c->d_sysfault.as<int>(), c->krun.as<int>(),
+                  c->ktable.as<unsigned>(), c->ktable_tiles, tiles, cells ? &A : nullptr);
 }
 
 // half: also take the leapfrog half step of the plan's integrated systems
@@ -1892,7 +1894,7 @@ void phase_sort_real(gr_ctx *c, Plan &P, bool half = false, int pack = 0) {
     all_real(c, arb, arn);
     const KeyTable kt =
         key_table_view(c->ktable.as<unsigned>(), c->ktable_tiles, P.tiles_real, c->keys2.as<unsigned>(),
-                       c->d_krange.as<unsigned>(), c->d_kbase.as<unsigned>(),
+                       c->krun.as<int>(), c->d_krange.as<unsigned>(), c->d_kbase.as<unsigned>(),
                        P.d_real_list.as<int>(), (int)P.real_list.size());
     Pool<R> A = pool_view<R>(c, c->cur), B = pool_view<R>(c, 1 - c->cur);
     launch_permute_real<R>(s, A, B, c->d_sd.as<SysDesc>(), arb, arn, P.d_bbase_real.as<int>(),
@@ -1954,7 +1956,7 @@ void phase_ghosts(gr_ctx *c, Plan &P, bool generate, bool sort) {
              (int)P.ghost_list.size(), P.n_ghost, P.tiles_ghost, sort_preps_cells(P, true));
     const KeyTable kt =
         key_table_view(c->ktable.as<unsigned>(), c->ktable_tiles, P.tiles_ghost, c->keys2.as<unsigned>(),
-                       c->d_krange.as<unsigned>(), c->d_kbase.as<unsigned>(),
+                       c->krun.as<int>(), c->d_krange.as<unsigned>(), c->d_kbase.as<unsigned>(),
                        P.d_ghost_list.as<int>(), (int)P.ghost_list.size());
     launch_permute_ghost(s, gx, c->gidx_s.as<int>(), c->gbnd_s.as<int>(), xpw_pool(c, c->cur),
                          A.gidx, A.gbnd, c->d_sd.as<SysDesc>(), c->d_n.as<int>(),

@@ -717,7 +717,8 @@ __global__ void __launch_bounds__(GR_BLOCK) k_cells_prep(CellsArgs A, int *flags
 // the counts into the cells' starts, k_key_place puts every particle into its
 // cell, and the permutations order each cell by the particles' former places
 // (the sort is stable): a particle's rank is the number of smaller former
-// places in its cell, which holds a handful.  Against the radix sort's scan
+// places in its cell, which holds a handful (of more than KT_BIG, the runs of
+// former neighbours are counted instead, key_slot).  Against the radix sort's scan
 // and scatter kernel per 8-bit digit (each 3 to 16 us, four of each launched
 // whatever the key range) it takes two kernels.  Sort phase, radix before:
 // 3D dam break of 1.4M particles 158 -> 140 us, 2D dam break of 23k 50 -> 30,
@@ -735,6 +736,14 @@ __global__ void __launch_bounds__(GR_BLOCK) k_cells_prep(CellsArgs A, int *flags
 
 #define KT_TILE 1024  // keys per workgroup of the scan
 #define KT_RANKS 8    // former places compared at a time in the rank within a cell
+// Largest cell whose particles are compared one by one.  Beyond it the runs of
+// equal keys along a wavefront, which the atomics of k_key_count place as one,
+// are: their former places are consecutive.  Sort of a step (us), one by one /
+// runs / radix kernels, 20k particles at 300 a cell 33 / 27 / 48, at 1024
+// 60 / 33 / 51, all in one cell 655 / 108 / 48; 200k at 300 81 / 75 / 76, at
+// 2048 181 / 87 / 66, in one cell 11500 / 1120 / 50.  (60k particles in one cell
+// that interact with each other: 0.3 ms of a step's 14.5.)
+#define KT_BIG 256
 // Copies of each tile's sum: k_key_count's atomics are spread over them (a tile
 // takes one from each of some 100 wavefronts; with one copy the kernel took
 // 154 us instead of 40 in the 3D dam break of 1.4M particles).
@@ -963,7 +972,7 @@ __global__ void __launch_bounds__(GR_BLOCK)
                 int *vals, unsigned *keys2, int *vals2, const unsigned *rank,
                 const unsigned *start, unsigned *tsum, int ntile, int N, const int *list,
                 int nlist, long long *bbmin, long long *bbmax, int rs, int *flags,
-                unsigned cap, int nprep, CellsArgs A, int *sysfault) {
+                unsigned cap, int nprep, CellsArgs A, int *sysfault, int *run) {
   if ((int)blockIdx.x < nprep) {
     cells_prep(A, (int)blockIdx.x, flags, sysfault);
     return;
@@ -989,7 +998,14 @@ __global__ void __launch_bounds__(GR_BLOCK)
   if (i >= n_dev[s]) return;
   const int p = bbase[s] + i;
   const unsigned key = keys[p];
-  const unsigned slot = start[key] + rank[p];
+  const unsigned first = start[key];
+  const unsigned slot = first + rank[p];
+  const bool big = start[key + 1] - first > KT_BIG;
+  if (__ballot(big) != 0ull) {  // the lengths of the runs, at their first slots
+    int len;
+    const int head = run_head(key, true, len);
+    if (big && head == (int)(threadIdx.x & 63) && slot < (unsigned)N) run[slot] = len;
+  }
   // the counts place every particle below N; a slot beyond it is reported,
   // never written
   if (slot >= (unsigned)N) {
@@ -1004,13 +1020,23 @@ __global__ void __launch_bounds__(GR_BLOCK)
 // the slot its rank in the cell gives it.
 __device__ __forceinline__ int key_slot(int p, const int *vals, const unsigned *keys2,
                                         const int *vals2, const unsigned *start, const int *flags,
-                                        unsigned cap, int &slot) {
+                                        unsigned cap, const int *run, int &slot) {
   slot = p;
   if ((unsigned)flags[2] > cap) return vals[p];
   const int v = vals2[p];
   const unsigned k = keys2[p];
   const int a = (int)start[k], e = (int)start[k + 1];
   int r = 0;
+  if (e - a > KT_BIG) {
+    for (int j = a; j < e;) {
+      const int u = vals2[j], len = run[j] > 1 ? run[j] : 1;
+      const int below = v - u;  // of the run's consecutive places
+      r += below > 0 ? (below < len ? below : len) : 0;
+      j += len;
+    }
+    slot = a + r;
+    return v;
+  }
   for (int j = a; j < e; j += KT_RANKS) {
     int u[KT_RANKS];
 #pragma unroll
@@ -1051,7 +1077,7 @@ __global__ void k_permute_real(Pool<R> A, Pool<R> B, const SysDesc *sd, const Bl
   if constexpr (TAB) {
     if (flags[0] != 0 && bbase[s] >= 0 && kt.krange[s * 3] != 0u) {  // not a faulted system
       int slot;
-      src = key_slot(bbase[s] + i, vals, kt.keys2, vals2, kt.start, flags, kt.cap, slot);
+      src = key_slot(bbase[s] + i, vals, kt.keys2, vals2, kt.start, flags, kt.cap, kt.run, slot);
       dst = S.off + (slot - bbase[s]);
     }
   } else {
@@ -1312,7 +1338,7 @@ __global__ void k_permute_ghost(XP gxs, const int *gidx_s, const int *gbnd_s, XP
         p0 = (int)kt.start[kt.kbase[g]];
       }
       int slot;
-      src = key_slot(p0 + k, vals, kt.keys2, vals2, kt.start, flags, kt.cap, slot);
+      src = key_slot(p0 + k, vals, kt.keys2, vals2, kt.start, flags, kt.cap, kt.run, slot);
       dst = G.off + (slot - p0);
     }
   } else {
@@ -2400,7 +2426,7 @@ void launch_key_sort(hipStream_t s, XP xs, const SysDesc *sd, const int *n, cons
                      int N, long long *bbmin, long long *bbmax, int rs, int *kmin, int *kmax,
                      unsigned *krange, unsigned *kbase, unsigned *keys, int *vals,
                      unsigned *keys2, int *vals2, unsigned *rank, int *flags, int *sysfault,
-                     unsigned *table, int tiles, int ntile, const CellsArgs *cells) {
+                     int *run, unsigned *table, int tiles, int ntile, const CellsArgs *cells) {
   if (nblk <= 0) {
     if (cells) launch_cells_prep(s, *cells, flags, sysfault);
     return;
@@ -2425,13 +2451,14 @@ void launch_key_sort(hipStream_t s, XP xs, const SysDesc *sd, const int *n, cons
   const int nprep = cells_prep_blocks(A);
   k_key_place<<<nblk + nprep, GR_BLOCK, 0, s>>>(
       sd, n, blk, bbase, keys, vals, keys2, vals2, rank, start, tsum, ntile, N, list, nlist, bbmin,
-      bbmax, rs, flags, cap, nprep, A, sysfault);
+      bbmax, rs, flags, cap, nprep, A, sysfault, run);
 }
 KeyTable key_table_view(unsigned *table, int tiles, int ntile, const unsigned *keys2,
-                        const unsigned *krange, const unsigned *kbase, const int *list,
+                        const int *run, const unsigned *krange, const unsigned *kbase, const int *list,
                         int nlist) {
   KeyTable kt;
   kt.keys2 = keys2;
+  kt.run = run;
   kt.start = table + (size_t)tiles * KT_TILE;
   kt.krange = krange;
   kt.kbase = kbase;

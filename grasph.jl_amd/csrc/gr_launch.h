@@ -107,15 +107,17 @@ void launch_key_sort(hipStream_t s, XP xs, const SysDesc *sd, const int *n, cons
                      int N, long long *bbmin, long long *bbmax, int rs, int *kmin, int *kmax,
                      unsigned *krange, unsigned *kbase, unsigned *keys, int *vals,
                      unsigned *keys2, int *vals2, unsigned *rank, int *flags, int *sysfault,
-                     unsigned *table, int tiles, int ntile, const CellsArgs *cells = nullptr);
+                     int *run, unsigned *table, int tiles, int ntile,
+                     const CellsArgs *cells = nullptr);
 struct KeyTable {  // what the permutations read of the counting sort
   const unsigned *keys2, *start, *krange, *kbase;
+  const int *run;  // at the first slot of a run in a large cell: its length
   const int *list;
   int nlist;
   unsigned cap;
 };
 KeyTable key_table_view(unsigned *table, int tiles, int ntile, const unsigned *keys2,
-                        const unsigned *krange, const unsigned *kbase, const int *list,
+                        const int *run, const unsigned *krange, const unsigned *kbase, const int *list,
                         int nlist);
 template <typename R>
 void launch_permute_real(hipStream_t s, const Pool<R> &A, const Pool<R> &B, const SysDesc *sd,
