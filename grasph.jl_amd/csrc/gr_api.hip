@@ -318,8 +318,12 @@ struct Plan {
   DBuf d_real_list, d_bbase_real, blk_real;
   int nblk_real = 0, n_real = 0;
   // tiles of the counting sort's table for the real and the ghost systems (0:
-  // more keys than a table is kept for, the step sorts by radix)
+  // more keys than a table is kept for, the step sorts by radix), and each
+  // system's budget of its entries
   int tiles_real = 0, tiles_ghost = 0;
+  std::vector<unsigned> budget_real, budget_ghost;
+  DBuf d_budget_real, d_budget_ghost;
+  unsigned long long x_epoch = 0;  // the context's, when the budgets were last checked
   // ghosts
   std::vector<int> ghost_list;
   // ghost generation: blocks of source particles per ghost system, and the
@@ -423,15 +427,17 @@ struct gr_ctx {
   bool vadj_any = false;  // some v_adjustment may be nonzero: permute and correct it
   // tables
   DBuf d_sd, d_n, d_st, d_bnd, d_kmin, d_kmax, d_bbmin, d_bbmax, d_kbase, d_krange, d_flags;
+  DBuf d_kshift;
   DBuf d_sysfault;  // per system: GR_FAULT_* bits raised by the step's kernels
   int bb_rs = 0;  // entries per replica of d_bbmin / d_bbmax (GR_BB_REP + 1 replicas)
+  unsigned long long x_epoch = 0;  // uploads of real systems' positions
   bool bb_valid = false;  // d_bbmin / d_bbmax hold the bounds of a step's key pass
   DBuf d_grids, d_carr, d_cellsz, d_inter_sys, d_inter_carr, cells, ctile;
   std::vector<CellArr> carr;
   int64_t cells_cap = 0;
   std::vector<StepSys> stepsys;
   // sort / scan scratch
-  DBuf keys, vals, keys2, vals2, krank, krun, hist, cand, cand_scan, scan_bsum;
+  DBuf keys, vals, keys2, vals2, krank, krun, kfull, hist, cand, cand_scan, scan_bsum;
   DBuf ktable;          // the counting sort's table (key_table_bytes)
   int ktable_tiles = 0;
   int64_t sort_cap = 0, cand_cap = 0;
@@ -707,6 +713,7 @@ void commit(gr_ctx *c) {
   std::vector<unsigned> zu(ns * 3, 0);
   c->d_kbase.upload(zu, c->stream);
   c->d_krange.upload(zu, c->stream);
+  c->d_kshift.upload(z, c->stream);
   c->d_sysfault.upload(std::vector<int>(std::max(ns, 1), 0), c->stream);
   if (!c->d_flags.p) {
     std::vector<int> f(4, 0);
@@ -735,6 +742,7 @@ void commit(gr_ctx *c) {
     c->vals2.alloc(sc * 4);
     c->krank.alloc(sc * 4);
     c->krun.alloc(sc * 4);
+    c->kfull.alloc(sc * 4);
     // the radix sort's tile counts start at zero (each sort leaves them so)
     c->hist.alloc(radix_scratch_bytes((int)sc));
     HIPCHK(hipMemsetAsync(c->hist.p, 0, c->hist.bytes, c->stream));
@@ -1092,14 +1100,22 @@ struct HostBounds {
   double hi(int s, int d) const { return dbl(mx[(size_t)s * 3 + d]); }
 };
 
-// Read back the folded bounds (replica 0 of d_bbmin / d_bbmax).
-void read_bounds(gr_ctx *c, HostBounds &h) {
-  const size_t n = c->sys.size() * 3;
-  h.mn.resize(n);
-  h.mx.resize(n);
-  HIPCHK(hipMemcpyAsync(h.mn.data(), c->d_bbmin.p, n * 8, hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(hipMemcpyAsync(h.mx.data(), c->d_bbmax.p, n * 8, hipMemcpyDeviceToHost, c->stream));
+// Read back the bounds: the folded ones (replica 0 of d_bbmin / d_bbmax), and in
+// `now` those a bounds pass has left in the other replicas.
+void read_bounds(gr_ctx *c, HostBounds &h, HostBounds *now = nullptr) {
+  const size_t n = c->sys.size() * 3, m = now ? n * (GR_BB_REP + 1) : n;
+  h.mn.resize(m);
+  h.mx.resize(m);
+  HIPCHK(hipMemcpyAsync(h.mn.data(), c->d_bbmin.p, m * 8, hipMemcpyDeviceToHost, c->stream));
+  HIPCHK(hipMemcpyAsync(h.mx.data(), c->d_bbmax.p, m * 8, hipMemcpyDeviceToHost, c->stream));
   HIPCHK(hipStreamSynchronize(c->stream));
+  if (!now) return;
+  now->mn.assign(n, LLONG_MAX);
+  now->mx.assign(n, LLONG_MIN);
+  for (size_t e = n; e < m; ++e) {
+    now->mn[e % n] = std::min(now->mn[e % n], h.mn[e]);
+    now->mx[e % n] = std::max(now->mx[e % n], h.mx[e]);
+  }
 }
 
 // Bounds of the given real systems (device reduction, host readback).
@@ -1144,18 +1160,21 @@ void host_bbox(gr_ctx *c, const std::vector<int> &systems, std::vector<double> &
 constexpr int kGrowChunk = 16;
 constexpr int kGrowMargin = 8;
 
-// Tiles of a counting table for the listed systems' cell keys, `margin` cells
-// wider than their bounds on every side; 0 beyond kMaxKeyTiles (8M keys, 68 MB
+// Tiles of a counting table for the listed systems' cell keys (`budget`: of each),
+// `margin` cells wider than their bounds on every side; 0 beyond kMaxKeyTiles (8M keys, 68 MB
 // of table, whose scan would cost as much as the radix passes).  A ghost
 // system's bounds are its source's, widened by twice its cutoff (a mirror
 // moves a particle by at most that).  Also 0 where the particles times the mean
 // number in a cell of their system exceed kKeyRank: the rank within the cell
 // grows with them (sort of particles in motion, us, table / radix kernels, 2D:
 // 1M at 32 a cell 92 / 111, at 128 149 / 111; 200k at 128 57 / 80, at 200 73 / 75,
-// at 1024 76 / 75; 20k at 1024 33 / 51, at 4096 54 / 49).
+// at 1024 76 / 75; 20k at 1024 33 / 51, at 4096 54 / 49).  `slack`: the limits are
+// so much higher for a table in use.
 constexpr int kMaxKeyTiles = 8192;
 constexpr double kKeyRank = 3.2e7;
-int key_tiles(gr_ctx *c, const std::vector<int> &systems, const HostBounds &h, int margin) {
+int key_tiles(gr_ctx *c, const std::vector<int> &systems, const HostBounds &h, int margin,
+              std::vector<unsigned> &budget, double slack = 1.0) {
+  budget.clear();
   double keys = 1.0, rank = 0.0;
   for (int s : systems) {
     const SysH &S = c->sys[s];
@@ -1169,12 +1188,13 @@ int key_tiles(gr_ctx *c, const std::vector<int> &systems, const HostBounds &h, i
       cells *= std::floor(ext / cut) + 1.0;
     }
     keys += r;
-    if (!(keys < 1e12)) return 0;
+    if (!(keys < 1e9)) return 0;
+    budget.push_back((unsigned)r);
     if (!ghost) rank += (double)S.n * (double)S.n / cells;
   }
-  if (rank > kKeyRank) return 0;
+  if (rank > slack * kKeyRank) return 0;
   const double t = std::floor(keys / key_table_tile()) + 1.0;
-  return t <= kMaxKeyTiles ? (int)t : 0;
+  return t <= slack * kMaxKeyTiles ? (int)t : 0;
 }
 
 // Destroy every captured step graph (device tables or pools they point to
@@ -1350,6 +1370,20 @@ void plan_ghosts(gr_ctx *c, Plan &P, const std::vector<int> &ghosts) {
   // up to 8192 slots a system, every workgroup that holds ghosts adds up the
   // slots before its own (32 loads a thread) instead of three scan kernels
   for (int g : ghosts) P.gslot_scan = P.gslot_scan || ghost_slots(c, c->sys[g]) > 8192;
+}
+
+// The bounds of a plan's real systems into replicas 1 .. of d_bbmin / d_bbmax.
+void step_minmax(gr_ctx *c, const Plan &P) {
+  launch_key_minmax(c->stream, xp_pool(c, c->cur), c->d_sd.as<SysDesc>(), c->d_n.as<int>(),
+                    P.blk_real.as<Blk>(), P.nblk_real, c->D, c->d_bbmin.as<long long>(),
+                    c->d_bbmax.as<long long>(), c->bb_rs, P.d_real_list.as<int>(),
+                    (int)P.real_list.size(), false, c->d_flags.as<int>());
+}
+void reset_replicas(gr_ctx *c, const Plan &P) {
+  launch_minmax_reset(c->stream, P.d_real_list.as<int>(), (int)P.real_list.size(),
+                      c->d_bbmin.as<long long>(), c->d_bbmax.as<long long>(), c->bb_rs);
+  launch_minmax_reset(c->stream, P.d_ghost_list.as<int>(), (int)P.ghost_list.size(),
+                      c->d_bbmin.as<long long>(), c->d_bbmax.as<long long>(), c->bb_rs);
 }
 
 // Stage plans of a batch of integrators: updater tables (with the fused EOS
@@ -1778,10 +1812,16 @@ Plan &get_plan(gr_ctx *c, const std::vector<int> &integs) {
   c->carr_used = nullptr;
   plan_grids(c, *P, inters, &used);
   if (!reals.empty()) {  // key tables with room for a few chunks of steps
-    HostBounds hb;
-    host_bounds(c, reals, hb);
-    P->tiles_real = key_tiles(c, reals, hb, kGrowMargin + 4);
-    P->tiles_ghost = ghosts.empty() ? 0 : key_tiles(c, ghosts, hb, kGrowMargin + 4);
+    HostBounds hb, now;
+    reset_replicas(c, *P);
+    step_minmax(c, *P);
+    read_bounds(c, hb, &now);
+    P->tiles_real = key_tiles(c, reals, now, kGrowMargin + 4, P->budget_real);
+    P->tiles_ghost =
+        ghosts.empty() ? 0 : key_tiles(c, ghosts, now, kGrowMargin + 4, P->budget_ghost);
+    if (P->tiles_real > 0) P->d_budget_real.upload(P->budget_real, c->stream);
+    if (P->tiles_ghost > 0) P->d_budget_ghost.upload(P->budget_ghost, c->stream);
+    P->x_epoch = c->x_epoch;
     const int t = std::max(P->tiles_real, P->tiles_ghost);
     if (t > c->ktable_tiles) {
       c->ktable.alloc(key_table_bytes(t));
@@ -1849,13 +1889,6 @@ constexpr int kBoundsBlocks = 1024;
 bool step_bounds(const Plan &P) {
   return P.tiles_real > 0 && !P.vadj_live && P.nblk_virt == 0 && P.nblk_int <= kBoundsBlocks;
 }
-// The bounds of the real systems for the counting sort, into reset replicas.
-void step_minmax(gr_ctx *c, const Plan &P) {
-  launch_key_minmax(c->stream, xp_pool(c, c->cur), c->d_sd.as<SysDesc>(), c->d_n.as<int>(),
-                    P.blk_real.as<Blk>(), P.nblk_real, c->D, c->d_bbmin.as<long long>(),
-                    c->d_bbmax.as<long long>(), c->bb_rs, P.d_real_list.as<int>(),
-                    (int)P.real_list.size(), false, c->d_flags.as<int>());
-}
 
 // Whether the real or ghost sort of a step prepares its cells: the last one,
 // where it is a counting sort.
@@ -1866,16 +1899,28 @@ bool sort_preps_cells(const Plan &P, bool ghost) {
 
 // The counting sort of a step's real or ghost systems (after their bounds).
 void key_sort(gr_ctx *c, const Plan &P, const XP &xs, const DBuf &blk, int nblk, const DBuf &bbase,
-              const DBuf &list, int nlist, int n, int tiles, bool cells) {
+              const DBuf &list, int nlist, int n, int tiles, const DBuf &budget, bool cells) {
   const CellsArgs A = cells_args(c, P);
   launch_key_sort(c->stream, xs, c->d_sd.as<SysDesc>(), c->d_n.as<int>(), c->d_st.as<StepSys>(),
                   blk.as<Blk>(), nblk, bbase.as<int>(), c->D, list.as<int>(), nlist, n,
                   c->d_bbmin.as<long long>(), c->d_bbmax.as<long long>(), c->bb_rs,
                   c->d_kmin.as<int>(), c->d_kmax.as<int>(), c->d_krange.as<unsigned>(),
-                  c->d_kbase.as<unsigned>(), c->keys.as<unsigned>(), c->vals.as<int>(),
-                  c->keys2.as<unsigned>(), c->vals2.as<int>(), c->krank.as<unsigned>(),
-                  c->d_flags.as<int>(), c->d_sysfault.as<int>(), c->krun.as<int>(),
-                  c->ktable.as<unsigned>(), c->ktable_tiles, tiles, cells ? &A : nullptr);
+                  c->d_kbase.as<unsigned>(), c->d_kshift.as<int>(), budget.as<unsigned>(),
+                  c->keys.as<unsigned>(), c->kfull.as<unsigned>(), c->keys2.as<unsigned>(),
+                  c->vals2.as<int>(), c->krank.as<unsigned>(), c->d_flags.as<int>(),
+                  c->d_sysfault.as<int>(), c->krun.as<int>(), c->ktable.as<unsigned>(),
+                  c->ktable_tiles, tiles, cells ? &A : nullptr);
+}
+KeyTable key_table(gr_ctx *c) {
+  KeyTable kt;
+  kt.keys2 = c->keys2.as<unsigned>();
+  kt.start = c->ktable.as<unsigned>() + (size_t)c->ktable_tiles * key_table_tile();
+  kt.krange = c->d_krange.as<unsigned>();
+  kt.kbase = c->d_kbase.as<unsigned>();
+  kt.kshift = c->d_kshift.as<int>();
+  kt.full = c->kfull.as<unsigned>();
+  kt.run = c->krun.as<int>();
+  return kt;
 }
 
 // half: also take the leapfrog half step of the plan's integrated systems
@@ -1890,12 +1935,10 @@ void phase_sort_real(gr_ctx *c, Plan &P, bool half = false, int pack = 0) {
   if (P.tiles_real > 0) {  // a step: counting sort (the bounds' replicas are reset already)
     if (!step_bounds(P)) step_minmax(c, P);
     key_sort(c, P, xs, P.blk_real, P.nblk_real, P.d_bbase_real, P.d_real_list,
-             (int)P.real_list.size(), P.n_real, P.tiles_real, sort_preps_cells(P, false));
+             (int)P.real_list.size(), P.n_real, P.tiles_real, P.d_budget_real,
+             sort_preps_cells(P, false));
     all_real(c, arb, arn);
-    const KeyTable kt =
-        key_table_view(c->ktable.as<unsigned>(), c->ktable_tiles, P.tiles_real, c->keys2.as<unsigned>(),
-                       c->krun.as<int>(), c->d_krange.as<unsigned>(), c->d_kbase.as<unsigned>(),
-                       P.d_real_list.as<int>(), (int)P.real_list.size());
+    const KeyTable kt = key_table(c);
     Pool<R> A = pool_view<R>(c, c->cur), B = pool_view<R>(c, 1 - c->cur);
     launch_permute_real<R>(s, A, B, c->d_sd.as<SysDesc>(), arb, arn, P.d_bbase_real.as<int>(),
                            c->vals.as<int>(), c->vals2.as<int>(), c->d_flags.as<int>(),
@@ -1953,11 +1996,9 @@ void phase_ghosts(gr_ctx *c, Plan &P, bool generate, bool sort) {
   if (table) {  // a step: counting sort (the bounds' replicas are reset already)
     const XP gx = xp_gxs(c);
     key_sort(c, P, gx, P.blk_ghost, P.nblk_ghost, P.d_bbase_ghost, P.d_ghost_list,
-             (int)P.ghost_list.size(), P.n_ghost, P.tiles_ghost, sort_preps_cells(P, true));
-    const KeyTable kt =
-        key_table_view(c->ktable.as<unsigned>(), c->ktable_tiles, P.tiles_ghost, c->keys2.as<unsigned>(),
-                       c->krun.as<int>(), c->d_krange.as<unsigned>(), c->d_kbase.as<unsigned>(),
-                       P.d_ghost_list.as<int>(), (int)P.ghost_list.size());
+             (int)P.ghost_list.size(), P.n_ghost, P.tiles_ghost, P.d_budget_ghost,
+             sort_preps_cells(P, true));
+    const KeyTable kt = key_table(c);
     launch_permute_ghost(s, gx, c->gidx_s.as<int>(), c->gbnd_s.as<int>(), xpw_pool(c, c->cur),
                          A.gidx, A.gbnd, c->d_sd.as<SysDesc>(), c->d_n.as<int>(),
                          P.blk_ghost.as<Blk>(), P.nblk_ghost, P.d_bbase_ghost.as<int>(),
@@ -2156,20 +2197,33 @@ void phase_xsph(gr_ctx *c, Plan &P) {
 // kGrowMargin cells wider on every side, would not fit gets new arrays sized
 // for its current extent (cell_capacity).  Cell arrays are rebuilt every
 // step, so nothing is copied; plans and captured graphs refer to the tables
-// and are dropped.  Returns whether anything was reallocated.
-bool grow_cells(gr_ctx *c, const Plan &P) {
-  if (P.inters.empty()) return false;
+// and are dropped.  So they are where a system outgrows its budget of the key
+// table; `moved`: by the bounds that a pass over the positions, uploaded since
+// the budgets were made, has just left (the cell arrays only by `stepped`, the
+// last call's bounds).  Returns whether the plan is to be made anew.
+bool grow_cells(gr_ctx *c, const Plan &P, bool stepped, bool moved) {
   const int ns = (int)c->sys.size();
   std::vector<int> nn(ns);
   HIPCHK(hipMemcpyAsync(nn.data(), c->d_n.p, ns * sizeof(int), hipMemcpyDeviceToHost, c->stream));
-  HostBounds hb;
-  read_bounds(c, hb);
-  auto outgrown = [&](const std::vector<int> &list, int tiles) {
-    if (list.empty() || tiles == 0) return false;
-    const int t = key_tiles(c, list, hb, kGrowMargin);
-    return t == 0 || t > tiles;
+  HostBounds hb, now;
+  read_bounds(c, hb, moved ? &now : nullptr);
+  auto outgrown = [&](const std::vector<int> &list, int tiles,
+                      const std::vector<unsigned> &budget) {
+    if (tiles == 0) return false;
+    std::vector<unsigned> b;
+    if (key_tiles(c, list, moved ? now : hb, kGrowMargin, b, 1.25) == 0) return true;
+    for (size_t q = 0; q < b.size(); ++q)
+      if (b[q] > budget[q]) return true;
+    return false;
   };
-  const bool tables = outgrown(P.real_list, P.tiles_real) || outgrown(P.ghost_list, P.tiles_ghost);
+  const bool tables = outgrown(P.real_list, P.tiles_real, P.budget_real) ||
+                      outgrown(P.ghost_list, P.tiles_ghost, P.budget_ghost);
+  if (!stepped) {
+    if (!tables) return false;
+    drop_graphs(c);
+    c->plans.clear();
+    return true;
+  }
   bool grew = false;
   for (int it : P.inters) {
     InterH &in = c->inter[it];
@@ -2401,18 +2455,23 @@ void do_steps(gr_ctx *c, const std::vector<int> &integs, int nsteps) {
   // the step's bounds passes find their replicas reset (each step's sort leaves
   // them so; other users of the bounds do not), and the first step the bounds
   auto reset_bounds = [&]() {
-    launch_minmax_reset(c->stream, P->d_real_list.as<int>(), (int)P->real_list.size(),
-                        c->d_bbmin.as<long long>(), c->d_bbmax.as<long long>(), c->bb_rs);
-    launch_minmax_reset(c->stream, P->d_ghost_list.as<int>(), (int)P->ghost_list.size(),
-                        c->d_bbmin.as<long long>(), c->d_bbmax.as<long long>(), c->bb_rs);
+    reset_replicas(c, *P);
     if (step_bounds(*P)) step_minmax(c, *P);
   };
   if (nsteps > 0) reset_bounds();
   for (int k0 = 0; k0 < nsteps; k0 += kGrowChunk) {
-    if ((k0 > 0 || c->bb_valid) && grow_cells(c, *P)) {
-      P = &get_plan(c, integs);
-      mark_grids(c, *P);
-      reset_bounds();
+    const bool stepped = k0 > 0 || c->bb_valid;
+    const bool moved = k0 == 0 && P->tiles_real > 0 && P->x_epoch != c->x_epoch;
+    if (moved) {
+      P->x_epoch = c->x_epoch;
+      if (!step_bounds(*P)) step_minmax(c, *P);
+    }
+    if (stepped || moved) {
+      if (grow_cells(c, *P, stepped, moved)) {
+        P = &get_plan(c, integs);
+        mark_grids(c, *P);
+        reset_bounds();
+      }
     }
     const int k1 = std::min(nsteps, k0 + kGrowChunk);
     for (int k = k0; k < k1; ++k) {
@@ -2767,6 +2826,7 @@ int gr_system_upload(gr_ctx *c, int sys, int field, const double *data, int64_t 
       }
     }
     copy_field(c, s, field, true, const_cast<double *>(data), n, nc);
+    if (field == GR_F_X && s.kind != GR_SYS_GHOST) ++c->x_epoch;
   });
 }
 

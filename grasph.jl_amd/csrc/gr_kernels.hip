@@ -365,6 +365,14 @@ __device__ inline void key_space_store(const KeySpace &K, int s, bool live, long
     atomicOr(&flags[1], 8);
   }
 }
+// Buckets of a system's `range` keys in the counting sort: a bucket is 2^sh keys,
+// one where the system keeps to its budget.
+__device__ inline unsigned key_buckets(unsigned long long range, unsigned budget, int &sh) {
+  sh = 0;
+  if (range == 0ull) return 0u;
+  while (((range - 1ull) >> sh) >= (unsigned long long)budget) ++sh;
+  return (unsigned)((range - 1ull) >> sh) + 1u;
+}
 // Flags of the whole key range: overflow, the bound of the keys and the radix
 // passes below it.  The running base only grows, so overflowing at some system
 // means the total overflows.
@@ -377,16 +385,18 @@ __device__ inline void key_flags(unsigned long long total, int *flags) {
 __global__ void __launch_bounds__(KB_THREADS)
     k_key_base(const int *list, int nlist, int D, int pad, const int *n_dev, const StepSys *st,
                long long *bbmin, long long *bbmax, int rs, int *kmin, int *kmax,
-               unsigned *kbase, unsigned *krange, int *flags, int *sysfault, int keep) {
+               unsigned *kbase, unsigned *krange, int *flags, int *sysfault,
+               const unsigned *budget, int *kshift) {
   // one workgroup: the systems' key ranges in parallel, KB_THREADS at a time,
   // and their exclusive prefix sum (each system's keys start after the ranges
-  // of the systems listed before it, plus one padding key each when `pad`)
-  __shared__ unsigned long long wsum[KB_THREADS / 64];
+  // of the systems listed before it, plus one padding key each when `pad`);
+  // with `budget`, for the counting sort, their buckets'
+  __shared__ unsigned long long wsum[KB_THREADS / 64], wall[KB_THREADS / 64];
   const int t = threadIdx.x, lane = t & 63, w = t >> 6;
-  unsigned long long carry = 0;
+  unsigned long long carry = 0, all = 0;
   for (int q0 = 0; q0 < nlist; q0 += KB_THREADS) {
     const int q = q0 + t;
-    unsigned long long range = 0;
+    unsigned long long range = 0, num = 0;
     int s = -1;
     if (q < nlist) {
       s = list[q];
@@ -396,26 +406,40 @@ __global__ void __launch_bounds__(KB_THREADS)
       if (!live) range = 0;
       key_space_store(K, s, live, bbmin, bbmax, kmin, kmax, krange, flags, sysfault);
       range += pad ? 1 : 0;
+      num = range;
+      if (budget) {
+        int sh;
+        num = key_buckets(range, budget[q], sh);
+        kshift[s] = sh;
+      }
     }
-    unsigned long long inc = range;
+    unsigned long long inc = num;
     for (int o = 1; o < 64; o <<= 1) {
       const unsigned long long u = __shfl_up(inc, o, 64);
       if (lane >= o) inc += u;
+      range += __shfl_xor(range, o, 64);
     }
-    if (lane == 63) wsum[w] = inc;
+    if (lane == 63) {
+      wsum[w] = inc;
+      wall[w] = range;
+    }
     __syncthreads();
     unsigned long long off = 0, tot = 0;
     for (int v = 0; v < KB_THREADS / 64; ++v) {
       off += v < w ? wsum[v] : 0ull;
       tot += wsum[v];
+      all += wall[v];
     }
-    if (q < nlist) kbase[s] = (unsigned)(carry + off + inc - range);
+    if (q < nlist) kbase[s] = (unsigned)(carry + off + inc - num);
     carry += tot;
     __syncthreads();  // wsum is written again for the next systems
   }
   if (t == 0) {
-    if (!keep) flags[0] = 0;
-    key_flags(carry, flags);
+    key_flags(all, flags);
+    if (budget)
+      flags[2] = (int)(unsigned)carry;
+    else
+      flags[0] = 0;
   }
 }
 
@@ -729,9 +753,12 @@ __global__ void __launch_bounds__(GR_BLOCK) k_cells_prep(CellsArgs A, int *flags
 //
 // Table (key_table_bytes): counts, starts, tile sums, laid out for the tiles it
 // was allocated with.  Every count and sum a sort raises is zero again when it
-// has ended.  `cap`, a multiple of KT_TILE less one, bounds the keys of the
-// step's sort; with more keys than that (a system that has run out since the
-// plan was made), one wavefront of k_key_place sorts the step's keys by radix.
+// has ended.  Each system has a budget of table entries.  One that has outgrown
+// its budget since the plan was made has 2^sh keys to an entry until the plan is
+// made anew (`kshift`), and its particles are ordered within an entry by their
+// keys (`full`) first; the others do not notice.  Sort of 200k particles, 20 a cell
+// (us), with a budget for all keys / 4 / 64 / 4096 keys to an entry: 2D 38 / 52 /
+// 124 / 2260, 3D 40 / 40 / 65 / 480.
 // ---------------------------------------------------------------------------
 
 #define KT_TILE 1024  // keys per workgroup of the scan
@@ -768,11 +795,11 @@ template <int D>
 __global__ void __launch_bounds__(GR_BLOCK)
     k_key_count(XP xs, const SysDesc *sd, const int *n_dev, const StepSys *st, const Blk *blk,
                 const int *bbase, const int *list, int nlist, long long *bbmin, long long *bbmax,
-                int rs, int *kmin, int *kmax, unsigned *krange, unsigned *kbase, unsigned *keys,
-                int *vals, unsigned *rank, int *flags, int *sysfault, unsigned *count,
-                unsigned *tsum, unsigned cap, int inl) {
-  __shared__ int s_kmin[3];
-  __shared__ unsigned s_kr[3], s_base, s_total;
+                int rs, int *kmin, int *kmax, unsigned *krange, unsigned *kbase, int *kshift,
+                const unsigned *budget, unsigned *keys, unsigned *full, unsigned *rank, int *flags,
+                int *sysfault, unsigned *count, unsigned *tsum, int inl) {
+  __shared__ int s_kmin[3], s_sh;
+  __shared__ unsigned s_kr[3], s_base;
   __shared__ unsigned kw[GR_BLOCK / 64];
   const Blk b = blk[blockIdx.x];
   const int s = b.item;
@@ -781,10 +808,6 @@ __global__ void __launch_bounds__(GR_BLOCK)
   const int n = n_dev[s];
   const int64_t gi = sd[s].off + i;
   if (b.first >= n && blockIdx.x != 0) {  // beyond the live ghosts
-    if (i < sd[s].cap) {
-      keys[bbase[s] + i] = 0xFFFFFFFFu;
-      vals[bbase[s] + i] = (int)gi;
-    }
     return;
   }
   const double cutoff = st[s].sort_cutoff;
@@ -795,32 +818,41 @@ __global__ void __launch_bounds__(GR_BLOCK)
     // the key bases, found by every workgroup for itself (the first stores them)
     if (w == 0) {
       unsigned long long range = 0;
-      int q = -1;
+      unsigned num = 0;
+      int q = -1, sh = 0;
       KeySpace K;
       if (lane < nlist) {
         q = list[lane];
         const bool live = n_dev[q] > 0;
         range = key_space(D, st[q].sort_cutoff, bbmin, bbmax, rs, q, K);
         if (!live) range = 0;
+        num = key_buckets(range, budget[lane], sh);
         if (blockIdx.x == 0)
           key_space_store(K, q, live, bbmin, bbmax, kmin, kmax, krange, flags, sysfault);
       }
-      unsigned long long inc = range;
+      unsigned inc = num;
       for (int o = 1; o < 64; o <<= 1) {
-        const unsigned long long u = __shfl_up(inc, o, 64);
+        const unsigned u = __shfl_up(inc, o, 64);
         if (lane >= o) inc += u;
       }
-      if (q >= 0 && blockIdx.x == 0) kbase[q] = (unsigned)(inc - range);
+      if (blockIdx.x == 0) {
+        if (q >= 0) {
+          kbase[q] = inc - num;
+          kshift[q] = sh;
+        }
+        for (int o = 1; o < 64; o <<= 1) range += __shfl_xor(range, o, 64);
+        if (lane == 63) {
+          key_flags(range, flags);
+          flags[2] = (int)inc;
+        }
+      }
       if (q == s) {
         for (int d = 0; d < 3; ++d) {
           s_kmin[d] = K.kmin[d];
           s_kr[d] = K.kr[d];
         }
-        s_base = (unsigned)(inc - range);
-      }
-      if (lane == 63) {
-        s_total = (unsigned)(inc < 0xFFFFFFFFull ? inc : 0xFFFFFFFFull);
-        if (blockIdx.x == 0) key_flags(inc, flags);
+        s_base = inc - num;
+        s_sh = sh;
       }
     }
   } else if (threadIdx.x == 0) {
@@ -829,16 +861,17 @@ __global__ void __launch_bounds__(GR_BLOCK)
       s_kr[d] = krange[s * 3 + d];
     }
     s_base = kbase[s];
-    s_total = (unsigned)flags[2];
+    s_sh = kshift[s];
   }
   __syncthreads();
   const bool faulted = s_kr[0] == 0u;
+  const int sh = s_sh;
   auto key_of = [&](const double *p) {
     unsigned k = 0;
 #pragma unroll
     for (int d = 0; d < D; ++d)
       k = k * s_kr[d] + (unsigned)(key_comp(p[d], cutoff) - s_kmin[d]);
-    return s_base + (faulted ? 0u : k);
+    return faulted ? 0u : k;
   };
   unsigned key = 0xFFFFFFFFu, kn = 0u;
   if (i < n) {
@@ -858,32 +891,29 @@ __global__ void __launch_bounds__(GR_BLOCK)
   if (lane == 63) k2 = w + 1 < GR_BLOCK / 64 ? kw[w + 1] : kn;
   const bool inv = i + 1 < n && k2 < key;
   if (__syncthreads_or(inv) && threadIdx.x == 0 && ld_dev(&flags[0]) == 0) atomicOr(&flags[0], 1);
-  if (i >= sd[s].cap) key = 0xFFFFFFFFu;
   const bool valid = i < n;
   const int p = bbase[s] + i;
-  if (i < sd[s].cap) {
-    keys[p] = key;
-    vals[p] = (int)gi;
+  const unsigned at = s_base + (key >> sh);  // the table's entry
+  if (valid) {
+    keys[p] = at;
+    if (sh > 0) full[p] = key;
   }
-  if (s_total > cap) return;  // sorted by k_key_place's workgroup
   int len;
   int head = run_head(key, valid, len);
   unsigned r0 = 0;
-  if (valid && head == lane) r0 = atomicAdd(&count[key], (unsigned)len);
+  if (valid && head == lane) r0 = atomicAdd(&count[at], (unsigned)len);
   r0 = __shfl(r0, head, 64);
   if (valid) rank[p] = faulted ? (unsigned)i : r0 + (unsigned)(lane - head);
-  head = run_head(key / KT_TILE, valid, len);
+  head = run_head(at / KT_TILE, valid, len);
   if (valid && head == lane)
-    atomicAdd(&tsum[key / KT_TILE * KT_REP + blockIdx.x % KT_REP], (unsigned)len);
+    atomicAdd(&tsum[at / KT_TILE * KT_REP + blockIdx.x % KT_REP], (unsigned)len);
 }
 
 // Starts of KT_TILE keys: the sums of the tiles before them, then a scan.
 __global__ void __launch_bounds__(GR_BLOCK)
-    k_key_scan(unsigned *count, const unsigned *tsum, unsigned *start, const int *flags,
-               unsigned cap) {
-  const unsigned total = (unsigned)flags[2];
+    k_key_scan(unsigned *count, const unsigned *tsum, unsigned *start, const int *flags) {
   const unsigned tile = blockIdx.x;
-  if (total > cap || tile * KT_TILE > total) return;
+  if (tile * KT_TILE > (unsigned)flags[2]) return;
   __shared__ unsigned wsum[GR_BLOCK / 64], psum[GR_BLOCK / 64];
   const int t = threadIdx.x, lane = t & 63, w = t >> 6;
   uint4 *c4 = reinterpret_cast<uint4 *>(count + (size_t)tile * KT_TILE) + t;
@@ -911,73 +941,20 @@ __global__ void __launch_bounds__(GR_BLOCK)
       make_uint4(run, run + c.x, run + c.x + c.y, run + c.x + c.y + c.z);
 }
 
-// Stable radix sort of N pairs by one wavefront, in place with (k1, v1) as the
-// other buffer: four 8-bit passes.
-__device__ void radix_one_wave(unsigned *k0, int *v0, unsigned *k1, int *v1, int N,
-                               unsigned *base) {
-  const int lane = threadIdx.x & 63;
-  const unsigned long long lt = lane == 0 ? 0ull : (~0ull >> (64 - lane));
-  for (int pass = 0; pass < 4; ++pass) {
-    const int shift = 8 * pass;
-    unsigned *ki = pass & 1 ? k1 : k0, *ko = pass & 1 ? k0 : k1;
-    int *vi = pass & 1 ? v1 : v0, *vo = pass & 1 ? v0 : v1;
-    for (int d = lane; d < 256; d += 64) base[d] = 0u;
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
-    for (int e = lane; e < N; e += 64) atomicAdd(&base[(ki[e] >> shift) & 255u], 1u);
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
-    unsigned carry = 0;
-    for (int d0 = 0; d0 < 256; d0 += 64) {
-      const unsigned c = base[d0 + lane];
-      unsigned inc = c;
-      for (int o = 1; o < 64; o <<= 1) {
-        const unsigned u = __shfl_up(inc, o, 64);
-        if (lane >= o) inc += u;
-      }
-      base[d0 + lane] = carry + inc - c;
-      carry += __shfl(inc, 63, 64);
-    }
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
-    for (int e0 = 0; e0 < N; e0 += 64) {
-      const int e = e0 + lane;
-      const bool valid = e < N;
-      const unsigned k = valid ? ki[e] : 0u;
-      const int v = valid ? vi[e] : 0;
-      const unsigned d = (k >> shift) & 255u;
-      unsigned long long m = __ballot(valid);
-      for (int q = 0; q < 8; ++q) {
-        const unsigned long long bal = __ballot((d >> q) & 1u);
-        m &= ((d >> q) & 1u) ? bal : ~bal;
-      }
-      const unsigned at = base[d];
-      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
-      if (valid) {
-        const unsigned r = (unsigned)__popcll(m & lt);
-        ko[at + r] = k;
-        vo[at + r] = v;
-        if (r == 0) base[d] = at + (unsigned)__popcll(m);
-      }
-      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
-    }
-    // the next pass reads what this one wrote to memory
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "agent");
-  }
-}
-
 // Every particle to its cell's slots (former place and key); also the tile
 // sums and the listed systems' bounds back to their initial values.  The
 // first nprep workgroups prepare the step's cell arrays (A): a longer chain of
 // dependent loads than the others', so they start first.
 __global__ void __launch_bounds__(GR_BLOCK)
-    k_key_place(const SysDesc *sd, const int *n_dev, const Blk *blk, const int *bbase, unsigned *keys,
-                int *vals, unsigned *keys2, int *vals2, const unsigned *rank,
-                const unsigned *start, unsigned *tsum, int ntile, int N, const int *list,
-                int nlist, long long *bbmin, long long *bbmax, int rs, int *flags,
-                unsigned cap, int nprep, CellsArgs A, int *sysfault, int *run) {
+    k_key_place(const SysDesc *sd, const int *n_dev, const Blk *blk, const int *bbase,
+                const unsigned *keys, const unsigned *full, const int *kshift, unsigned *keys2,
+                int *vals2, const unsigned *rank, const unsigned *start, unsigned *tsum, int ntile,
+                int N, const int *list, int nlist, long long *bbmin, long long *bbmax, int rs,
+                int *flags, int nprep, CellsArgs A, int *sysfault, int *run) {
   if ((int)blockIdx.x < nprep) {
     cells_prep(A, (int)blockIdx.x, flags, sysfault);
     return;
   }
-  __shared__ unsigned base[256];
   const int bid = (int)blockIdx.x - nprep;
   const int nthr = ((int)gridDim.x - nprep) * GR_BLOCK, me = bid * GR_BLOCK + threadIdx.x;
   for (int k = me; k < ntile * KT_REP; k += nthr) tsum[k] = 0u;
@@ -988,10 +965,6 @@ __global__ void __launch_bounds__(GR_BLOCK)
     bbmax[at] = LLONG_MIN;
   }
   if (flags[0] == 0) return;
-  if ((unsigned)flags[2] > cap) {
-    if (bid == 0 && threadIdx.x < 64) radix_one_wave(keys, vals, keys2, vals2, N, base);
-    return;
-  }
   const Blk b = blk[bid];
   const int s = b.item;
   const int i = b.first + threadIdx.x;
@@ -1000,10 +973,11 @@ __global__ void __launch_bounds__(GR_BLOCK)
   const unsigned key = keys[p];
   const unsigned first = start[key];
   const unsigned slot = first + rank[p];
-  const bool big = start[key + 1] - first > KT_BIG;
+  const int sh = kshift[s];
+  const bool big = sh > 0 || start[key + 1] - first > KT_BIG;
   if (__ballot(big) != 0ull) {  // the lengths of the runs, at their first slots
     int len;
-    const int head = run_head(key, true, len);
+    const int head = run_head(sh > 0 ? full[p] : key, true, len);
     if (big && head == (int)(threadIdx.x & 63) && slot < (unsigned)N) run[slot] = len;
   }
   // the counts place every particle below N; a slot beyond it is reported,
@@ -1017,21 +991,21 @@ __global__ void __launch_bounds__(GR_BLOCK)
 }
 
 // Slot p of the sorted order: the particle placed there (its pool index) and
-// the slot its rank in the cell gives it.
-__device__ __forceinline__ int key_slot(int p, const int *vals, const unsigned *keys2,
-                                        const int *vals2, const unsigned *start, const int *flags,
-                                        unsigned cap, const int *run, int &slot) {
-  slot = p;
-  if ((unsigned)flags[2] > cap) return vals[p];
+// the slot its rank in the cell gives it.  sh: its system's kshift; rel: from a
+// pool index of the system to its place in `full`.
+__device__ __forceinline__ int key_slot(int p, const int *vals2, const KeyTable &kt, int sh,
+                                        int64_t rel, int &slot) {
   const int v = vals2[p];
-  const unsigned k = keys2[p];
-  const int a = (int)start[k], e = (int)start[k + 1];
+  const unsigned k = kt.keys2[p];
+  const int a = (int)kt.start[k], e = (int)kt.start[k + 1];
   int r = 0;
-  if (e - a > KT_BIG) {
+  if (sh > 0 || e - a > KT_BIG) {
+    const unsigned kv = sh > 0 ? kt.full[rel + v] : 0u;
     for (int j = a; j < e;) {
-      const int u = vals2[j], len = run[j] > 1 ? run[j] : 1;
+      const int u = vals2[j], len = kt.run[j] > 1 ? kt.run[j] : 1;
+      const unsigned ku = sh > 0 ? kt.full[rel + u] : 0u;
       const int below = v - u;  // of the run's consecutive places
-      r += below > 0 ? (below < len ? below : len) : 0;
+      r += ku < kv ? len : ku > kv || below <= 0 ? 0 : below < len ? below : len;
       j += len;
     }
     slot = a + r;
@@ -1077,7 +1051,7 @@ __global__ void k_permute_real(Pool<R> A, Pool<R> B, const SysDesc *sd, const Bl
   if constexpr (TAB) {
     if (flags[0] != 0 && bbase[s] >= 0 && kt.krange[s * 3] != 0u) {  // not a faulted system
       int slot;
-      src = key_slot(bbase[s] + i, vals, kt.keys2, vals2, kt.start, flags, kt.cap, kt.run, slot);
+      src = key_slot(bbase[s] + i, vals2, kt, kt.kshift[s], bbase[s] - S.off, slot);
       dst = S.off + (slot - bbase[s]);
     }
   } else {
@@ -1330,15 +1304,9 @@ __global__ void k_permute_ghost(XP gxs, const int *gidx_s, const int *gbnd_s, XP
   int64_t src = dst;
   if constexpr (TAB) {
     if (flags[0] != 0 && kt.krange[g * 3] != 0u) {
-      // the live ghosts of the systems listed before this one
-      int p0 = 0;
-      if ((unsigned)flags[2] > kt.cap) {
-        for (int q = 0; q < kt.nlist && kt.list[q] != g; ++q) p0 += n_dev[kt.list[q]];
-      } else {
-        p0 = (int)kt.start[kt.kbase[g]];
-      }
+      const int p0 = (int)kt.start[kt.kbase[g]];  // the live ghosts of the systems before
       int slot;
-      src = key_slot(p0 + k, vals, kt.keys2, vals2, kt.start, flags, kt.cap, kt.run, slot);
+      src = key_slot(p0 + k, vals2, kt, kt.kshift[g], bbase[g] - G.off, slot);
       dst = G.off + (slot - p0);
     }
   } else {
@@ -2411,7 +2379,7 @@ void launch_key_base(hipStream_t s, const int *list, int nlist, int D, int pad, 
                      const StepSys *st, long long *bbmin, long long *bbmax, int rs, int *kmin,
                      int *kmax, unsigned *kbase, unsigned *krange, int *flags, int *sysfault) {
   k_key_base<<<1, KB_THREADS, 0, s>>>(list, nlist, D, pad, n, st, bbmin, bbmax, rs, kmin, kmax,
-                                      kbase, krange, flags, sysfault, 0);
+                                      kbase, krange, flags, sysfault, nullptr, nullptr);
 }
 static int cells_prep_blocks(const CellsArgs &A) { return nb_of(A.n_inter, GR_BLOCK) + A.ncblk; }
 void launch_cells_prep(hipStream_t s, const CellsArgs &A, int *flags, int *sysfault) {
@@ -2424,48 +2392,35 @@ int key_table_tile() { return KT_TILE; }
 void launch_key_sort(hipStream_t s, XP xs, const SysDesc *sd, const int *n, const StepSys *st,
                      const Blk *blk, int nblk, const int *bbase, int D, const int *list, int nlist,
                      int N, long long *bbmin, long long *bbmax, int rs, int *kmin, int *kmax,
-                     unsigned *krange, unsigned *kbase, unsigned *keys, int *vals,
-                     unsigned *keys2, int *vals2, unsigned *rank, int *flags, int *sysfault,
-                     int *run, unsigned *table, int tiles, int ntile, const CellsArgs *cells) {
+                     unsigned *krange, unsigned *kbase, int *kshift, const unsigned *budget,
+                     unsigned *keys, unsigned *full, unsigned *keys2, int *vals2, unsigned *rank,
+                     int *flags, int *sysfault, int *run, unsigned *table, int tiles, int ntile,
+                     const CellsArgs *cells) {
   if (nblk <= 0) {
     if (cells) launch_cells_prep(s, *cells, flags, sysfault);
     return;
   }
   unsigned *count = table, *start = table + (size_t)tiles * KT_TILE;
   unsigned *tsum = table + (size_t)tiles * KT_TILE * 2;
-  const unsigned cap = (unsigned)ntile * KT_TILE - 1u;
   const int inl = nlist <= KC_SYSTEMS && nblk <= KC_BLOCKS;
   if (!inl)
     k_key_base<<<1, KB_THREADS, 0, s>>>(list, nlist, D, 0, n, st, bbmin, bbmax, rs, kmin, kmax,
-                                        kbase, krange, flags, sysfault, 1);
+                                        kbase, krange, flags, sysfault, budget, kshift);
+  auto go = [&](auto dc) {
+    k_key_count<decltype(dc)::value><<<nblk, GR_BLOCK, 0, s>>>(
+        xs, sd, n, st, blk, bbase, list, nlist, bbmin, bbmax, rs, kmin, kmax, krange, kbase, kshift,
+        budget, keys, full, rank, flags, sysfault, count, tsum, inl);
+  };
   if (D == 2)
-    k_key_count<2><<<nblk, GR_BLOCK, 0, s>>>(xs, sd, n, st, blk, bbase, list, nlist, bbmin, bbmax,
-                                             rs, kmin, kmax, krange, kbase, keys, vals, rank,
-                                             flags, sysfault, count, tsum, cap, inl);
+    go(std::integral_constant<int, 2>{});
   else
-    k_key_count<3><<<nblk, GR_BLOCK, 0, s>>>(xs, sd, n, st, blk, bbase, list, nlist, bbmin, bbmax,
-                                             rs, kmin, kmax, krange, kbase, keys, vals, rank,
-                                             flags, sysfault, count, tsum, cap, inl);
-  k_key_scan<<<ntile, GR_BLOCK, 0, s>>>(count, tsum, start, flags, cap);
+    go(std::integral_constant<int, 3>{});
+  k_key_scan<<<ntile, GR_BLOCK, 0, s>>>(count, tsum, start, flags);
   const CellsArgs A = cells ? *cells : CellsArgs{};
   const int nprep = cells_prep_blocks(A);
-  k_key_place<<<nblk + nprep, GR_BLOCK, 0, s>>>(
-      sd, n, blk, bbase, keys, vals, keys2, vals2, rank, start, tsum, ntile, N, list, nlist, bbmin,
-      bbmax, rs, flags, cap, nprep, A, sysfault, run);
-}
-KeyTable key_table_view(unsigned *table, int tiles, int ntile, const unsigned *keys2,
-                        const int *run, const unsigned *krange, const unsigned *kbase, const int *list,
-                        int nlist) {
-  KeyTable kt;
-  kt.keys2 = keys2;
-  kt.run = run;
-  kt.start = table + (size_t)tiles * KT_TILE;
-  kt.krange = krange;
-  kt.kbase = kbase;
-  kt.list = list;
-  kt.nlist = nlist;
-  kt.cap = (unsigned)ntile * KT_TILE - 1u;
-  return kt;
+  k_key_place<<<nblk + nprep, GR_BLOCK, 0, s>>>(sd, n, blk, bbase, keys, full, kshift, keys2, vals2,
+                                                rank, start, tsum, ntile, N, list, nlist, bbmin,
+                                                bbmax, rs, flags, nprep, A, sysfault, run);
 }
 void launch_key_write(hipStream_t s, XP xs, const SysDesc *sd, const int *n, const StepSys *st,
                       const Blk *blk, int nblk, const int *bbase, int D, const int *kmin,

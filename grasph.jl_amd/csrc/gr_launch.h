@@ -95,30 +95,26 @@ struct CellsArgs {
 };
 // The counting sort of a step (keys, table, placement) after the bounds pass:
 // `table` of key_table_bytes(tiles) bytes, zeroed when allocated, of which this
-// sort uses ntile <= tiles tiles (ntile·key_table_tile() - 1 keys; the layout
-// goes by `tiles`, as sorts of different sizes share the table).  flags[0] must
-// be clear; the permutations take the order by key_table_view.  Replicas 1..
-// of the listed systems' bounds are reset, and `cells` prepared (as
-// launch_cells_prep does).
+// sort uses ntile <= tiles tiles: the listed systems' budgets of entries (at
+// least one each) come to less than ntile·key_table_tile().  (The layout goes by
+// `tiles`, as sorts of different sizes share the table.)  flags[0] must be clear;
+// the permutations take the order by a KeyTable.  Replicas 1.. of the listed
+// systems' bounds are reset, and `cells` prepared (as launch_cells_prep does).
 size_t key_table_bytes(int64_t ntile);
 int key_table_tile();
 void launch_key_sort(hipStream_t s, XP xs, const SysDesc *sd, const int *n, const StepSys *st,
                      const Blk *blk, int nblk, const int *bbase, int D, const int *list, int nlist,
                      int N, long long *bbmin, long long *bbmax, int rs, int *kmin, int *kmax,
-                     unsigned *krange, unsigned *kbase, unsigned *keys, int *vals,
-                     unsigned *keys2, int *vals2, unsigned *rank, int *flags, int *sysfault,
-                     int *run, unsigned *table, int tiles, int ntile,
+                     unsigned *krange, unsigned *kbase, int *kshift, const unsigned *budget,
+                     unsigned *keys, unsigned *full, unsigned *keys2, int *vals2, unsigned *rank,
+                     int *flags, int *sysfault, int *run, unsigned *table, int tiles, int ntile,
                      const CellsArgs *cells = nullptr);
 struct KeyTable {  // what the permutations read of the counting sort
   const unsigned *keys2, *start, *krange, *kbase;
-  const int *run;  // at the first slot of a run in a large cell: its length
-  const int *list;
-  int nlist;
-  unsigned cap;
+  const int *kshift;     // log2 of a system's keys to an entry
+  const unsigned *full;  // a particle's key in its system, where those are several
+  const int *run;        // at the first slot of a run: its length (large cells)
 };
-KeyTable key_table_view(unsigned *table, int tiles, int ntile, const unsigned *keys2,
-                        const int *run, const unsigned *krange, const unsigned *kbase, const int *list,
-                        int nlist);
 template <typename R>
 void launch_permute_real(hipStream_t s, const Pool<R> &A, const Pool<R> &B, const SysDesc *sd,
                          const Blk *blk, int nblk, const int *bbase, const int *vals,
