@@ -1161,16 +1161,24 @@ constexpr int kGrowChunk = 16;
 constexpr int kGrowMargin = 8;
 
 // Tiles of a counting table for the listed systems' cell keys (`budget`: of each),
-// `margin` cells wider than their bounds on every side; 0 beyond kMaxKeyTiles (8M keys, 68 MB
-// of table, whose scan would cost as much as the radix passes).  A ghost
-// system's bounds are its source's, widened by twice its cutoff (a mirror
-// moves a particle by at most that).  Also 0 where the particles times the mean
-// number in a cell of their system exceed kKeyRank: the rank within the cell
-// grows with them (sort of particles in motion, us, table / radix kernels, 2D:
-// 1M at 32 a cell 92 / 111, at 128 149 / 111; 200k at 128 57 / 80, at 200 73 / 75,
-// at 1024 76 / 75; 20k at 1024 33 / 51, at 4096 54 / 49).  `slack`: the limits are
-// so much higher for a table in use.
-constexpr int kMaxKeyTiles = 8192;
+// `margin` cells wider than their bounds on every side.  A ghost system's bounds
+// are its source's, widened by twice its cutoff (a mirror moves a particle by at
+// most that).
+//
+// 0, for the radix kernels, beyond kMaxKeyTiles (4M keys, 34 MB of table), where
+// the scan of the table and of its tile sums costs more than they do.  Step (us)
+// with table / radix kernels, 2D: 300 particles in a box of 2.5M keys 111 / 108,
+// 3.5M 137 / 124, 4.5M 163 / 134; 30k in 3.5M 138 / 145, 4.5M 164 / 155; 300k in
+// 4.5M 208 / 228, 7M 286 / 246; 3D: 300 in 3.5M 122 / 128, 30k in 4.5M 158 / 173, 7M
+// 206 / 195, 1M in 4.5M 541 / 550, 7M 607 / 594.
+//
+// Also 0 where the particles times the mean number in a cell of their system
+// exceed kKeyRank: the rank within the cell grows with them (particles in motion,
+// 2D: 1M at 32 a cell 92 / 111, at 128 149 / 111; 200k at 128 57 / 80, at 200
+// 73 / 75, at 1024 76 / 75; 20k at 1024 33 / 51, at 4096 54 / 49).
+//
+// `slack`: the limits are so much higher for a table in use.
+constexpr int kMaxKeyTiles = 4096;
 constexpr double kKeyRank = 3.2e7;
 int key_tiles(gr_ctx *c, const std::vector<int> &systems, const HostBounds &h, int margin,
               std::vector<unsigned> &budget, double slack = 1.0) {

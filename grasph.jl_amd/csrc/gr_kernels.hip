@@ -397,9 +397,10 @@ __global__ void __launch_bounds__(KB_THREADS)
   for (int q0 = 0; q0 < nlist; q0 += KB_THREADS) {
     const int q = q0 + t;
     unsigned long long range = 0, num = 0;
-    int s = -1;
+    int s = -1, sh = 0;
     if (q < nlist) {
       s = list[q];
+      const unsigned most = budget ? budget[q] : 0u;
       KeySpace K;
       const bool live = n_dev[s] > 0;
       range = key_space(D, st[s].sort_cutoff, bbmin, bbmax, rs, s, K);
@@ -408,8 +409,7 @@ __global__ void __launch_bounds__(KB_THREADS)
       range += pad ? 1 : 0;
       num = range;
       if (budget) {
-        int sh;
-        num = key_buckets(range, budget[q], sh);
+        num = key_buckets(range, most, sh);
         kshift[s] = sh;
       }
     }
@@ -417,11 +417,15 @@ __global__ void __launch_bounds__(KB_THREADS)
     for (int o = 1; o < 64; o <<= 1) {
       const unsigned long long u = __shfl_up(inc, o, 64);
       if (lane >= o) inc += u;
-      range += __shfl_xor(range, o, 64);
+    }
+    unsigned long long sum = inc;  // of the ranges (at lane 63)
+    if (__ballot(sh > 0) != 0ull) {
+      sum = range;
+      for (int o = 1; o < 64; o <<= 1) sum += __shfl_xor(sum, o, 64);
     }
     if (lane == 63) {
       wsum[w] = inc;
-      wall[w] = range;
+      wall[w] = sum;
     }
     __syncthreads();
     unsigned long long off = 0, tot = 0;
@@ -811,6 +815,9 @@ __global__ void __launch_bounds__(GR_BLOCK)
     return;
   }
   const double cutoff = st[s].sort_cutoff;
+  // (read early, though it is asked again below: the line is then at hand; 2D
+  // cloud of 300k particles 14.6 -> 9.2 us)
+  const int unsorted = threadIdx.x == 0 ? ld_dev(&flags[0]) : 0;
   double x[D];
 #pragma unroll
   for (int d = 0; d < D; ++d) x[d] = i < n ? xs[d][gi] : 0.0;
@@ -890,7 +897,8 @@ __global__ void __launch_bounds__(GR_BLOCK)
   unsigned k2 = __shfl_down(key, 1, 64);
   if (lane == 63) k2 = w + 1 < GR_BLOCK / 64 ? kw[w + 1] : kn;
   const bool inv = i + 1 < n && k2 < key;
-  if (__syncthreads_or(inv) && threadIdx.x == 0 && ld_dev(&flags[0]) == 0) atomicOr(&flags[0], 1);
+  if (__syncthreads_or(inv) && threadIdx.x == 0 && unsorted == 0 && ld_dev(&flags[0]) == 0)
+    atomicOr(&flags[0], 1);
   const bool valid = i < n;
   const int p = bbase[s] + i;
   const unsigned at = s_base + (key >> sh);  // the table's entry
