@@ -746,7 +746,7 @@ __device__ inline int wave_red_dpp(int v) {
 // of the sort's order) has r >= 3/4 a² and an error of u(12aX + 22a²), too
 // small to change its sign while X <= 1e5 c; beyond that all are tested, and
 // where c is so small or large that c² (or the tolerance's products) could
-// leave FP32's normal range (`all`).
+// leave FP32's normal range (`all`: cells outside 2^±40).
 template <int D>
 struct Screen {
   float xf[D], c2, tol;
@@ -755,7 +755,7 @@ struct Screen {
     finite = true;
 #pragma unroll
     for (int d = 0; d < D; ++d) {
-      xf[d] = stage(xi[d], O[d]);
+      xf[d] = (float)(xi[d] - O[d]);
       finite = finite && fabs(xi[d]) <= 1.7976931348623157e308;  // else it has no partner
     }
   }
@@ -768,10 +768,10 @@ struct Screen {
     tol = 6.1e-8f * (c * (24.0f * X + 96.0f * c));
     if (!(X <= 1.0e5f * c) || !(cutoff2 <= cell * cell * (1.0 + 1e-9))) tol = __builtin_inff();
     const unsigned e = (unsigned)((unsigned long long)__double_as_longlong(cell) >> 52);
-    all = e - (1023u - 40u) > 80u;  // (the exponent: scalar arithmetic)
+    all = e - (1023u - 40u) > 80u;  // (by the exponent: scalar arithmetic)
   }
   // a staged coordinate; one beyond FP32's range (or not finite) is far from
-  // every target that is not tested in FP64 throughout
+  // every target of a cell whose candidates are screened
   static __device__ inline float stage(double x, double o) {
     const float f = (float)(x - o);
     return fabsf(f) < 3.0e38f ? f : 3.0e38f;
