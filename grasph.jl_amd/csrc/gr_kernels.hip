@@ -432,8 +432,9 @@ __global__ void __launch_bounds__(KB_THREADS)
     for (int v = 0; v < KB_THREADS / 64; ++v) {
       off += v < w ? wsum[v] : 0ull;
       tot += wsum[v];
-      all += wall[v];
     }
+    if (t == 0)
+      for (int v = 0; v < KB_THREADS / 64; ++v) all += wall[v];
     if (q < nlist) kbase[s] = (unsigned)(carry + off + inc - num);
     carry += tot;
     __syncthreads();  // wsum is written again for the next systems
