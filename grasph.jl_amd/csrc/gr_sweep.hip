@@ -1919,22 +1919,24 @@ __global__ void __launch_bounds__(64)
 // ---------------------------------------------------------------------------
 
 // Up to this many targets a launch of force or strain-rate sweeps takes four
-// lanes per target (k_sweep_split).  Measured, us with one / four lanes (FP32):
-// 3D dam breaks of 27k targets 89 / 39, 64k 79 / 47, 125k 95 / 74, 216k
-// 107 / 114; visco-plastic columns (both stages) 32k 137 / 74, 144k 176 / 163,
-// 256k 216 / 245; 2D dam breaks 20k 21 / 13, 80k 21 / 17, 163k 26 / 29; EP
-// columns 26k 79 / 53, 102k 90 / 75, 205k 109 / 108; FP64 alike (3D 27k
-// 130 / 68, 125k 167 / 158, 216k 238 / 242).
-template <int D>
+// lanes per target (k_sweep_split).  Measured, us with one / four lanes (FP32; the
+// columns both stages): 3D dam breaks of 22k targets 89 / 38, 69k 88 / 54, 125k
+// 87 / 66, 157k 98 / 77; visco-plastic columns 72k 119 / 86, 144k 143 / 128, 216k
+// 176 / 167; 2D dam breaks, whose entries are not staged, 20k 21 / 14, 80k 21 / 18,
+// 99k 21 / 22, 163k 27 / 29; EP columns 13k 66 / 30, 97k 80 / 48, 157k 86 / 67, 259k
+// 97 / 94.  FP64: 3D 69k 166 / 103, 125k 149 / 139, 216k 218 / 218, columns 144k
+// 279 / 241; 2D 80k 36 / 31, 99k 34 / 35, EP 97k 96 / 80, 157k 116 / 113, 259k
+// 149 / 166.
+template <int D, int FAM>
 constexpr int64_t sweep_split_targets() {
-  return D == 3 ? 150000 : 115000;
+  return D == 3 ? 150000 : split_stages<D, FAM>() ? 115000 : 90000;
 }
 
 template <int D, typename R, int FAM>
 static void launch_one(hipStream_t s, const Pool<R> &P, const SweepArgs &a, bool cnt) {
   if constexpr (FAM == FAM_FORCE || FAM == FAM_FORCE_FLUID || FAM == FAM_FORCE_FLUID_INV ||
                 FAM == FAM_STRAIN) {
-    if (a.lt && (int64_t)a.nblk * a.block <= sweep_split_targets<D>()) {
+    if (a.lt && (int64_t)a.nblk * a.block <= sweep_split_targets<D, FAM>()) {
       const int nsub = a.block / 16;
       if (cnt)
         k_sweep_split<D, R, FAM, true><<<a.nblk * nsub, 64, 0, s>>>(
