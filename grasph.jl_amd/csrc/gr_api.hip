@@ -2289,7 +2289,7 @@ bool grow_cells(gr_ctx *c, const Plan &P, bool stepped, bool moved) {
 }
 
 // Phase events of one step (timing mode): 0 start, 1 sorted, 2 ghosts,
-// 3 grids, 4 half-step, then per stage (updaters end, sweeps end), last
+// 3 grids, 4 half-step, then per stage (records written, sweeps end), last
 // full-step end.  Recorded without synchronisation; read after the call.
 std::vector<hipEvent_t> &step_events(gr_ctx *c, int k, int nst) {
   if ((int)c->tev.size() <= k) c->tev.resize(k + 1);

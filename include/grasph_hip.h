@@ -375,8 +375,12 @@ int gr_get_cell_start(gr_ctx *ctx, int inter, int which, int64_t *out,
  * mode bit 0: record HIP events on the context stream at every phase of
  * every step of the following gr_step/gr_step_many calls (no extra
  * synchronisation inside a call); gr_get_timing returns the mean ms per step
- * of phases 0 sort, 1 ghosts, 2 grid, 3 half-step, 4 updaters + ghost
- * copies, 5 sweeps, 6 full step, 7 whole step, 8 neighbour search.
+ * of phases 0 sort, 1 ghosts, 2 grid, 3 half-step, 4 updaters, ghost
+ * kinematics and copies, partner records, 5 sweeps, 6 full step, 7 whole
+ * step, 8 neighbour search.  Work that a kernel of another phase does along
+ * with its own counts there: the half step and the first records with the
+ * sort, the grids and the cleared cell arrays with the last sort, the bounds
+ * of the next step's sort with the full step.
  * mode bit 1: count pairs with r < 2h in the sweeps; gr_get_pair_count
  * returns unique pairs per step (self pairs once, coupled pairs once),
  * gr_get_pair_stats the ordered self pairs (each unordered pair from both
