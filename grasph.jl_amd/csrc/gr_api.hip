@@ -877,56 +877,96 @@ FieldSets field_sets(gr_ctx *c, const SysH &s, int field, bool in) {
   return f;
 }
 
-// Transfers of 8-byte elements through the context's pinned buffers, one part on
-// the bus while the host copies its neighbour: launch(host buffer, first
-// element, elements) moves one part of whole particles.  Against a pageable copy
-// and a strided host loop for each component, a call that steps and downloads
-// (us): 64 2D columns, 59 MB, 157900 -> 134100, 3D dam break of 1.4M 98800 ->
-// 92100, of 224k with its upload 14100 -> 12800, 2D of 1.4k 1640 -> 1420.  Parts
-// of 32, 64 and 128 KB instead of 1 MB took 151800, 146600 and 137400 for the
-// columns.
+// Transfers through the context's pinned buffers, one part on the bus while the
+// host copies its neighbour: launch(host buffer, first element, elements) moves
+// one part of whole particles.  Against a pageable copy and a strided host loop
+// for each component, a call that steps and downloads (us): 64 2D columns, 59 MB,
+// 157900 -> 134100, 3D dam break of 1.4M 98800 -> 92100, of 224k with its upload
+// 14100 -> 12800, 2D of 1.4k 1640 -> 1420.  Parts of 32, 64 and 128 KB instead of
+// 1 MB took 151800, 146600 and 137400 for the columns.
+//
+// W is the element on the bus, which the host converts to and from (indices are
+// `add` larger for the caller): 4 bytes for what the device holds in 4 (with 8 an
+// upload of 1.4M of them took 365 us, 312 by the pageable copy, with 4 186; a
+// download 815, 637 and 423).
 constexpr size_t kStageBytes = 1 << 20;
-template <typename T, typename L>
-void staged(gr_ctx *c, bool in, T *user, int64_t count, int nc, L &&launch) {
-  static_assert(sizeof(T) == 8, "8-byte elements");
+template <typename W, typename T, typename L>
+void staged(gr_ctx *c, bool in, T *user, int64_t count, int nc, int add, L &&launch) {
   if (count <= 0) return;
   HostStage &H = c->stage;
   H.init(kStageBytes);
-  const int64_t part = (int64_t)(kStageBytes / 8) / nc * nc;
+  const int64_t part = (int64_t)(kStageBytes / sizeof(W)) / nc * nc;
   const int64_t parts = (count + part - 1) / part;
-  auto host = [&](int64_t r) { return reinterpret_cast<T *>(H.buf[r & 1]); };
+  auto host = [&](int64_t r) { return reinterpret_cast<W *>(H.buf[r & 1]); };
   auto len = [&](int64_t r) { return std::min(part, count - r * part); };
-  auto go = [&](int64_t r) {
+  // an event ends the use of a part's buffer where the end of the stream is not
+  // waited for instead
+  auto go = [&](int64_t r, bool event) {
     launch(host(r), r * part, len(r));
     HIPCHK(hipGetLastError());
-    HIPCHK(hipEventRecord(H.ev[r & 1], c->stream));
+    if (event) HIPCHK(hipEventRecord(H.ev[r & 1], c->stream));
   };
   if (in) {
     for (int64_t r = 0; r < parts; ++r) {
       if (r >= 2) HIPCHK(hipEventSynchronize(H.ev[r & 1]));
-      std::memcpy(host(r), user + r * part, (size_t)len(r) * 8);
-      go(r);
+      const T *u = user + r * part;
+      W *h = host(r);
+      if constexpr (std::is_same_v<W, T>)
+        std::memcpy(h, u, (size_t)len(r) * sizeof(W));
+      else
+        for (int64_t e = 0, n = len(r); e < n; ++e) h[e] = (W)(add != 0 ? u[e] - add : u[e]);
+      go(r, r + 2 < parts);
     }
     HIPCHK(hipStreamSynchronize(c->stream));
     return;
   }
-  for (int64_t r = 0; r < std::min<int64_t>(2, parts); ++r) go(r);
+  for (int64_t r = 0; r < std::min<int64_t>(2, parts); ++r) go(r, r + 1 < parts);
   for (int64_t r = 0; r < parts; ++r) {
-    HIPCHK(hipEventSynchronize(H.ev[r & 1]));
-    std::memcpy(user + r * part, host(r), (size_t)len(r) * 8);
-    if (r + 2 < parts) go(r + 2);
+    if (r + 1 < parts)
+      HIPCHK(hipEventSynchronize(H.ev[r & 1]));
+    else
+      HIPCHK(hipStreamSynchronize(c->stream));
+    T *u = user + r * part;
+    const W *h = host(r);
+    if constexpr (std::is_same_v<W, T>)
+      std::memcpy(u, h, (size_t)len(r) * sizeof(W));
+    else
+      for (int64_t e = 0, n = len(r); e < n; ++e) u[e] = add != 0 ? (T)h[e] + add : (T)h[e];
+    if (r + 2 < parts) go(r + 2, r + 3 < parts);
   }
+}
+// A single array of one part goes by a copy command instead: uploads of 12.8k floats
+// 17.3 us by the kernel, 12.4 by the copy, downloads 19.8 and 15.0.
+template <typename W>
+void copy_part(gr_ctx *c, bool in, W *host, W *dev, int64_t m) {
+  HIPCHK(hipMemcpyAsync(in ? dev : host, in ? host : dev, (size_t)m * sizeof(W),
+                        in ? hipMemcpyHostToDevice : hipMemcpyDeviceToHost, c->stream));
 }
 void copy_field(gr_ctx *c, const SysH &s, int field, bool in, double *data, int64_t n, int nc) {
   const FieldSets F = field_sets(c, s, field, in);
-  staged(c, in, data, n * nc, nc, [&](double *host, int64_t e0, int64_t m) {
-    launch_field(c->stream, in, host, m, nc, c->pool_cap, s.off + e0 / nc, F);
-  });
+  auto move = [&](auto tag) {
+    using W = decltype(tag);
+    const bool single = F.n == 1 && nc == 1 && (size_t)n * sizeof(W) <= kStageBytes;
+    staged<W>(c, in, data, n * nc, nc, 0, [&](W *host, int64_t e0, int64_t m) {
+      if (single)
+        copy_part(c, in, host, static_cast<W *>(F.p[0]) + s.off, m);
+      else
+        launch_field(c->stream, in, host, m, nc, c->pool_cap, s.off + e0 / nc, F);
+    });
+  };
+  if (F.n == 1 && F.esz[0] == 4)
+    move(0.0f);
+  else
+    move(0.0);
 }
 void copy_index(gr_ctx *c, const SysH &s, bool in, int64_t *data, int64_t n, int add,
                 const DBuf &b) {
-  staged(c, in, data, n, 1, [&](int64_t *host, int64_t e0, int64_t m) {
-    launch_index(c->stream, in, host, m, s.off + e0, add, (int *)b.p);
+  staged<int>(c, in, data, n, 1, add, [&](int *host, int64_t e0, int64_t m) {
+    int *dev = (int *)b.p + s.off + e0;
+    if ((size_t)n * sizeof(int) <= kStageBytes)
+      copy_part(c, in, host, dev, m);
+    else
+      launch_index(c->stream, in, host, m, dev);
   });
 }
 

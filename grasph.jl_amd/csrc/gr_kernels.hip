@@ -2319,15 +2319,16 @@ __global__ void k_fill_i32(int *p, int v, long long n) {
   if (i < n) p[i] = v;
 }
 
-// Fields between the caller's layout (particle-major FP64, staged in pinned host
-// memory) and the pool's component arrays: element e of `host` is component
-// e % nc of particle e / nc.  The kernels read and write the host memory over
-// the bus themselves, so a transfer is one launch, in whole lines both ways.
+// Fields between the caller's layout (particle-major, staged in pinned host memory)
+// and the pool's component arrays: element e of `host` is component e % nc of
+// particle e / nc.  The kernels read and write the host memory over the bus
+// themselves, so a transfer is one launch, in whole lines both ways.
+template <typename W>
 __global__ void __launch_bounds__(GR_BLOCK)
-    k_field_in(const double *host, int64_t count, int nc, int64_t cap, int64_t off, FieldSets F) {
+    k_field_in(const W *host, int64_t count, int nc, int64_t cap, int64_t off, FieldSets F) {
   const int64_t e = (int64_t)blockIdx.x * GR_BLOCK + threadIdx.x;
   if (e >= count) return;
-  const double v = host[e];
+  const W v = host[e];
   const int64_t at = (e % nc) * cap + off + e / nc;
   for (int q = 0; q < F.n; ++q) {
     if (F.esz[q] == 8)
@@ -2336,24 +2337,18 @@ __global__ void __launch_bounds__(GR_BLOCK)
       static_cast<float *>(F.p[q])[at] = (float)v;
   }
 }
+template <typename W>
 __global__ void __launch_bounds__(GR_BLOCK)
-    k_field_out(double *host, int64_t count, int nc, int64_t cap, int64_t off, FieldSets F) {
+    k_field_out(W *host, int64_t count, int nc, int64_t cap, int64_t off, FieldSets F) {
   const int64_t e = (int64_t)blockIdx.x * GR_BLOCK + threadIdx.x;
   if (e >= count) return;
   const int64_t at = (e % nc) * cap + off + e / nc;
-  host[e] = F.esz[0] == 8 ? static_cast<const double *>(F.p[0])[at]
-                          : (double)static_cast<const float *>(F.p[0])[at];
+  host[e] = F.esz[0] == 8 ? (W)static_cast<const double *>(F.p[0])[at]
+                          : (W)static_cast<const float *>(F.p[0])[at];
 }
-// 32-bit indices, the caller's being 64-bit and `add` larger.
-__global__ void __launch_bounds__(GR_BLOCK)
-    k_index_in(const int64_t *host, int64_t count, int64_t off, int add, int *dst) {
+__global__ void __launch_bounds__(GR_BLOCK) k_copy_i32(const int *src, int64_t count, int *dst) {
   const int64_t e = (int64_t)blockIdx.x * GR_BLOCK + threadIdx.x;
-  if (e < count) dst[off + e] = (int)(host[e] - add);
-}
-__global__ void __launch_bounds__(GR_BLOCK)
-    k_index_out(int64_t *host, int64_t count, int64_t off, int add, const int *src) {
-  const int64_t e = (int64_t)blockIdx.x * GR_BLOCK + threadIdx.x;
-  if (e < count) host[e] = (int64_t)src[off + e] + add;
+  if (e < count) dst[e] = src[e];
 }
 
 // ---------------------------------------------------------------------------
@@ -2694,21 +2689,22 @@ INST(float)
 INST(double)
 #undef INST
 
-void launch_field(hipStream_t s, bool in, double *host, int64_t count, int nc, int64_t cap,
-                  int64_t off, const FieldSets &F) {
+template <typename W>
+void launch_field(hipStream_t s, bool in, W *host, int64_t count, int nc, int64_t cap, int64_t off,
+                  const FieldSets &F) {
   if (count <= 0) return;
   if (in)
-    k_field_in<<<nb_of(count, GR_BLOCK), GR_BLOCK, 0, s>>>(host, count, nc, cap, off, F);
+    k_field_in<W><<<nb_of(count, GR_BLOCK), GR_BLOCK, 0, s>>>(host, count, nc, cap, off, F);
   else
-    k_field_out<<<nb_of(count, GR_BLOCK), GR_BLOCK, 0, s>>>(host, count, nc, cap, off, F);
+    k_field_out<W><<<nb_of(count, GR_BLOCK), GR_BLOCK, 0, s>>>(host, count, nc, cap, off, F);
 }
-void launch_index(hipStream_t s, bool in, int64_t *host, int64_t count, int64_t off, int add,
-                  int *dev) {
-  if (count <= 0) return;
-  if (in)
-    k_index_in<<<nb_of(count, GR_BLOCK), GR_BLOCK, 0, s>>>(host, count, off, add, dev);
-  else
-    k_index_out<<<nb_of(count, GR_BLOCK), GR_BLOCK, 0, s>>>(host, count, off, add, dev);
+template void launch_field<float>(hipStream_t, bool, float *, int64_t, int, int64_t, int64_t,
+                                  const FieldSets &);
+template void launch_field<double>(hipStream_t, bool, double *, int64_t, int, int64_t, int64_t,
+                                   const FieldSets &);
+void launch_index(hipStream_t s, bool in, int *host, int64_t count, int *dev) {
+  if (count > 0)
+    k_copy_i32<<<nb_of(count, GR_BLOCK), GR_BLOCK, 0, s>>>(in ? host : dev, count, in ? dev : host);
 }
 
 template <typename R>

@@ -202,11 +202,12 @@ struct FieldSets {
   int esz[3];  // 8: double, 4: float
   int n;
 };
-// `count` elements between pinned host memory and the particles from `off` on.
-void launch_field(hipStream_t s, bool in, double *host, int64_t count, int nc, int64_t cap,
-                  int64_t off, const FieldSets &F);
-void launch_index(hipStream_t s, bool in, int64_t *host, int64_t count, int64_t off, int add,
-                  int *dev);
+// `count` elements between pinned host memory and the particles from `off` on
+// (W: double, or float for a field held in 4 bytes).
+template <typename W>
+void launch_field(hipStream_t s, bool in, W *host, int64_t count, int nc, int64_t cap, int64_t off,
+                  const FieldSets &F);
+void launch_index(hipStream_t s, bool in, int *host, int64_t count, int *dev);
 void launch_fill_i32(hipStream_t s, int *p, int v, long long n);
 void launch_alias_check(hipStream_t s, const int *n, int ghost, int src_n, int *flags);
 template <typename R>
