@@ -734,8 +734,11 @@ void commit(gr_ctx *c) {
       nreal += s.cap;
     }
   }
-  const int64_t sc = std::max<int64_t>(std::max(nreal, nghost), 1);
+  int64_t sc = std::max<int64_t>(std::max(nreal, nghost), 1);
   if (sc > c->sort_cap) {
+    // by half at least, as the pool: systems laid out one by one would have all
+    // of these taken and given back each time
+    sc = std::max(sc, c->sort_cap + c->sort_cap / 2);
     c->keys.alloc(sc * 4);
     c->vals.alloc(sc * 4);
     c->keys2.alloc(sc * 4);
