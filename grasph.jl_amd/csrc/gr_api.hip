@@ -322,7 +322,6 @@ struct Plan {
   // system's budget of its entries
   int tiles_real = 0, tiles_ghost = 0;
   std::vector<unsigned> budget_real, budget_ghost;
-  DBuf d_budget_real, d_budget_ghost;
   unsigned long long x_epoch = 0;  // the context's, when the budgets were last checked
   // ghosts
   std::vector<int> ghost_list;
@@ -1796,7 +1795,6 @@ void plan_stages(gr_ctx *c, Plan &P, bool count_pairs_unused) {
     for (int g : c->integ[ig].ghost) P.stepsys.push_back({g, c->stepsys[g]});
     for (int q : c->integ[ig].probes) P.stepsys.push_back({q, c->stepsys[q]});
   }
-  upload_stepsys(c);
 }
 
 Plan &get_plan(gr_ctx *c, const std::vector<int> &integs) {
@@ -1870,8 +1868,13 @@ Plan &get_plan(gr_ctx *c, const std::vector<int> &integs) {
     P->tiles_real = key_tiles(c, reals, now, kGrowMargin + 4, P->budget_real);
     P->tiles_ghost =
         ghosts.empty() ? 0 : key_tiles(c, ghosts, now, kGrowMargin + 4, P->budget_ghost);
-    if (P->tiles_real > 0) P->d_budget_real.upload(P->budget_real, c->stream);
-    if (P->tiles_ghost > 0) P->d_budget_ghost.upload(P->budget_ghost, c->stream);
+    auto set = [&](const std::vector<int> &list, int tiles, const std::vector<unsigned> &budget) {
+      for (size_t q = 0; tiles > 0 && q < list.size(); ++q)
+        c->stepsys[list[q]].key_budget = budget[q];
+    };
+    set(reals, P->tiles_real, P->budget_real);
+    set(ghosts, P->tiles_ghost, P->budget_ghost);
+    for (auto &e : P->stepsys) e.second.key_budget = c->stepsys[e.first].key_budget;
     P->x_epoch = c->x_epoch;
     const int t = std::max(P->tiles_real, P->tiles_ghost);
     if (t > c->ktable_tiles) {
@@ -1881,6 +1884,7 @@ Plan &get_plan(gr_ctx *c, const std::vector<int> &integs) {
       drop_graphs(c);
     }
   }
+  upload_stepsys(c);
   HIPCHK(hipStreamSynchronize(c->stream));
   Plan &ref = *P;
   c->plans[integs] = std::move(P);
@@ -1950,15 +1954,15 @@ bool sort_preps_cells(const Plan &P, bool ghost) {
 
 // The counting sort of a step's real or ghost systems (after their bounds).
 void key_sort(gr_ctx *c, const Plan &P, const XP &xs, const DBuf &blk, int nblk, const DBuf &bbase,
-              const DBuf &list, int nlist, int n, int tiles, const DBuf &budget, bool cells) {
+              const DBuf &list, int nlist, int n, int tiles, bool cells) {
   const CellsArgs A = cells_args(c, P);
   launch_key_sort(c->stream, xs, c->d_sd.as<SysDesc>(), c->d_n.as<int>(), c->d_st.as<StepSys>(),
                   blk.as<Blk>(), nblk, bbase.as<int>(), c->D, list.as<int>(), nlist, n,
                   c->d_bbmin.as<long long>(), c->d_bbmax.as<long long>(), c->bb_rs,
                   c->d_kmin.as<int>(), c->d_kmax.as<int>(), c->d_krange.as<unsigned>(),
-                  c->d_kbase.as<unsigned>(), c->d_kshift.as<int>(), budget.as<unsigned>(),
-                  c->keys.as<unsigned>(), c->kfull.as<unsigned>(), c->keys2.as<unsigned>(),
-                  c->vals2.as<int>(), c->krank.as<unsigned>(), c->d_flags.as<int>(),
+                  c->d_kbase.as<unsigned>(), c->d_kshift.as<int>(), c->keys.as<unsigned>(),
+                  c->kfull.as<unsigned>(), c->keys2.as<unsigned>(), c->vals2.as<int>(),
+                  c->krank.as<unsigned>(), c->d_flags.as<int>(),
                   c->d_sysfault.as<int>(), c->krun.as<int>(), c->ktable.as<unsigned>(),
                   c->ktable_tiles, tiles, cells ? &A : nullptr);
 }
@@ -1986,8 +1990,7 @@ void phase_sort_real(gr_ctx *c, Plan &P, bool half = false, int pack = 0) {
   if (P.tiles_real > 0) {  // a step: counting sort (the bounds' replicas are reset already)
     if (!step_bounds(P)) step_minmax(c, P);
     key_sort(c, P, xs, P.blk_real, P.nblk_real, P.d_bbase_real, P.d_real_list,
-             (int)P.real_list.size(), P.n_real, P.tiles_real, P.d_budget_real,
-             sort_preps_cells(P, false));
+             (int)P.real_list.size(), P.n_real, P.tiles_real, sort_preps_cells(P, false));
     all_real(c, arb, arn);
     const KeyTable kt = key_table(c);
     Pool<R> A = pool_view<R>(c, c->cur), B = pool_view<R>(c, 1 - c->cur);
@@ -2047,8 +2050,7 @@ void phase_ghosts(gr_ctx *c, Plan &P, bool generate, bool sort) {
   if (table) {  // a step: counting sort (the bounds' replicas are reset already)
     const XP gx = xp_gxs(c);
     key_sort(c, P, gx, P.blk_ghost, P.nblk_ghost, P.d_bbase_ghost, P.d_ghost_list,
-             (int)P.ghost_list.size(), P.n_ghost, P.tiles_ghost, P.d_budget_ghost,
-             sort_preps_cells(P, true));
+             (int)P.ghost_list.size(), P.n_ghost, P.tiles_ghost, sort_preps_cells(P, true));
     const KeyTable kt = key_table(c);
     launch_permute_ghost(s, gx, c->gidx_s.as<int>(), c->gbnd_s.as<int>(), xpw_pool(c, c->cur),
                          A.gidx, A.gbnd, c->d_sd.as<SysDesc>(), c->d_n.as<int>(),

@@ -65,6 +65,7 @@ struct StepSys {
   // first force stage assigns them), 2 strain rate, 4 vorticity (the first
   // strain-rate stage assigns them and no updater before it reads them)
   int32_t perm_skip;
+  uint32_t key_budget;  // entries of the counting sort's table (>= 1)
 };
 
 struct Bnd {  // ghost boundary plane

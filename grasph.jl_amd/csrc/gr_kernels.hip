@@ -370,7 +370,7 @@ __device__ inline void key_space_store(const KeySpace &K, int s, bool live, long
 __device__ inline unsigned key_buckets(unsigned long long range, unsigned budget, int &sh) {
   sh = 0;
   if (range == 0ull) return 0u;
-  while (((range - 1ull) >> sh) >= (unsigned long long)budget) ++sh;
+  while (sh < 32 && ((range - 1ull) >> sh) >= (unsigned long long)budget) ++sh;
   return (unsigned)((range - 1ull) >> sh) + 1u;
 }
 // Flags of the whole key range: overflow, the bound of the keys and the radix
@@ -386,11 +386,11 @@ __global__ void __launch_bounds__(KB_THREADS)
     k_key_base(const int *list, int nlist, int D, int pad, const int *n_dev, const StepSys *st,
                long long *bbmin, long long *bbmax, int rs, int *kmin, int *kmax,
                unsigned *kbase, unsigned *krange, int *flags, int *sysfault,
-               const unsigned *budget, int *kshift) {
+               int *kshift) {
   // one workgroup: the systems' key ranges in parallel, KB_THREADS at a time,
   // and their exclusive prefix sum (each system's keys start after the ranges
   // of the systems listed before it, plus one padding key each when `pad`);
-  // with `budget`, for the counting sort, their buckets'
+  // with `kshift`, for the counting sort, their buckets'
   __shared__ unsigned long long wsum[KB_THREADS / 64], wall[KB_THREADS / 64];
   const int t = threadIdx.x, lane = t & 63, w = t >> 6;
   unsigned long long carry = 0, all = 0;
@@ -400,7 +400,7 @@ __global__ void __launch_bounds__(KB_THREADS)
     int s = -1, sh = 0;
     if (q < nlist) {
       s = list[q];
-      const unsigned most = budget ? budget[q] : 0u;
+      const unsigned most = st[s].key_budget;
       KeySpace K;
       const bool live = n_dev[s] > 0;
       range = key_space(D, st[s].sort_cutoff, bbmin, bbmax, rs, s, K);
@@ -408,7 +408,7 @@ __global__ void __launch_bounds__(KB_THREADS)
       key_space_store(K, s, live, bbmin, bbmax, kmin, kmax, krange, flags, sysfault);
       range += pad ? 1 : 0;
       num = range;
-      if (budget) {
+      if (kshift) {
         num = key_buckets(range, most, sh);
         kshift[s] = sh;
       }
@@ -441,7 +441,7 @@ __global__ void __launch_bounds__(KB_THREADS)
   }
   if (t == 0) {
     key_flags(all, flags);
-    if (budget)
+    if (kshift)
       flags[2] = (int)(unsigned)carry;
     else
       flags[0] = 0;
@@ -801,8 +801,8 @@ __global__ void __launch_bounds__(GR_BLOCK)
     k_key_count(XP xs, const SysDesc *sd, const int *n_dev, const StepSys *st, const Blk *blk,
                 const int *bbase, const int *list, int nlist, long long *bbmin, long long *bbmax,
                 int rs, int *kmin, int *kmax, unsigned *krange, unsigned *kbase, int *kshift,
-                const unsigned *budget, unsigned *keys, unsigned *full, unsigned *rank, int *flags,
-                int *sysfault, unsigned *count, unsigned *tsum, int inl) {
+                unsigned *keys, unsigned *full, unsigned *rank, int *flags, int *sysfault,
+                unsigned *count, unsigned *tsum, int inl) {
   __shared__ int s_kmin[3], s_sh;
   __shared__ unsigned s_kr[3], s_base;
   __shared__ unsigned kw[GR_BLOCK / 64];
@@ -834,7 +834,7 @@ __global__ void __launch_bounds__(GR_BLOCK)
         const bool live = n_dev[q] > 0;
         range = key_space(D, st[q].sort_cutoff, bbmin, bbmax, rs, q, K);
         if (!live) range = 0;
-        num = key_buckets(range, budget[lane], sh);
+        num = key_buckets(range, st[q].key_budget, sh);
         if (blockIdx.x == 0)
           key_space_store(K, q, live, bbmin, bbmax, kmin, kmax, krange, flags, sysfault);
       }
@@ -2383,7 +2383,7 @@ void launch_key_base(hipStream_t s, const int *list, int nlist, int D, int pad, 
                      const StepSys *st, long long *bbmin, long long *bbmax, int rs, int *kmin,
                      int *kmax, unsigned *kbase, unsigned *krange, int *flags, int *sysfault) {
   k_key_base<<<1, KB_THREADS, 0, s>>>(list, nlist, D, pad, n, st, bbmin, bbmax, rs, kmin, kmax,
-                                      kbase, krange, flags, sysfault, nullptr, nullptr);
+                                      kbase, krange, flags, sysfault, nullptr);
 }
 static int cells_prep_blocks(const CellsArgs &A) { return nb_of(A.n_inter, GR_BLOCK) + A.ncblk; }
 void launch_cells_prep(hipStream_t s, const CellsArgs &A, int *flags, int *sysfault) {
@@ -2396,8 +2396,8 @@ int key_table_tile() { return KT_TILE; }
 void launch_key_sort(hipStream_t s, XP xs, const SysDesc *sd, const int *n, const StepSys *st,
                      const Blk *blk, int nblk, const int *bbase, int D, const int *list, int nlist,
                      int N, long long *bbmin, long long *bbmax, int rs, int *kmin, int *kmax,
-                     unsigned *krange, unsigned *kbase, int *kshift, const unsigned *budget,
-                     unsigned *keys, unsigned *full, unsigned *keys2, int *vals2, unsigned *rank,
+                     unsigned *krange, unsigned *kbase, int *kshift, unsigned *keys,
+                     unsigned *full, unsigned *keys2, int *vals2, unsigned *rank,
                      int *flags, int *sysfault, int *run, unsigned *table, int tiles, int ntile,
                      const CellsArgs *cells) {
   if (nblk <= 0) {
@@ -2409,11 +2409,11 @@ void launch_key_sort(hipStream_t s, XP xs, const SysDesc *sd, const int *n, cons
   const int inl = nlist <= KC_SYSTEMS && nblk <= KC_BLOCKS;
   if (!inl)
     k_key_base<<<1, KB_THREADS, 0, s>>>(list, nlist, D, 0, n, st, bbmin, bbmax, rs, kmin, kmax,
-                                        kbase, krange, flags, sysfault, budget, kshift);
+                                        kbase, krange, flags, sysfault, kshift);
   auto go = [&](auto dc) {
     k_key_count<decltype(dc)::value><<<nblk, GR_BLOCK, 0, s>>>(
         xs, sd, n, st, blk, bbase, list, nlist, bbmin, bbmax, rs, kmin, kmax, krange, kbase, kshift,
-        budget, keys, full, rank, flags, sysfault, count, tsum, inl);
+        keys, full, rank, flags, sysfault, count, tsum, inl);
   };
   if (D == 2)
     go(std::integral_constant<int, 2>{});

@@ -95,8 +95,8 @@ struct CellsArgs {
 };
 // The counting sort of a step (keys, table, placement) after the bounds pass:
 // `table` of key_table_bytes(tiles) bytes, zeroed when allocated, of which this
-// sort uses ntile <= tiles tiles: the listed systems' budgets of entries (at
-// least one each) come to less than ntile·key_table_tile().  (The layout goes by
+// sort uses ntile <= tiles tiles: the listed systems' budgets of entries
+// (key_budget) come to less than ntile·key_table_tile().  (The layout goes by
 // `tiles`, as sorts of different sizes share the table.)  flags[0] must be clear;
 // the permutations take the order by a KeyTable.  Replicas 1.. of the listed
 // systems' bounds are reset, and `cells` prepared (as launch_cells_prep does).
@@ -105,8 +105,8 @@ int key_table_tile();
 void launch_key_sort(hipStream_t s, XP xs, const SysDesc *sd, const int *n, const StepSys *st,
                      const Blk *blk, int nblk, const int *bbase, int D, const int *list, int nlist,
                      int N, long long *bbmin, long long *bbmax, int rs, int *kmin, int *kmax,
-                     unsigned *krange, unsigned *kbase, int *kshift, const unsigned *budget,
-                     unsigned *keys, unsigned *full, unsigned *keys2, int *vals2, unsigned *rank,
+                     unsigned *krange, unsigned *kbase, int *kshift, unsigned *keys,
+                     unsigned *full, unsigned *keys2, int *vals2, unsigned *rank,
                      int *flags, int *sysfault, int *run, unsigned *table, int tiles, int ntile,
                      const CellsArgs *cells = nullptr);
 struct KeyTable {  // what the permutations read of the counting sort
