@@ -1217,7 +1217,9 @@ constexpr int kGrowMargin = 8;
 // Also 0 where the particles times the mean number in a cell of their system
 // exceed kKeyRank: the rank within the cell grows with them (particles in motion,
 // 2D: 1M at 32 a cell 92 / 111, at 128 149 / 111; 200k at 128 57 / 80, at 200
-// 73 / 75, at 1024 76 / 75; 20k at 1024 33 / 51, at 4096 54 / 49).
+// 73 / 75, at 1024 76 / 75; 20k at 1024 33 / 51, at 4096 54 / 49; whole steps: 256
+// columns, 6.7M at 9 a cell, 3785 / 3745, 3D dam breaks of 3.0M at 14 1726 / 1729,
+// of 4.2M 2275 / 2236).
 //
 // `slack`: the limits are so much higher for a table in use.
 constexpr int kMaxKeyTiles = 4096;
